@@ -1339,9 +1339,8 @@ int hymi_prolongate( hymi_function f, int srcLevel, int flag )
       requireLevel( f->f, srcLevel );
       requireLevel( f->f, srcLevel + 1 );
       // Replace: the fine flag DoFs become P c, all other fine values keep theirs (the gather form writes every
-      // flag DoF of the fine level once, so zeroing them first and adding is the replacement)
-      launchLincomb( f->f, srcLevel + 1, flag, 0, nullptr, nullptr, false, 0.0 );
-      launchProlongateAdd( f->f, srcLevel, flag );
+      // flag DoF of the fine level once)
+      launchProlongate( f->f, srcLevel, flag );
    } );
 }
 
@@ -1505,8 +1504,7 @@ int hymi_fmg_solve( hymi_gmg g, hymi_function x, hymi_function b, int level, int
          {
             // prolongate with Replace: the next level's Inner | Neumann DoFs become P x (the others keep
             // their values); the first cycle there refreshes every closure copy
-            launchLincomb( x->f, cur + 1, flag, 0, nullptr, nullptr, false, 0.0 );
-            launchProlongateAdd( x->f, cur, flag, true );
+            launchProlongate( x->f, cur, flag );
          }
       }
    } );

@@ -2665,7 +2665,9 @@ __device__ __forceinline__ void prolongDir( int px, int py, int pz, int& dx, int
 
 // Several right-hand sides: a wave owns a row segment of kRowSeg fine points and walks it 64 / NR points at a
 // time; the coarse rows of both x-parity classes are formed once per segment (32-bit, see kCellApply).
-template < typename T, int NR >
+// REPL (here and in the other prolongation parts): the fine points become the interpolated value instead of gaining
+// it (0 + value, so a replacement gives the bits of adding to zeroed points); the fine values are not read.
+template < typename T, int NR, bool REPL >
 __global__ __launch_bounds__( 256 ) void kProlongCell( LV gc, LV gf, const CellSeg* __restrict__ segs, int64_t nseg,
                                                        const int* __restrict__ ctype, int flag,
                                                        const T* __restrict__ uc, T* __restrict__ uf )
@@ -2694,7 +2696,8 @@ __global__ __launch_bounds__( 256 ) void kProlongCell( LV gc, LV gf, const CellS
       const int dx = px ? d1x : d0x;
       const int im = ( px ? m1 : m0 ) + ( x - dx ) / 2, ip = ( px ? p1 : p0 ) + ( x + dx ) / 2;
       const T   v  = T( 0.5 ) * ( cu[im * NR + r] + cu[ip * NR + r] );
-      fu[( rf + x ) * NR + r] += v;
+      const int o  = ( rf + x ) * NR + r;
+      fu[o]        = ( REPL ? T( 0 ) : fu[o] ) + v;
    }
 }
 
@@ -2708,7 +2711,7 @@ struct ProlongWindows
    bool ok[kTransferWindows];
 };
 
-template < typename T >
+template < typename T, bool REPL >
 __device__ __forceinline__ void prolongFlatLoad( const MarchUnit& U, bool active, int lane, LV gc, LV gf,
                                                  const T* __restrict__ uc, T* __restrict__ uf, ProlongWindows< T >& P )
 {
@@ -2762,7 +2765,7 @@ __device__ __forceinline__ void prolongFlatLoad( const MarchUnit& U, bool active
             P.fo[j] = S0 + e;
          }
       }
-      P.fv[j] = fu[P.fo[j]];
+      P.fv[j] = REPL ? T( 0 ) : fu[P.fo[j]];
       P.ca[j] = cu[im];
       P.cb[j] = cu[ip];
    }
@@ -2796,7 +2799,7 @@ constexpr int prolongUnitsPerWave()
 {
    return sizeof( T ) == 4 ? 2 : 1;
 }
-template < typename T >
+template < typename T, bool REPL >
 __device__ __forceinline__ void kProlongFlat_b( const Blk& B, LV gc, LV gf, const MarchUnit* __restrict__ units,
                                                 int64_t nUnits, const int* __restrict__ ctype, int flag,
                                                 const T* __restrict__ uc, T* __restrict__ uf )
@@ -2816,20 +2819,20 @@ __device__ __forceinline__ void kProlongFlat_b( const Blk& B, LV gc, LV gf, cons
       const MarchUnit U1 = u1 < nUnits ? units[u1] : U0;
       const bool      a1 = u1 < nUnits && ( ctype[U1.cell] & flag ) != 0;
       ProlongWindows< T > P1;
-      prolongFlatLoad( U0, a0, lane, gc, gf, uc, uf, P0 );
-      prolongFlatLoad( U1, a1, lane, gc, gf, uc, uf, P1 );
+      prolongFlatLoad< T, REPL >( U0, a0, lane, gc, gf, uc, uf, P0 );
+      prolongFlatLoad< T, REPL >( U1, a1, lane, gc, gf, uc, uf, P1 );
       prolongFlatStore( U0, a0, gf, uf, P0 );
       prolongFlatStore( U1, a1, gf, uf, P1 );
    }
    else
    {
       static_assert( UPW == 1, "one or two units per wave" );
-      prolongFlatLoad( U0, a0, lane, gc, gf, uc, uf, P0 );
+      prolongFlatLoad< T, REPL >( U0, a0, lane, gc, gf, uc, uf, P0 );
       prolongFlatStore( U0, a0, gf, uf, P0 );
    }
 }
 
-template < typename T, int NR >
+template < typename T, int NR, bool REPL >
 __device__ __forceinline__ void kProlongFace_b( const Blk& B, LV gc, LV gf, const FaceGeom* __restrict__ fg, int flag, const T* __restrict__ uc,
                               T* __restrict__ uf )
 {
@@ -2856,10 +2859,11 @@ __device__ __forceinline__ void kProlongFace_b( const Blk& B, LV gc, LV gf, cons
       v = T( 0.5 ) * ( uc[( co + fidx( gc.w, ( i - di ) / 2, ( j - dj ) / 2 ) ) * NR + r] +
                        uc[( co + fidx( gc.w, ( i + di ) / 2, ( j + dj ) / 2 ) ) * NR + r] );
    }
-   uf[( gf.offF + (int64_t) G.face * gf.fS + fidx( gf.w, i, j ) ) * NR + r] += v;
+   const int64_t o = ( gf.offF + (int64_t) G.face * gf.fS + fidx( gf.w, i, j ) ) * NR + r;
+   uf[o]           = ( REPL ? T( 0 ) : uf[o] ) + v;
 }
 
-template < typename T, int NR >
+template < typename T, int NR, bool REPL >
 __device__ __forceinline__ void kProlongEdge_b( const Blk& B, LV gc, LV gf, const EdgeGeom* __restrict__ eg, int flag, const T* __restrict__ uc,
                               T* __restrict__ uf )
 {
@@ -2872,10 +2876,11 @@ __device__ __forceinline__ void kProlongEdge_b( const Blk& B, LV gc, LV gf, cons
    const int64_t co = gc.offE + (int64_t) G.edge * gc.eS;
    const T       v  = ( x & 1 ) ? T( 0.5 ) * ( uc[( co + x / 2 ) * NR + r] + uc[( co + x / 2 + 1 ) * NR + r] )
                                 : uc[( co + x / 2 ) * NR + r];
-   uf[( gf.offE + (int64_t) G.edge * gf.eS + x ) * NR + r] += v;
+   const int64_t o = ( gf.offE + (int64_t) G.edge * gf.eS + x ) * NR + r;
+   uf[o]           = ( REPL ? T( 0 ) : uf[o] ) + v;
 }
 
-template < typename T, int NR >
+template < typename T, int NR, bool REPL >
 __device__ __forceinline__ void kProlongVertex_b( const Blk& B, const VertexGeom* __restrict__ vg, int nV, int flag, const T* __restrict__ uc,
                                 T* __restrict__ uf )
 {
@@ -2884,12 +2889,12 @@ __device__ __forceinline__ void kProlongVertex_b( const Blk& B, const VertexGeom
    const int64_t v = t / NR;
    if ( v >= nV ) return;
    if ( !( vg[v].type & flag ) ) return;
-   uf[v * NR + r] += uc[v * NR + r];
+   uf[v * NR + r] = ( REPL ? T( 0 ) : uf[v * NR + r] ) + uc[v * NR + r];
 }
 
 // a prolongation in one launch (LowGrid): vertex, edge and face parts, and the macro-cell part (one right-hand
 // side: kProlongFlat_b over the fine level's transfer units)
-template < typename T, int NR >
+template < typename T, int NR, bool REPL >
 __global__ __launch_bounds__( 256 ) void kLowProlong( LowGrid L, LV gc, LV gf, const VertexGeom* __restrict__ vgFine,
                                                       int nV, const EdgeGeom* __restrict__ egFine,
                                                       const FaceGeom* __restrict__ fgFine, int flag,
@@ -2900,14 +2905,14 @@ __global__ __launch_bounds__( 256 ) void kLowProlong( LowGrid L, LV gc, LV gf, c
    Blk       B;
    const int part = lowPart( L, B );
    if ( part == 0 )
-      kProlongVertex_b< T, NR >( B, vgFine, nV, flag, uc, uf );
+      kProlongVertex_b< T, NR, REPL >( B, vgFine, nV, flag, uc, uf );
    else if ( part == 1 )
-      kProlongEdge_b< T, NR >( B, gc, gf, egFine, flag, uc, uf );
+      kProlongEdge_b< T, NR, REPL >( B, gc, gf, egFine, flag, uc, uf );
    else if ( part == 2 )
-      kProlongFace_b< T, NR >( B, gc, gf, fgFine, flag, uc, uf );
+      kProlongFace_b< T, NR, REPL >( B, gc, gf, fgFine, flag, uc, uf );
    else if ( part == 3 )
    {
-      if constexpr ( NR == 1 ) kProlongFlat_b< T >( B, gc, gf, cellUnits, nCellUnits, ctypeF, flag, uc, uf );
+      if constexpr ( NR == 1 ) kProlongFlat_b< T, REPL >( B, gc, gf, cellUnits, nCellUnits, ctypeF, flag, uc, uf );
    }
 }
 
@@ -3898,7 +3903,7 @@ void residualRestrictT( Operator& op, Function& x, Function& r, Function& b, int
    restrictT< T, NR >( r, b, L, flag, true, false, zeroCoarse );
 }
 
-template < typename T, int NR >
+template < typename T, int NR, bool REPL >
 void prolongT( Function& f, int srcLevel, int flag, bool refreshCoarse )
 {
    Mesh&       M  = *f.mesh;
@@ -3927,14 +3932,14 @@ void prolongT( Function& f, int srcLevel, int flag, bool refreshCoarse )
       constexpr int upw = prolongUnitsPerWave< T >();
       lg.nbC            = nu > 0 ? (int) xcdGrid( ( ( nu + upw - 1 ) / upw + 3 ) / 4 ) : 0;
    }
-   hipLaunchKernelGGL( ( kLowProlong< T, NR > ), dim3( lowBlocks( lg ) ), dim3( 256 ), 0, s, lg, gc, gf, Pf.dVertexGeom.p, nV,
+   hipLaunchKernelGGL( ( kLowProlong< T, NR, REPL > ), dim3( lowBlocks( lg ) ), dim3( 256 ), 0, s, lg, gc, gf, Pf.dVertexGeom.p, nV,
                        Pf.dEdgeGeom.p, Pf.dFaceGeom.p, flag, uc, uf, tu, nu, Pf.dCellType.p );
    if ( NR == 1 ) return;
    int64_t        nseg = 0;
    rowSegFits< NR >( Pf );
    const CellSeg* sg   = M.segments( Pf, kRowSeg, &nseg );
    if ( nseg > 0 )
-      hipLaunchKernelGGL( ( kProlongCell< T, NR > ), dim3( (unsigned) xcdGrid( ( nseg + 3 ) / 4 ) ), dim3( 256 ), 0, s, gc,
+      hipLaunchKernelGGL( ( kProlongCell< T, NR, REPL > ), dim3( (unsigned) xcdGrid( ( nseg + 3 ) / 4 ) ), dim3( 256 ), 0, s, gc,
                           gf, sg, nseg, Pf.dCellType.p, flag, uc, uf );
 }
 
@@ -4104,7 +4109,13 @@ struct ResidualRestrictF
 template < typename T, int NR >
 struct ProlongF
 {
-   static void run( Function& f, int L, int flag, bool refresh ) { prolongT< T, NR >( f, L, flag, refresh ); }
+   static void run( Function& f, int L, int flag, bool refresh, bool replace )
+   {
+      if ( replace )
+         prolongT< T, NR, true >( f, L, flag, refresh );
+      else
+         prolongT< T, NR, false >( f, L, flag, refresh );
+   }
 };
 template < typename T, int NR >
 struct DotF
@@ -4220,7 +4231,12 @@ void launchResidualRestrict( Operator& op, Function& x, Function& r, Function& b
 
 void launchProlongateAdd( Function& f, int srcLevel, int flag, bool refreshCoarse )
 {
-   dispatch< ProlongF >( f.prec, f.nrhs, f, srcLevel, flag, refreshCoarse );
+   dispatch< ProlongF >( f.prec, f.nrhs, f, srcLevel, flag, refreshCoarse, false );
+}
+
+void launchProlongate( Function& f, int srcLevel, int flag )
+{
+   dispatch< ProlongF >( f.prec, f.nrhs, f, srcLevel, flag, true, true );
 }
 
 void launchLincomb( Function& dst, int level, int flag, int n, const double* c, Function* const* src, bool accumulate,

@@ -37,6 +37,8 @@ void launchRestrict( Function& f, Function& dst, int srcLevel, int flag, bool ba
 void launchResidualRestrict( Operator& op, Function& x, Function& r, Function& b, int level, int flag,
                              bool refreshSrc, Function* zeroCoarse = nullptr );
 void launchProlongateAdd( Function& f, int srcLevel, int flag, bool refreshCoarse = true );
+// the flag DoFs of level srcLevel + 1 become the prolongation of srcLevel (written, not read)
+void launchProlongate( Function& f, int srcLevel, int flag );
 // the coarse-grid CG of a V-cycle in one launch where it applies (level 0, one right-hand side, at most
 // kCgVertexMax vertices): x's owned values are updated, its closure copies are not; returns false (nothing
 // launched) where it does not apply
