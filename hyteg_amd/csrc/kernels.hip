@@ -107,7 +107,8 @@ __device__ __forceinline__ int64_t xcdBlockOf( int64_t b, int64_t nLogical )
 }
 
 __device__ __forceinline__ int64_t tet( int64_t w ) { return w * ( w + 1 ) * ( w + 2 ) / 6; }
-__device__ __forceinline__ int64_t fidx( int64_t w, int64_t x, int64_t y ) { return y * ( w + 1 ) - y * ( y + 1 ) / 2 + x; }
+// face-relative index (a face of level 12 holds 8 million points)
+__device__ __forceinline__ int     fidx( int w, int x, int y ) { return y * ( w + 1 ) - ( y * ( y + 1 ) >> 1 ) + x; }
 __device__ __forceinline__ int64_t cidx( int64_t w, int64_t x, int64_t y, int64_t z )
 {
    const int64_t wz = w - z;
@@ -136,19 +137,38 @@ __device__ __forceinline__ int crow32( int w, int t0, int y, int z )
 }
 // cell-relative index of (x, y, z) and face-relative index of (i, j), 32-bit (t0 = tet32(w))
 __device__ __forceinline__ int cellRel( int w, int t0, int x, int y, int z ) { return crow32( w, t0, y, z ) + x; }
-__device__ __forceinline__ int faceRel( int w, int i, int j ) { return j * ( w + 1 ) - ( j * ( j + 1 ) >> 1 ) + i; }
-// (a, b) of flat index k in the triangle of width m (row-major, row b has m - b points)
-__device__ __forceinline__ void triPos( int64_t m, int64_t k, int& a, int& b )
+__device__ __forceinline__ int faceRel( int w, int i, int j ) { return fidx( w, i, j ); }
+// Row of flat index f in a triangle of width W stored row by row (row y has W - y points and starts at
+// R(y) = y (2W + 1 - y) / 2): the integer part of the smaller root of R(y) = f, taken in float, corrected by
+// one row either way (the float root is off by less than one row for W <= 1025).  0 <= f < W (W + 1) / 2.
+__device__ __forceinline__ int triRow32( int W, int f )
 {
-   const double  q  = double( 2 * m + 1 );
-   int64_t       bb = (int64_t) ( ( q - sqrt( q * q - 8.0 * double( k ) ) ) * 0.5 );
-   if ( bb < 0 ) bb = 0;
-   while ( bb > 0 && fidx( m, 0, bb ) > k )
-      bb--;
-   while ( fidx( m, 0, bb + 1 ) <= k )
-      bb++;
-   b = (int) bb;
-   a = (int) ( k - fidx( m, 0, bb ) );
+   const float q = (float) ( 2 * W + 1 );
+   int         y = (int) ( 0.5f * ( q - sqrtf( q * q - 8.0f * (float) f ) ) );
+   y += ( y + 1 ) * ( 2 * W - y ) / 2 <= f ? 1 : 0;
+   y -= y * ( 2 * W + 1 - y ) / 2 > f ? 1 : 0;
+   return y;
+}
+
+// (a, b) of flat index k in the triangle of width m (row-major, row b has m - b points).  The closed form in float
+// holds up to the widths of level 11 (triRow32).  With a double root and 64-bit products instead, the level-8 FP32
+// prolongation took 302 us (296 us now) and a level-4 V(2,2) cycle of 6 macro-tets 345 us (342 us); the level-8 apply
+// did not change: its face part is bound by the scattered cell reads.
+constexpr int kTriRowMaxW = 2050;
+__device__ __forceinline__ void triPos( int m, int k, int& a, int& b )
+{
+   if ( m <= kTriRowMaxW )
+      b = triRow32( m, k );
+   else
+   {
+      const double q = double( 2 * m + 1 );
+      b              = max( 0, (int) ( ( q - sqrt( q * q - 8.0 * double( k ) ) ) * 0.5 ) );
+      while ( b > 0 && fidx( m, 0, b ) > k )
+         b--;
+      while ( fidx( m, 0, b + 1 ) <= k )
+         b++;
+   }
+   a = k - fidx( m, 0, b );
 }
 
 // XCD-aware block order: XCD k (blocks b with b % 8 == k) gets a contiguous range of logical blocks
@@ -219,18 +239,6 @@ __global__ void kE2F( LV g, const E2F* __restrict__ tab, int n, T* __restrict__ 
    const int64_t dst = g.offF + (int64_t) m.face * g.fS + fidx( g.w, col, row );
    const int64_t src = g.offE + (int64_t) m.edge * g.eS + p;
    u[dst * NR + r]   = u[src * NR + r];
-}
-
-// Row of flat index f in a triangle of width W stored row by row (row y has W - y points and starts at
-// R(y) = y (2W + 1 - y) / 2): the integer part of the smaller root of R(y) = f, taken in float, corrected by
-// one row either way (the float root is off by less than one row for W <= 1025).  0 <= f < W (W + 1) / 2.
-__device__ __forceinline__ int triRow32( int W, int f )
-{
-   const float q = (float) ( 2 * W + 1 );
-   int         y = (int) ( 0.5f * ( q - sqrtf( q * q - 8.0f * (float) f ) ) );
-   y += ( y + 1 ) * ( 2 * W - y ) / 2 <= f ? 1 : 0;
-   y -= y * ( 2 * W + 1 - y ) / 2 > f ? 1 : 0;
-   return y;
 }
 
 // Face-to-cell closure copy.  Block = (chunk of 256 * U values of one face, cell-face pair); thread t takes
@@ -1572,7 +1580,7 @@ __device__ __forceinline__ void kFaceApply_b( const Blk& B, LV g, const FaceGeom
    const int64_t k  = t / NR;
    if ( k >= np ) return;
    int a, bb;
-   triPos( m, k, a, bb );
+   triPos( m, (int) k, a, bb );
    const int     i   = a + 1, j = bb + 1;
    const int64_t fo  = g.offF + (int64_t) G.face * g.fS;
    const T       acc = faceStencilSum< T, NR >( g, G, FW + (int64_t) G.face * kFaceW, u, fo, i, j, r, true );
@@ -2244,7 +2252,7 @@ __global__ void kModesFace( LV g, const FaceGeom* __restrict__ fg, int frameOff,
    const int64_t   k  = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
    if ( k >= np || !( G.type & flag ) ) return;
    int a, bb;
-   triPos( m, k, a, bb );
+   triPos( m, (int) k, a, bb );
    const int i = a + 1, j = bb + 1;
    putModes< T, NR >( u, g.offF + (int64_t) G.face * g.fS + fidx( g.w, i, j ), fr + 12 * ( (int64_t) frameOff + G.face ),
                       1.0 / ( g.w - 1 ), i, j, 0, modes, nModes );
@@ -2517,7 +2525,7 @@ __device__ __forceinline__ void kRestrictFace_b( const Blk& B, LV gc, LV gf, con
    const int64_t k  = t / NR;
    if ( k >= np ) return;
    int a, bb;
-   triPos( m, k, a, bb );
+   triPos( m, (int) k, a, bb );
    const int I = a + 1, J = bb + 1;
    const int i = 2 * I, j = 2 * J, w = gf.w;
    const int64_t fo = gf.offF + (int64_t) G.face * gf.fS;
@@ -2845,7 +2853,7 @@ __device__ __forceinline__ void kProlongFace_b( const Blk& B, LV gc, LV gf, cons
    const int64_t k  = t / NR;
    if ( k >= np ) return;
    int a, bb;
-   triPos( m, k, a, bb );
+   triPos( m, (int) k, a, bb );
    const int     i = a + 1, j = bb + 1;
    const int64_t co = gc.offF + (int64_t) G.face * gc.fS;
    const int     pi = i & 1, pj = j & 1;
@@ -3173,7 +3181,7 @@ __global__ __launch_bounds__( 256 ) void kDotLow( LV g, const FaceGeom* __restri
          if ( fg[f].type & flag )
          {
             int aa, bb;
-            triPos( g.w - 3, k % mF, aa, bb );
+            triPos( g.w - 3, (int) ( k % mF ), aa, bb );
             o = g.offF + (int64_t) f * g.fS + fidx( g.w, aa + 1, bb + 1 );
          }
       }
