@@ -190,6 +190,29 @@ __device__ __forceinline__ void static_for( F&& f )
    }
 }
 
+// The 15-point sums and SOR updates of the macro-cell kernels, with the fused multiply-adds written out: every kernel
+// rounds at the same places, whatever the compiler contracts around it, so the forms of a phase stay equal bit for
+// bit.  A sum runs in three chains (the point's slab, the slabs above and below) of 15 instructions in place of 22 for
+// products added in pairs; no kernel got faster or slower by it (level-8 apply 793 us, level-7 FP64 V(3,3) 3.48 ms).
+__device__ __forceinline__ double fmaT( double a, double b, double c ) { return __builtin_fma( a, b, c ); }
+__device__ __forceinline__ float  fmaT( float a, float b, float c ) { return __builtin_fmaf( a, b, c ); }
+template < typename T >
+__device__ __forceinline__ T fma2( T a, T x, T b, T y )
+{
+   return fmaT( b, y, a * x );
+}
+template < typename T >
+__device__ __forceinline__ T fma2( T a, T x, T b, T y, T sum )
+{
+   return fmaT( b, y, fmaT( a, x, sum ) );
+}
+// (1 - omega) z + relax (b - sum)
+template < typename T >
+__device__ __forceinline__ T sorUpdate( T omega, T relax, T z, T b, T sum )
+{
+   return fmaT( relax, b - sum, ( T( 1 ) - omega ) * z );
+}
+
 enum
 {
    dC,
@@ -425,13 +448,14 @@ __global__ __launch_bounds__( 256 ) void kCellApply( LV g, const CellSeg* __rest
    {
 #define U( i ) cu[( ( i ) + x ) * NR + r]
       T acc = cC * U( r0 );
-      acc += cW * U( r0 - 1 ) + cE * U( r0 + 1 );
-      acc += cN * U( rN ) + cNW * U( rN - 1 );
-      acc += cS * U( rS ) + cSE * U( rS + 1 );
-      acc += cTC * U( rT ) + cTW * U( rT - 1 );
-      acc += cTS * U( rTS ) + cTSE * U( rTS + 1 );
-      acc += cBC * U( rB ) + cBE * U( rB + 1 );
-      acc += cBN * U( rBN ) + cBNW * U( rBN - 1 );
+      acc   = fma2( cW, U( r0 - 1 ), cE, U( r0 + 1 ), acc );
+      acc   = fma2( cN, U( rN ), cNW, U( rN - 1 ), acc );
+      acc   = fma2( cS, U( rS ), cSE, U( rS + 1 ), acc );
+      T up  = fma2( cTC, U( rT ), cTW, U( rT - 1 ) );
+      up    = fma2( cTS, U( rTS ), cTSE, U( rTS + 1 ), up );
+      T dn  = fma2( cBC, U( rB ), cBE, U( rB + 1 ) );
+      dn    = fma2( cBN, U( rBN ), cBNW, U( rBN - 1 ), dn );
+      acc   = acc + ( up + dn );
 #undef U
       const int64_t o = base + ( r0 + x ) * NR + r;
       if ( MODE == kReplace )
@@ -472,16 +496,17 @@ __global__ __launch_bounds__( 256 ) void kCellSor( LV g, const CellSeg* __restri
    for ( int x = xc + 4 * ( lane / NR ); x < xEnd; x += 4 * ( 64 / NR ) )
    {
 #define U( i ) cu[( ( i ) + x ) * NR + r]
-      T acc = cW * U( r0 - 1 ) + cE * U( r0 + 1 );
-      acc += cN * U( rN ) + cNW * U( rN - 1 );
-      acc += cS * U( rS ) + cSE * U( rS + 1 );
-      acc += cTC * U( rT ) + cTW * U( rT - 1 );
-      acc += cTS * U( rTS ) + cTSE * U( rTS + 1 );
-      acc += cBC * U( rB ) + cBE * U( rB + 1 );
-      acc += cBN * U( rBN ) + cBNW * U( rBN - 1 );
+      T acc = fma2( cW, U( r0 - 1 ), cE, U( r0 + 1 ) );
+      acc   = fma2( cN, U( rN ), cNW, U( rN - 1 ), acc );
+      acc   = fma2( cS, U( rS ), cSE, U( rS + 1 ), acc );
+      T up  = fma2( cTC, U( rT ), cTW, U( rT - 1 ) );
+      up    = fma2( cTS, U( rTS ), cTSE, U( rTS + 1 ), up );
+      T dn  = fma2( cBC, U( rB ), cBE, U( rB + 1 ) );
+      dn    = fma2( cBN, U( rBN ), cBNW, U( rBN - 1 ), dn );
+      acc   = acc + ( up + dn );
 #undef U
       const int o = ( r0 + x ) * NR + r;
-      cu[o]       = ( T( 1 ) - omega ) * cu[o] + relax * ( cb[o] - acc );
+      cu[o]       = sorUpdate( omega, relax, cu[o], cb[o], acc );
    }
 }
 
@@ -659,27 +684,29 @@ __global__ __launch_bounds__( 256 ) void kCellMarch( LV g, const MarchUnit* __re
          {
             if ( out && ( ( x + 2 * yy + 3 * z ) & 3 ) == colour )
             {
-               T acc = cW * Z0l + cE * Z0r;
-               acc += cN * Zp + cNW * Zpl;
-               acc += cS * Zm + cSE * Zmr;
-               acc += cTC * T0 + cTW * T0l;
-               acc += cTS * Tm + cTSE * Tmr;
-               acc += cBC * B0 + cBE * B0r;
-               acc += cBN * Bp + cBNW * Bpl;
+               T acc = fma2( cW, Z0l, cE, Z0r );
+               acc   = fma2( cN, Zp, cNW, Zpl, acc );
+               acc   = fma2( cS, Zm, cSE, Zmr, acc );
+               T up  = fma2( cTC, T0, cTW, T0l );
+               up    = fma2( cTS, Tm, cTSE, Tmr, up );
+               T dn  = fma2( cBC, B0, cBE, B0r );
+               dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+               acc   = acc + ( up + dn );
                const int o = rz0 + x;
-               cy[o]       = ( T( 1 ) - omega ) * Z0 + relax * ( cb[o] - acc );
+               cy[o]       = sorUpdate( omega, relax, Z0, cb[o], acc );
             }
          }
          else if ( out )
          {
             T acc = cC * Z0;
-            acc += cW * Z0l + cE * Z0r;
-            acc += cN * Zp + cNW * Zpl;
-            acc += cS * Zm + cSE * Zmr;
-            acc += cTC * T0 + cTW * T0l;
-            acc += cTS * Tm + cTSE * Tmr;
-            acc += cBC * B0 + cBE * B0r;
-            acc += cBN * Bp + cBNW * Bpl;
+            acc   = fma2( cW, Z0l, cE, Z0r, acc );
+            acc   = fma2( cN, Zp, cNW, Zpl, acc );
+            acc   = fma2( cS, Zm, cSE, Zmr, acc );
+            T up  = fma2( cTC, T0, cTW, T0l );
+            up    = fma2( cTS, Tm, cTSE, Tmr, up );
+            T dn  = fma2( cBC, B0, cBE, B0r );
+            dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+            acc   = acc + ( up + dn );
             const int o = rz0 + x;
             if ( MODE == kReplace )
                cy[o] = acc;
@@ -707,13 +734,13 @@ __global__ __launch_bounds__( 256 ) void kCellMarch( LV g, const MarchUnit* __re
 // loads of R windows are in flight together.  MarchUnit fields here: cell, z, x0 = first output element
 // ws of the first window, y0 = row of element ws - 1.
 template < typename T, int MODE, int R >
-__global__ __launch_bounds__( 256 ) void kCellFlat( LV g, const MarchUnit* __restrict__ units, int64_t nUnits,
-                                                    const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
-                                                    const T* u, T* y, const T* b, T omega, int colour, int rows )
+__device__ __forceinline__ void cellFlat_b( int64_t blk, LV g, const MarchUnit* __restrict__ units, int64_t nUnits,
+                                            const T* __restrict__ W8, const int* __restrict__ ctype, int flag, const T* u,
+                                            T* y, const T* b, T omega, int colour, int rows )
 {
    const int     wpb  = blockDim.x >> 6;
    const int     wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
-   const int64_t ui   = xcdBlock( ( nUnits + wpb - 1 ) / wpb ) * wpb + wave;
+   const int64_t ui   = xcdBlockOf( blk, ( nUnits + wpb - 1 ) / wpb ) * wpb + wave;
    if ( ui >= nUnits ) return;
    const MarchUnit U = units[ui];
    if ( !( ctype[U.cell] & flag ) ) return;
@@ -774,26 +801,28 @@ __global__ __launch_bounds__( 256 ) void kCellFlat( LV g, const MarchUnit* __res
       {
          if ( out && ( ( x + 2 * yy + 3 * z ) & 3 ) == colour )
          {
-            T acc = cW * Z0l + cE * Z0r;
-            acc += cN * Zp + cNW * Zpl;
-            acc += cS * Zm + cSE * Zmr;
-            acc += cTC * T0 + cTW * T0l;
-            acc += cTS * Tm + cTSE * Tmr;
-            acc += cBC * B0 + cBE * B0r;
-            acc += cBN * Bp + cBNW * Bpl;
-            cy[o] = ( T( 1 ) - omega ) * Z0 + relax * ( cb[o] - acc );
+            T acc = fma2( cW, Z0l, cE, Z0r );
+            acc   = fma2( cN, Zp, cNW, Zpl, acc );
+            acc   = fma2( cS, Zm, cSE, Zmr, acc );
+            T up  = fma2( cTC, T0, cTW, T0l );
+            up    = fma2( cTS, Tm, cTSE, Tmr, up );
+            T dn  = fma2( cBC, B0, cBE, B0r );
+            dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+            acc   = acc + ( up + dn );
+            cy[o] = sorUpdate( omega, relax, Z0, cb[o], acc );
          }
       }
       else if ( out )
       {
          T acc = cC * Z0;
-         acc += cW * Z0l + cE * Z0r;
-         acc += cN * Zp + cNW * Zpl;
-         acc += cS * Zm + cSE * Zmr;
-         acc += cTC * T0 + cTW * T0l;
-         acc += cTS * Tm + cTSE * Tmr;
-         acc += cBC * B0 + cBE * B0r;
-         acc += cBN * Bp + cBNW * Bpl;
+         acc   = fma2( cW, Z0l, cE, Z0r, acc );
+         acc   = fma2( cN, Zp, cNW, Zpl, acc );
+         acc   = fma2( cS, Zm, cSE, Zmr, acc );
+         T up  = fma2( cTC, T0, cTW, T0l );
+         up    = fma2( cTS, Tm, cTSE, Tmr, up );
+         T dn  = fma2( cBC, B0, cBE, B0r );
+         dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+         acc   = acc + ( up + dn );
          if ( MODE == kReplace )
             cy[o] = acc;
          else if ( MODE == kAdd )
@@ -803,6 +832,14 @@ __global__ __launch_bounds__( 256 ) void kCellFlat( LV g, const MarchUnit* __res
       }
    }
    }
+}
+
+template < typename T, int MODE, int R >
+__global__ __launch_bounds__( 256 ) void kCellFlat( LV g, const MarchUnit* __restrict__ units, int64_t nUnits,
+                                                    const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
+                                                    const T* u, T* y, const T* b, T omega, int colour, int rows )
+{
+   cellFlat_b< T, MODE, R >( blockIdx.x, g, units, nUnits, W8, ctype, flag, u, y, b, omega, colour, rows );
 }
 
 // LDS-staged slab tiles (schedule kind 2).  A workgroup owns rows y in [ya, ya+R) of one macro-cell for the
@@ -880,25 +917,27 @@ __global__ __launch_bounds__( 256 ) void kCellTile( LV g, const MarchUnit* __res
             const int o = go + x;
             if ( MODE == kMarchSor )
             {
-               T acc = cW * Z0l + cE * Z0r;
-               acc += cN * Zp + cNW * Zpl;
-               acc += cS * Zm + cSE * Zmr;
-               acc += cTC * T0 + cTW * T0l;
-               acc += cTS * Tm + cTSE * Tmr;
-               acc += cBC * B0 + cBE * B0r;
-               acc += cBN * Bp + cBNW * Bpl;
-               cy[o] = ( T( 1 ) - omega ) * Z0 + relax * ( cb[o] - acc );
+               T acc = fma2( cW, Z0l, cE, Z0r );
+               acc   = fma2( cN, Zp, cNW, Zpl, acc );
+               acc   = fma2( cS, Zm, cSE, Zmr, acc );
+               T up  = fma2( cTC, T0, cTW, T0l );
+               up    = fma2( cTS, Tm, cTSE, Tmr, up );
+               T dn  = fma2( cBC, B0, cBE, B0r );
+               dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+               acc   = acc + ( up + dn );
+               cy[o] = sorUpdate( omega, relax, Z0, cb[o], acc );
             }
             else
             {
                T acc = cC * Z0;
-               acc += cW * Z0l + cE * Z0r;
-               acc += cN * Zp + cNW * Zpl;
-               acc += cS * Zm + cSE * Zmr;
-               acc += cTC * T0 + cTW * T0l;
-               acc += cTS * Tm + cTSE * Tmr;
-               acc += cBC * B0 + cBE * B0r;
-               acc += cBN * Bp + cBNW * Bpl;
+               acc   = fma2( cW, Z0l, cE, Z0r, acc );
+               acc   = fma2( cN, Zp, cNW, Zpl, acc );
+               acc   = fma2( cS, Zm, cSE, Zmr, acc );
+               T up  = fma2( cTC, T0, cTW, T0l );
+               up    = fma2( cTS, Tm, cTSE, Tmr, up );
+               T dn  = fma2( cBC, B0, cBE, B0r );
+               dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+               acc   = acc + ( up + dn );
                if ( MODE == kReplace )
                   cy[o] = acc;
                else if ( MODE == kAdd )
@@ -1007,14 +1046,15 @@ __global__ __launch_bounds__( 1024 ) void kCellSorSmall( LV g, const int* __rest
                  Zmr = cu[rS + 1];
          const T T0 = cu[rT], T0l = cu[rT - 1], Tm = cu[rTS], Tmr = cu[rTS + 1];
          const T B0 = cu[rB], B0r = cu[rB + 1], Bp = cu[rBN], Bpl = cu[rBN - 1];
-         T       acc = cW * Z0l + cE * Z0r;
-         acc += cN * Zp + cNW * Zpl;
-         acc += cS * Zm + cSE * Zmr;
-         acc += cTC * T0 + cTW * T0l;
-         acc += cTS * Tm + cTSE * Tmr;
-         acc += cBC * B0 + cBE * B0r;
-         acc += cBN * Bp + cBNW * Bpl;
-         cu[r0] = ( T( 1 ) - omega ) * Z0 + relax * ( cb[r0] - acc );
+         T       acc = fma2( cW, Z0l, cE, Z0r );
+         acc   = fma2( cN, Zp, cNW, Zpl, acc );
+         acc   = fma2( cS, Zm, cSE, Zmr, acc );
+         T up  = fma2( cTC, T0, cTW, T0l );
+         up    = fma2( cTS, Tm, cTSE, Tmr, up );
+         T dn  = fma2( cBC, B0, cBE, B0r );
+         dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+         acc   = acc + ( up + dn );
+         cu[r0] = sorUpdate( omega, relax, Z0, cb[r0], acc );
       }
       __syncthreads(); // the next colour reads this colour's values
    }
@@ -1270,14 +1310,15 @@ __global__ __launch_bounds__( 1024, sizeof( T ) == 4 ? 8 : 4 ) void kCellSorTile
          const T  Z0 = Zs[0], Z0l = Zs[-1], Z0r = Zs[1], Zp = Zs[RP], Zpl = Zs[RP - 1], Zm = Zs[-RP], Zmr = Zs[1 - RP];
          const T  T0 = Ts[0], T0l = Ts[-1], Tm = Ts[-RP], Tmr = Ts[1 - RP];
          const T  B0 = Bs[0], B0r = Bs[1], Bp = Bs[RP], Bpl = Bs[RP - 1];
-         T        acc = cW * Z0l + cE * Z0r;
-         acc += cN * Zp + cNW * Zpl;
-         acc += cS * Zm + cSE * Zmr;
-         acc += cTC * T0 + cTW * T0l;
-         acc += cTS * Tm + cTSE * Tmr;
-         acc += cBC * B0 + cBE * B0r;
-         acc += cBN * Bp + cBNW * Bpl;
-         lds[sl * RS + uq[j]] = ( T( 1 ) - omega ) * Z0 + relax * ( bbuf[P][j] - acc );
+         T        acc = fma2( cW, Z0l, cE, Z0r );
+         acc   = fma2( cN, Zp, cNW, Zpl, acc );
+         acc   = fma2( cS, Zm, cSE, Zmr, acc );
+         T up  = fma2( cTC, T0, cTW, T0l );
+         up    = fma2( cTS, Tm, cTSE, Tmr, up );
+         T dn  = fma2( cBC, B0, cBE, B0r );
+         dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+         acc   = acc + ( up + dn );
+         lds[sl * RS + uq[j]] = sorUpdate( omega, relax, Z0, bbuf[P][j], acc );
       }
       storeSlab( ( tm + 2 ) & ( RING - 1 ), xbuf[( P + 2 ) % ( DP + 1 )] );
       __syncthreads();
@@ -1382,15 +1423,15 @@ __global__ __launch_bounds__( 256 ) void kCellSorBand( LV g, int nCells, const i
 // into 0 and such values reach no output.  NT: stores marked non-temporal (streamed past the caches).
 // MarchUnit fields: cell, z = za | zEnd << 16, x0 = ws, y0 = row of element ws - 1 in slab za.
 template < typename T, int MODE, int D, int NT >
-__global__ __launch_bounds__( 1024 ) void kCellColumn( LV g, const MarchUnit* __restrict__ units, int64_t nUnits,
-                                                      const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
-                                                      const T* u, T* y, const T* b, T omega, int colour, int rows,
-                                                      float* rlow, double* partials )
+__device__ __forceinline__ void cellColumn_b( int64_t blk, LV g, const MarchUnit* __restrict__ units, int64_t nUnits,
+                                              const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
+                                              const T* u, T* y, const T* b, T omega, int colour, float* rlow,
+                                              double* partials )
 {
    constexpr int NS   = 3 + D;
    const int     wpb  = blockDim.x >> 6;
    const int     wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
-   const int64_t ui   = xcdBlock( ( nUnits + wpb - 1 ) / wpb ) * wpb + wave;
+   const int64_t ui   = xcdBlockOf( blk, ( nUnits + wpb - 1 ) / wpb ) * wpb + wave;
    if ( ui >= nUnits ) return;
    const MarchUnit U = units[ui];
    if ( !( ctype[U.cell] & flag ) )
@@ -1486,26 +1527,28 @@ __global__ __launch_bounds__( 1024 ) void kCellColumn( LV g, const MarchUnit* __
          // every lane computes, only output lanes store (branch-free, see CellBuf::store)
          if ( MODE == kMarchSor )
          {
-            T acc = cW * Z0l + cE * Z0r;
-            acc += cN * Zp + cNW * Zpl;
-            acc += cS * Zm + cSE * Zmr;
-            acc += cTC * T0 + cTW * T0l;
-            acc += cTS * Tm + cTSE * Tmr;
-            acc += cBC * B0 + cBE * B0r;
-            acc += cBN * Bp + cBNW * Bpl;
-            cy.template store< NT ? 2 : 0 >( Po, ( T( 1 ) - omega ) * Z0 + relax * ( vb[sZ] - acc ),
+            T acc = fma2( cW, Z0l, cE, Z0r );
+            acc   = fma2( cN, Zp, cNW, Zpl, acc );
+            acc   = fma2( cS, Zm, cSE, Zmr, acc );
+            T up  = fma2( cTC, T0, cTW, T0l );
+            up    = fma2( cTS, Tm, cTSE, Tmr, up );
+            T dn  = fma2( cBC, B0, cBE, B0r );
+            dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+            acc   = acc + ( up + dn );
+            cy.template store< NT ? 2 : 0 >( Po, sorUpdate( omega, relax, Z0, vb[sZ], acc ),
                                               out && ( ( x + 2 * yy + 3 * z ) & 3 ) == colour );
          }
          else
          {
             T acc = cC * Z0;
-            acc += cW * Z0l + cE * Z0r;
-            acc += cN * Zp + cNW * Zpl;
-            acc += cS * Zm + cSE * Zmr;
-            acc += cTC * T0 + cTW * T0l;
-            acc += cTS * Tm + cTSE * Tmr;
-            acc += cBC * B0 + cBE * B0r;
-            acc += cBN * Bp + cBNW * Bpl;
+            acc   = fma2( cW, Z0l, cE, Z0r, acc );
+            acc   = fma2( cN, Zp, cNW, Zpl, acc );
+            acc   = fma2( cS, Zm, cSE, Zmr, acc );
+            T up  = fma2( cTC, T0, cTW, T0l );
+            up    = fma2( cTS, Tm, cTSE, Tmr, up );
+            T dn  = fma2( cBC, B0, cBE, B0r );
+            dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
+            acc   = acc + ( up + dn );
             if constexpr ( MODE == kResidualSplit )
             {
                const T r = vb[sZ] - acc;
@@ -1525,6 +1568,15 @@ __global__ __launch_bounds__( 1024 ) void kCellColumn( LV g, const MarchUnit* __
       nsum = waveSum( nsum );
       if ( lane == 0 ) partials[ui] = nsum;
    }
+}
+
+template < typename T, int MODE, int D, int NT >
+__global__ __launch_bounds__( 1024 ) void kCellColumn( LV g, const MarchUnit* __restrict__ units, int64_t nUnits,
+                                                      const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
+                                                      const T* u, T* y, const T* b, T omega, int colour, float* rlow,
+                                                      double* partials )
+{
+   cellColumn_b< T, MODE, D, NT >( blockIdx.x, g, units, nUnits, W8, ctype, flag, u, y, b, omega, colour, rlow, partials );
 }
 
 // --------------------------------------------------------------------------------------------------------
@@ -1910,6 +1962,48 @@ __device__ __forceinline__ void kVertexApply_b( const Blk& B, LV g, const Vertex
       y[o] += acc;
    else
       y[o] = b[o] - acc;
+}
+
+// What the macro-cell part of a merged apply needs: the work units of the level's schedule (KIND 1 flat windows, 3
+// column march; both 4 waves per workgroup).
+template < typename T >
+struct CellPart
+{
+   const MarchUnit* units;
+   int64_t          nUnits;
+   const T*         W;
+   const int*       ctype;
+   int              rows;
+};
+
+// Apply / residual of all primitives in one launch (LowGrid): its parts read only src (and b) and write disjoint points
+// of dst.  The vertex, edge and face workgroups come first: they wait on scattered cell reads while the macro-cell
+// workgroups behind them stream (spread evenly among the cell workgroups, or after them, both lose a little).  One
+// launch against two, with the closure refresh before it, us: FP64 48 macro-tets level 3 16.0 -> 12.5, level 6 32.3 ->
+// 26.8, level 7 137 -> 129, level 8 793 -> 783; FP32 162 macro-tets level 6 50.8 -> 44.5, 48 at level 8 467 -> 448.
+template < typename T, int MODE, int KIND, int D >
+__global__ __launch_bounds__( 256 ) void kApply( LowGrid L, LV g, const VertexGeom* __restrict__ vg,
+                                                 const int64_t* __restrict__ vterms, int nV, const T* __restrict__ VW,
+                                                 const EdgeGeom* __restrict__ eg, const EdgeTerm* __restrict__ eterms,
+                                                 const T* __restrict__ EW, const FaceGeom* __restrict__ fg,
+                                                 const T* __restrict__ FW, int flag, CellPart< T > C, const T* u, T* y,
+                                                 const T* b )
+{
+   Blk       B;
+   const int part = lowPart( L, B );
+   if ( part == 0 )
+      kVertexApply_b< T, 1, MODE >( B, g, vg, vterms, nV, VW, flag, u, y, b );
+   else if ( part == 1 )
+      kEdgeApply_b< T, 1, MODE >( B, g, eg, eterms, EW, flag, u, y, b );
+   else if ( part == 2 )
+      kFaceApply_b< T, 1, MODE >( B, g, fg, FW, flag, u, y, b );
+   else if ( part == 3 )
+   {
+      if constexpr ( KIND == 3 )
+         cellColumn_b< T, MODE, D, 0 >( B.x, g, C.units, C.nUnits, C.W, C.ctype, flag, u, y, b, T( 0 ), 0, nullptr, nullptr );
+      else
+         cellFlat_b< T, MODE, D >( B.x, g, C.units, C.nUnits, C.W, C.ctype, flag, u, y, b, T( 0 ), 0, C.rows );
+   }
 }
 
 // vertex, edge and face parts of an apply / residual in one launch (LowGrid)
@@ -2405,13 +2499,14 @@ __global__ __launch_bounds__( 64 * ( 2 * kResBandY + 1 ), 8 ) void kResidualRest
          const int       oT = idx( x, y, z + 1 ), oTS = idx( x, y - 1, z + 1 );
          const int       oB = idx( x, y, z - 1 ), oBN = idx( x, y + 1, z - 1 );
          T               acc = cC * cu[o];
-         acc += cW * cu[o - 1] + cE * cu[o + 1];
-         acc += cN * cu[oN] + cNW * cu[oN - 1];
-         acc += cS * cu[oS] + cSE * cu[oS + 1];
-         acc += cTC * cu[oT] + cTW * cu[oT - 1];
-         acc += cTS * cu[oTS] + cTSE * cu[oTS + 1];
-         acc += cBC * cu[oB] + cBE * cu[oB + 1];
-         acc += cBN * cu[oBN] + cBNW * cu[oBN - 1];
+         acc   = fma2( cW, cu[o - 1], cE, cu[o + 1], acc );
+         acc   = fma2( cN, cu[oN], cNW, cu[oN - 1], acc );
+         acc   = fma2( cS, cu[oS], cSE, cu[oS + 1], acc );
+         T up  = fma2( cTC, cu[oT], cTW, cu[oT - 1] );
+         up    = fma2( cTS, cu[oTS], cTSE, cu[oTS + 1], up );
+         T dn  = fma2( cBC, cu[oB], cBE, cu[oB + 1] );
+         dn    = fma2( cBN, cu[oBN], cBNW, cu[oBN - 1], dn );
+         acc   = acc + ( up + dn );
          cr.store( o, cb[o] - acc, true );
       }
 
@@ -2445,13 +2540,14 @@ __global__ __launch_bounds__( 64 * ( 2 * kResBandY + 1 ), 8 ) void kResidualRest
    auto residual = [&]( int z, int sB, int sZ, int sT, bool store ) {
       const T Z0 = v0[sZ], Zp = vp[sZ], Zm = vm[sZ], T0 = v0[sT], Tm = vm[sT], B0 = v0[sB], Bp = vp[sB];
       T       acc = cC * Z0;
-      acc += cW * laneDown( Z0 ) + cE * laneUp( Z0 );
-      acc += cN * Zp + cNW * laneDown( Zp );
-      acc += cS * Zm + cSE * laneUp( Zm );
-      acc += cTC * T0 + cTW * laneDown( T0 );
-      acc += cTS * Tm + cTSE * laneUp( Tm );
-      acc += cBC * B0 + cBE * laneUp( B0 );
-      acc += cBN * Bp + cBNW * laneDown( Bp );
+      acc   = fma2( cW, laneDown( Z0 ), cE, laneUp( Z0 ), acc );
+      acc   = fma2( cN, Zp, cNW, laneDown( Zp ), acc );
+      acc   = fma2( cS, Zm, cSE, laneUp( Zm ), acc );
+      T up  = fma2( cTC, T0, cTW, laneDown( T0 ) );
+      up    = fma2( cTS, Tm, cTSE, laneUp( Tm ), up );
+      T dn  = fma2( cBC, B0, cBE, laneUp( B0 ) );
+      dn    = fma2( cBN, Bp, cBNW, laneDown( Bp ), dn );
+      acc   = acc + ( up + dn );
       const int  lim = w - 2 - y - z, xo = opaqueInt( x ); // last interior x of the row
       const bool in  = xo <= lim;
       const T    rv  = in ? vb[sZ] - acc : T( 0 );
@@ -3295,7 +3391,7 @@ void marchLaunch( Mesh& M, LevelPlan& P, const T* CW, int flag, const T* u, T* y
                        omega, colour, S.rows )
 #define HYMI_COLUMN( DD, NT )                                                                                      \
    hipLaunchKernelGGL( ( kCellColumn< T, MODE, DD, NT > ), grid, block, 0, s, g, mu, n, CW, P.dCellType.p, flag, u, y,  \
-                       b, omega, colour, S.rows, rlow, partials )
+                       b, omega, colour, rlow, partials )
    if constexpr ( MODE == kResidualSplit )
    {
       if ( S.kind != 3 ) throw std::logic_error( "the split residual needs the column schedule" );
@@ -3626,6 +3722,44 @@ void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, in
       lg.nxF = (int) blocksFor( m * ( m + 1 ) / 2 * NR, 256 );
       lg.nyF = nF;
    }
+   if constexpr ( NR == 1 )
+      if ( level >= 2 && cells )
+      {
+         CellPart< T > C{ nullptr, 0, CW, P.dCellType.p, 0 };
+         C.units                = M.marchUnits( P, &C.nUnits );
+         const MarchSchedule& S = P.sched;
+         C.rows                 = S.rows;
+         // the merged launch knows the default schedules (always four waves per workgroup); others run as a launch of
+         // their own.  The values are the same, bit for bit
+         if ( C.nUnits > 0 && S.waves <= 4 && S.block == 1 && ( S.kind == 3 || S.kind == 1 ) )
+         {
+            lg.nbC = (int) xcdGrid( ( C.nUnits + 3 ) / 4 );
+#define HYMI_APPLY( MODE, KIND )                                                                                     \
+   hipLaunchKernelGGL( ( kApply< T, MODE, KIND, 1 > ), dim3( lowBlocks( lg ) ), dim3( 256 ), 0, s, lg, g,              \
+                       P.dVertexGeom.p, P.dVertexTerms.p, nV, VW, P.dEdgeGeom.p, P.dEdgeTerms.p, EW, P.dFaceGeom.p, FW, \
+                       flag, C, u, y, b )
+            if ( S.kind == 3 )
+            {
+               if ( mode == kReplace )
+                  HYMI_APPLY( kReplace, 3 );
+               else if ( mode == kAdd )
+                  HYMI_APPLY( kAdd, 3 );
+               else
+                  HYMI_APPLY( kResidual, 3 );
+            }
+            else
+            {
+               if ( mode == kReplace )
+                  HYMI_APPLY( kReplace, 1 );
+               else if ( mode == kAdd )
+                  HYMI_APPLY( kAdd, 1 );
+               else
+                  HYMI_APPLY( kResidual, 1 );
+            }
+#undef HYMI_APPLY
+            return;
+         }
+      }
    LAUNCH_MODES( kLowApply, dim3( lowBlocks( lg ) ), dim3( 256 ), lg, g, P.dVertexGeom.p, P.dVertexTerms.p, nV, VW,
                  P.dEdgeGeom.p, P.dEdgeTerms.p, EW, P.dFaceGeom.p, FW, flag, u, y, b );
    if ( level >= 2 && cells ) cellApplyLaunch< T, NR >( M, P, CW, flag, mode, u, y, b );
