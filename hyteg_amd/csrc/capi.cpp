@@ -1402,6 +1402,8 @@ int hymi_gmg_create( hymi_operator op, hymi_function xt, int minL, int maxL, int
          if ( g->nrhs > 1 ) M.segments( P, kRowSeg, &n ); // cell apply, SOR and prolongation, several right-hand sides
          M.marchUnits( P, &n );
          M.transferUnits( P, &n );
+         int perCell = 0;
+         if ( g->nrhs == 1 ) M.prolongUnits( P, &perCell );
          if ( g->nrhs == 1 ) M.faceGhost( P );
          M.closureRanges( P, kInner | kNeumann, &n );
          M.closureRanges( P, kInner | kNeumann | kFreeslip, &n );

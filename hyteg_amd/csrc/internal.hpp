@@ -134,6 +134,10 @@ struct LevelPlan
    // grid-transfer kernels; fields as for the flat macro-cell kernel (x0 = first element, y0 = its row)
    std::unique_ptr< DevBuf< MarchUnit > > transfer;
    int64_t                                transferCount = -1;
+   // work units of the prolongation to this level, of one macro-cell (the same for every cell): 64-element windows of
+   // slab za marched up to zEnd, z = za | zEnd << 16, za odd, x0 = first element
+   std::unique_ptr< DevBuf< MarchUnit > > prolong;
+   int                                    prolongPerCell = -1;
    // work units of the fused residual-and-restriction kernel (this level as the coarse one): cell, run of coarse
    // slabs Za | Zb << 16, x0, y0 of the tile (1 + multiples of kResBandX, kResBandY), longest runs first; then the fine
    // points next to the faces that no tile computes, as (0, z, x, y)
@@ -179,6 +183,7 @@ struct Mesh
    const CellSeg* segments( LevelPlan& P, int len, int64_t* count );
    const MarchUnit* marchUnits( LevelPlan& P, int64_t* count );
    const MarchUnit* transferUnits( LevelPlan& P, int64_t* count );
+   const MarchUnit* prolongUnits( LevelPlan& P, int* perCell );
    const MarchUnit* residualRestrictUnits( LevelPlan& Pc, int64_t* count, int* extra );
    // face ghost buffer of level P (allocated on first use)
    void* faceGhost( LevelPlan& P );

@@ -2805,134 +2805,84 @@ __global__ __launch_bounds__( 256 ) void kProlongCell( LV gc, LV gf, const CellS
    }
 }
 
-// the windows of one unit of the flat prolongation: fine and coarse values loaded, fine offsets, and whether
-// the lane's element is an interior point (a lane without one reads index 0 and stores nothing)
-template < typename T >
-struct ProlongWindows
-{
-   T    fv[kTransferWindows], ca[kTransferWindows], cb[kTransferWindows];
-   int  fo[kTransferWindows];
-   bool ok[kTransferWindows];
-};
-
+// Column form for one right-hand side: a wave takes 64 consecutive elements of slab za of one macro-cell (unit:
+// z = za | zEnd << 16 with za odd, x0 = first element, the units of one cell, the same for every cell)
+// and marches these positions (x, y) up through slabs za .. zEnd.  What bounded the flat form (64-element windows of
+// one slab) was its index arithmetic, about 60 vector instructions per window; here a position's row and parities are
+// found once per unit, and a step advances the fine index by W (W + 1) / 2 - y (W: width of the slab) and, every
+// second step, the coarse row start by the same rule.  With h = y / 2, hx = x / 2 and Q(Z) the coarse index of row h,
+// column hx of coarse slab Z, (p - d) / 2 and (p + d) / 2 (prolongDir) are, for odd z = 2Z + 1,
+//   Q(Z) + [y odd] (W_Z - h) + [x odd, y even]  and  Q(Z + 1) + [x odd, y odd],
+// and for even z = 2Z
+//   Q(Z) + [x odd, y odd] (W_Z - h)  and  Q(Z) + [x even, y odd] (W_Z - h) + [x odd].
+// Slabs are taken kProlongGroup at a time, all loads of a group before its stores.  Closure positions are written too
+// (with the interpolation along the closure; every reader of a closure refreshes it first): left out, each row would
+// have a hole, and its lines would go to memory in parts.  A replacement of an array larger than the memory-side cache
+// (kStreamBytes) is written with non-temporal stores.  Bound by memory traffic now.  With the coarse refresh, 48
+// macro-tets, level 8, us: replacement FP32 296 -> 192 in turn with other work, 172 alone (265 with ordinary stores), FP64 600 -> 282 (448);
+// level 7 FP64 49 -> 41 (49 with non-temporal stores); addition FP32 333 -> 299, FP64 551 -> 552 (4.6 TB/s).  Units of 8
+// slabs: 4 or 16 are 2 to 30 % slower.
+constexpr int     kProlongGroup = 8;
+constexpr int64_t kStreamBytes  = int64_t( 256 ) << 20; // the card's memory-side cache
 template < typename T, bool REPL >
-__device__ __forceinline__ void prolongFlatLoad( const MarchUnit& U, bool active, int lane, LV gc, LV gf,
-                                                 const T* __restrict__ uc, T* __restrict__ uf, ProlongWindows< T >& P )
+__device__ __forceinline__ void kProlongColumn_b( const Blk& B, LV gc, LV gf, const MarchUnit* __restrict__ units,
+                                                  int perCell, int nUnits, const int* __restrict__ ctype, int flag,
+                                                  const T* __restrict__ uc, T* __restrict__ uf, bool stream )
 {
-#pragma unroll
-   for ( int j = 0; j < kTransferWindows; j++ )
+   const int ui = (int) xcdBlockOf( B.x, ( nUnits + 3 ) / 4 ) * 4 + __builtin_amdgcn_readfirstlane( B.tid >> 6 );
+   if ( ui >= nUnits ) return;
+   const int cell = ui / perCell;
+   if ( !( ctype[cell] & flag ) ) return;
+   const MarchUnit    U    = units[ui - cell * perCell];
+   const int          lane = B.tid & 63, w = gf.w, wc = gc.w, za = U.z & 0xffff, zEnd = U.z >> 16, Wa = w - za;
+   const CellBuf< T > cu( uc + gc.offC + (int64_t) cell * gc.cS, gc.cS );
+   const CellBuf< T > fu( uf + gf.offC + (int64_t) cell * gf.cS, gf.cS );
+   const int          nEl = Wa * ( Wa + 1 ) / 2, e = U.x0 + lane, y = triRow32( Wa, min( e, nEl - 1 ) );
+   const int          x = e - y * ( 2 * Wa + 1 - y ) / 2;
+   // last slab that holds the position, closure included (a lane without one reads and writes nothing)
+   const int zLast = e < nEl ? min( zEnd, w - 1 - x - y ) : -1;
+   const int px = x & 1, py = y & 1, h = y >> 1;
+   const int oy = -py, oxy = -( px & py ), oy0 = -( py & ~px ); // masks: y odd; x, y odd; x even, y odd
+   int       Pf = tet32( w ) - tet32( Wa ) + e, Wf = Wa;
+   int       Wm = wc - ( za >> 1 ), Q = tet32( wc ) - tet32( Wm ) + h * ( Wm + 1 ) - ( h * ( h + 1 ) >> 1 ) + ( x >> 1 );
+   for ( int z = za; z <= zEnd; z += kProlongGroup )
    {
-      P.ok[j] = false;
-      P.fo[j] = 0;
-   }
-   if ( !active ) return;
-   const int w = gf.w, z = U.z, Wd = w - z, wc = gc.w;
-   const int tf = tet32( w ), tc = tet32( wc );
-   const int nEl = Wd * ( Wd + 1 ) / 2;
-   const int S0  = tf - tet32( Wd );
-   const int pz  = z & 1;
-   // coarse slabs of (p - d) / 2 and (p + d) / 2 and their widths
-   const int Zm = ( z - pz ) / 2, Zp = ( z + pz ) / 2;
-   const int Cm = tc - tet32( wc - Zm ), Cp = tc - tet32( wc - Zp ); // coarse slab starts
-   const int Wm = wc - Zm, Wp = wc - Zp;
-   const CellBuf< T > cu( uc + gc.offC + (int64_t) U.cell * gc.cS, gc.cS );
-   const CellBuf< T > fu( uf + gf.offC + (int64_t) U.cell * gf.cS, gf.cS );
-   auto      rs = [&]( int WW, int yy ) { return yy * ( WW + 1 ) - ( yy * ( yy + 1 ) >> 1 ); };
-   int       e0 = U.x0;
-   // the lane's row yy, its start rowS and the next row's start rowE
-   int yy = U.y0, rowS = rs( Wd, U.y0 ), rowE = rowS + Wd - U.y0;
+      T   ca[kProlongGroup], cb[kProlongGroup], fv[kProlongGroup];
+      int fo[kProlongGroup];
 #pragma unroll
-   for ( int j = 0; j < kTransferWindows; j++, e0 += 64 )
-   {
-      int im = 0, ip = 0;
-      if ( e0 < nEl )
+      for ( int k = 0; k < kProlongGroup; k++ )
       {
-         const int e = e0 + lane;
-         while ( e >= rowE && yy < Wd - 1 )
+         const bool ok = z + k <= zLast;
+         const int  up = Wm - h; // from row h to row h + 1
+         int        im, ip;
+         if ( k % 2 == 0 ) // odd slab
          {
-            yy++;
-            rowS = rowE;
-            rowE += Wd - yy;
+            im = Q + ( oy & up ) + ( px & ~py );
+            Q += Wm * ( Wm + 1 ) / 2 - h;
+            Wm--;
+            ip = Q + ( px & py );
          }
-         const int x = e - rowS;
-         P.ok[j]     = e < nEl && x >= 1 && yy >= 1 && x + yy <= Wd - 2;
-         if ( P.ok[j] )
+         else
          {
-            // prolongDir's direction: dy = -1 for odd y unless x and z are even (then +1), dx = -1 for odd x
-            // with odd z and even y, else the parity of x
-            const int  px = x & 1, py = yy & 1, h = yy >> 1, hx = x >> 1;
-            const int  rm = rs( Wm, h ), rp = rm - ( pz ? h : 0 ); // row h of the coarse slabs Zm, Zp
-            const bool dyNeg = py && ( px || pz ), dyPos = py && !px && !pz;
-            const bool dxNeg = px && pz && !py, dxPos = px && !dxNeg;
-            im      = Cm + ( dyNeg ? rm + Wm - h : rm ) + hx + ( dxNeg ? 1 : 0 );
-            ip      = Cp + ( dyPos ? rp + Wp - h : rp ) + hx + ( dxPos ? 1 : 0 );
-            P.fo[j] = S0 + e;
+            im = Q + ( oxy & up );
+            ip = Q + ( oy0 & up ) + px;
          }
+         ca[k] = cu.load( im, ok );
+         cb[k] = cu.load( ip, ok );
+         fo[k] = Pf;
+         fv[k] = REPL ? T( 0 ) : fu.load( Pf, ok );
+         Pf += Wf * ( Wf + 1 ) / 2 - y;
+         Wf--;
       }
-      P.fv[j] = REPL ? T( 0 ) : fu[P.fo[j]];
-      P.ca[j] = cu[im];
-      P.cb[j] = cu[ip];
-   }
-}
-
-template < typename T >
-__device__ __forceinline__ void prolongFlatStore( const MarchUnit& U, bool active, LV gf, T* __restrict__ uf,
-                                                  const ProlongWindows< T >& P )
-{
-   if ( !active ) return;
-   const CellBuf< T > fu( uf + gf.offC + (int64_t) U.cell * gf.cS, gf.cS );
 #pragma unroll
-   for ( int j = 0; j < kTransferWindows; j++ )
-      fu.store( P.fo[j], P.fv[j] + T( 0.5 ) * ( P.ca[j] + P.cb[j] ), P.ok[j] );
-}
-
-// Flat form for one right-hand side: a wave takes prolongUnitsPerWave consecutive units (Mesh::transferUnits)
-// of kTransferWindows windows of 64 consecutive elements of one fine slab z each, and issues the loads of all
-// before the first store.  In FP32 it takes two (24 loads in flight per lane: a wave that took one unit spent
-// most of its short life waiting for the unit's and the cell type's scalar loads and for one round of vector
-// loads; level 8, 376 -> 310 us); FP64 moves twice the bytes per load and runs near the HBM rate with one
-// (two were 2 % slower).  The coarse
-// indices use 32-bit arithmetic.  The coarse slabs (z -/+ pz) / 2 are wave-uniform because the z-component of
-// the direction always equals the parity of z.  A lane's row starts at the unit's first row and advances over
-// the row ends its elements pass (at most one per window where rows hold 64 or more elements).  With h = y / 2,
-// the coarse rows of (p - d) / 2 and (p + d) / 2 are both h for even y and h, h + 1 in the order the sign of
-// dy gives for odd y, and the start of row h in coarse slab Zp is that in slab Zm less pz h (the slab is pz
-// narrower), so one triangular term serves both; likewise in x with hx = x / 2.
-template < typename T >
-constexpr int prolongUnitsPerWave()
-{
-   return sizeof( T ) == 4 ? 2 : 1;
-}
-template < typename T, bool REPL >
-__device__ __forceinline__ void kProlongFlat_b( const Blk& B, LV gc, LV gf, const MarchUnit* __restrict__ units,
-                                                int64_t nUnits, const int* __restrict__ ctype, int flag,
-                                                const T* __restrict__ uc, T* __restrict__ uf )
-{
-   constexpr int UPW     = prolongUnitsPerWave< T >();
-   const int64_t nGroups = ( nUnits + UPW - 1 ) / UPW;
-   const int64_t gi = xcdBlockOf( B.x, ( nGroups + 3 ) / 4 ) * 4 + __builtin_amdgcn_readfirstlane( B.tid >> 6 );
-   if ( gi >= nGroups ) return;
-   const int64_t   u0   = UPW * gi;
-   const int       lane = B.tid & 63;
-   const MarchUnit U0   = units[u0];
-   const bool      a0   = ( ctype[U0.cell] & flag ) != 0;
-   ProlongWindows< T > P0;
-   if constexpr ( UPW == 2 )
-   {
-      const int64_t   u1 = u0 + 1;
-      const MarchUnit U1 = u1 < nUnits ? units[u1] : U0;
-      const bool      a1 = u1 < nUnits && ( ctype[U1.cell] & flag ) != 0;
-      ProlongWindows< T > P1;
-      prolongFlatLoad< T, REPL >( U0, a0, lane, gc, gf, uc, uf, P0 );
-      prolongFlatLoad< T, REPL >( U1, a1, lane, gc, gf, uc, uf, P1 );
-      prolongFlatStore( U0, a0, gf, uf, P0 );
-      prolongFlatStore( U1, a1, gf, uf, P1 );
-   }
-   else
-   {
-      static_assert( UPW == 1, "one or two units per wave" );
-      prolongFlatLoad< T, REPL >( U0, a0, lane, gc, gf, uc, uf, P0 );
-      prolongFlatStore( U0, a0, gf, uf, P0 );
+      for ( int k = 0; k < kProlongGroup; k++ )
+      {
+         const T v = fv[k] + T( 0.5 ) * ( ca[k] + cb[k] );
+         if ( stream )
+            fu.template store< 2 >( fo[k], v, z + k <= zLast );
+         else
+            fu.store( fo[k], v, z + k <= zLast );
+      }
    }
 }
 
@@ -2997,14 +2947,14 @@ __device__ __forceinline__ void kProlongVertex_b( const Blk& B, const VertexGeom
 }
 
 // a prolongation in one launch (LowGrid): vertex, edge and face parts, and the macro-cell part (one right-hand
-// side: kProlongFlat_b over the fine level's transfer units)
+// side: kProlongColumn_b over the fine level's prolongation units)
 template < typename T, int NR, bool REPL >
 __global__ __launch_bounds__( 256 ) void kLowProlong( LowGrid L, LV gc, LV gf, const VertexGeom* __restrict__ vgFine,
                                                       int nV, const EdgeGeom* __restrict__ egFine,
                                                       const FaceGeom* __restrict__ fgFine, int flag,
                                                       const T* __restrict__ uc, T* __restrict__ uf,
-                                                      const MarchUnit* __restrict__ cellUnits, int64_t nCellUnits,
-                                                      const int* __restrict__ ctypeF )
+                                                      const MarchUnit* __restrict__ cellUnits, int perCell,
+                                                      int nCellUnits, const int* __restrict__ ctypeF, bool stream )
 {
    Blk       B;
    const int part = lowPart( L, B );
@@ -3016,7 +2966,7 @@ __global__ __launch_bounds__( 256 ) void kLowProlong( LowGrid L, LV gc, LV gf, c
       kProlongFace_b< T, NR, REPL >( B, gc, gf, fgFine, flag, uc, uf );
    else if ( part == 3 )
    {
-      if constexpr ( NR == 1 ) kProlongFlat_b< T, REPL >( B, gc, gf, cellUnits, nCellUnits, ctypeF, flag, uc, uf );
+      if constexpr ( NR == 1 ) kProlongColumn_b< T, REPL >( B, gc, gf, cellUnits, perCell, nCellUnits, ctypeF, flag, uc, uf, stream );
    }
 }
 
@@ -4066,16 +4016,17 @@ void prolongT( Function& f, int srcLevel, int flag, bool refreshCoarse )
       lg.nxF = (int) blocksFor( m * ( m + 1 ) / 2 * NR, 256 );
       lg.nyF = nF;
    }
-   int64_t          nu = 0;
-   const MarchUnit* tu = nullptr;
+   int              perCell = 0, nu = 0;
+   const MarchUnit* tu      = nullptr;
    if ( NR == 1 )
    {
-      tu     = M.transferUnits( Pf, &nu );
-      constexpr int upw = prolongUnitsPerWave< T >();
-      lg.nbC            = nu > 0 ? (int) xcdGrid( ( ( nu + upw - 1 ) / upw + 3 ) / 4 ) : 0;
+      tu     = M.prolongUnits( Pf, &perCell );
+      nu     = perCell * M.T.nC();
+      lg.nbC = nu > 0 ? (int) xcdGrid( ( nu + 3 ) / 4 ) : 0;
    }
+   const bool stream = REPL && Pf.total * (int64_t) sizeof( T ) > kStreamBytes;
    hipLaunchKernelGGL( ( kLowProlong< T, NR, REPL > ), dim3( lowBlocks( lg ) ), dim3( 256 ), 0, s, lg, gc, gf, Pf.dVertexGeom.p, nV,
-                       Pf.dEdgeGeom.p, Pf.dFaceGeom.p, flag, uc, uf, tu, nu, Pf.dCellType.p );
+                       Pf.dEdgeGeom.p, Pf.dFaceGeom.p, flag, uc, uf, tu, perCell, nu, Pf.dCellType.p, stream );
    if ( NR == 1 ) return;
    int64_t        nseg = 0;
    rowSegFits< NR >( Pf );

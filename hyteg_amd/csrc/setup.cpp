@@ -801,6 +801,38 @@ const MarchUnit* Mesh::transferUnits( LevelPlan& P, int64_t* count )
    return P.transfer->p;
 }
 
+const MarchUnit* Mesh::prolongUnits( LevelPlan& P, int* perCell )
+{
+   if ( P.prolongPerCell < 0 )
+   {
+      std::vector< MarchUnit > v;
+      const int                w = P.w, Zc = 8; // kProlongGroup slabs, all in flight together
+      for ( int z = 1; z <= w - 4; z += Zc )
+      {
+         const int W     = w - z;
+         const int lastE = slabRowStart( W, W - 3 ) + 1; // the last interior position of the slab
+         for ( int e0 = slabRowStart( W, 1 ) + 1, y = 1; e0 <= lastE; e0 += 64 )
+         {
+            while ( slabRowStart( W, y + 1 ) <= e0 )
+               y++;
+            // the interior position of the window that lies in the most slabs: the least x + y over its rows
+            int least = 1 << 30;
+            for ( int r = y, s = e0; s < e0 + 64 && r <= W - 3; s = slabRowStart( W, ++r ) )
+               if ( const int x = std::max( 1, s - slabRowStart( W, r ) ); slabRowStart( W, r ) + x < e0 + 64 )
+                  least = std::min( least, x + r );
+            const int zEnd = std::min( z + Zc - 1, w - 2 - least );
+            if ( zEnd >= z ) v.push_back( { 0, z | ( zEnd << 16 ), e0, 0 } );
+         }
+      }
+      P.prolong = std::make_unique< DevBuf< MarchUnit > >();
+      P.prolong->upload( v, ctx->stream );
+      HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
+      P.prolongPerCell = (int) v.size();
+   }
+   *perCell = P.prolongPerCell;
+   return P.prolong->p;
+}
+
 // the SOR face phase's scratch: two ghost layers per face and a snapshot of the faces (face layout each)
 void* Mesh::faceGhost( LevelPlan& P )
 {
