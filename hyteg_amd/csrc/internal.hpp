@@ -79,6 +79,12 @@ struct Context
    DevBuf< double > scalars;
    DevBuf< double > modes; // staging of per-call coefficient tables (interpolation of Fourier modes)
    size_t           bytesInUse = 0;
+   // pinned host buffers that owned values pass through on their way to or from the caller's memory (allocated on first
+   // use, kept until the context goes), the event after which each is free, and the lock of the transfer using them
+   static constexpr int kStageValues = 1 << 19;
+   double*              stage[2]     = { nullptr, nullptr };
+   hipEvent_t           staged[2]    = { nullptr, nullptr };
+   std::mutex           stageLock;
 };
 
 // Per-level layout and geometry tables of a mesh (shared by all functions and operators on it).

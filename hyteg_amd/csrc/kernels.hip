@@ -2999,7 +2999,7 @@ __global__ void kLincomb( const Range* __restrict__ ranges, T* __restrict__ dst,
 // Column operations on interleaved functions ([dof][column], NR columns; a Range offset is a dof index, so the
 // column of element o * NR + k is k mod NR).  kColumnSelect zeroes the columns not in `keep`; kColumnAddFrom
 // adds src to dst on the columns in `mask` with the arithmetic of kLincomb's accumulate form
-// (v = constant + c0 src, then v + dst); kColumnGather copies column `col` of n dofs to a contiguous array.
+// (v = constant + c0 src, then v + dst).
 template < typename T, int NR >
 __global__ void kColumnSelect( const Range* __restrict__ ranges, T* __restrict__ dst, unsigned keep )
 {
@@ -3027,11 +3027,51 @@ __global__ void kColumnAddFrom( const Range* __restrict__ ranges, T* __restrict_
       }
 }
 
-template < typename T, int NR >
-__global__ void kColumnGather( const T* __restrict__ src, int64_t n, int col, double* __restrict__ out )
+// Element of owned DoF q (vertices, then edge, face and cell interiors in primitive order) in a function's level.  A
+// cell's slab comes from a binary search over the slab starts of its interior points, which form a tetrahedron of width
+// w - 4; the row of a face or slab from triPos.
+__device__ __forceinline__ int64_t ownedElement( const LV& g, int nV, int nE, int nF, int64_t q )
 {
-   for ( int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (int64_t) gridDim.x * blockDim.x )
-      out[k] = (double) src[k * NR + col];
+   const int w = g.w, mE = w - 2, mF = w - 3, n = w - 4;
+   if ( q < nV ) return q;
+   q -= nV;
+   if ( q < (int64_t) nE * mE ) return g.offE + q / mE * g.eS + 1 + q % mE;
+   q -= (int64_t) nE * mE;
+   const int64_t perF = (int64_t) mF * ( mF + 1 ) / 2, perC = tet( n );
+   int           i, j;
+   if ( q < nF * perF )
+   {
+      triPos( mF, (int) ( q % perF ), i, j );
+      return g.offF + q / perF * g.fS + fidx( w, i + 1, j + 1 );
+   }
+   q -= nF * perF;
+   const int64_t cell = q / perC, rest = perC - q % perC; // points of the cell from this one on
+   int           lo = 1, hi = n; // the slab's width W: tet(W - 1) < rest <= tet(W)
+   while ( lo < hi )
+   {
+      const int mid = ( lo + hi ) >> 1;
+      if ( tet( mid ) >= rest )
+         hi = mid;
+      else
+         lo = mid + 1;
+   }
+   triPos( lo, (int) ( tet( lo ) - rest ), i, j );
+   return g.offC + cell * g.cS + cidx( w, i + 1, j + 1, n - lo + 1 );
+}
+
+// Values of owned DoFs between a function's level and host memory the device can address: value k of the batch is
+// right-hand side k mod NR of DoF q0 + k / NR, or (col >= 0) column col of DoF q0 + k.  Bound by the link to the host.
+template < typename T, int NR, bool UPLOAD >
+__global__ __launch_bounds__( 256 ) void kOwnedValues( LV g, int nV, int nE, int nF, int64_t q0, int n, int col,
+                                                       T* __restrict__ u, double* __restrict__ host )
+{
+   const int k = (int) ( blockIdx.x * 256 + threadIdx.x );
+   if ( k >= n ) return;
+   const int64_t o = ownedElement( g, nV, nE, nF, q0 + ( col < 0 ? k / NR : k ) ) * NR + ( col < 0 ? k % NR : col );
+   if ( UPLOAD )
+      u[o] = (T) host[k];
+   else
+      host[k] = (double) u[o];
 }
 
 template < typename T, int NR >
@@ -4582,23 +4622,28 @@ struct ColumnSelectF
    }
 };
 template < typename T, int NR >
-struct ColumnGatherF
+struct OwnedValuesF
 {
-   static void run( Function& f, int level, int col, double* out )
+   static void run( Function& f, int level, int64_t q0, int n, int col, double* host, bool upload )
    {
-      Mesh&         M = *f.mesh;
-      const int64_t n = M.plan( level ).total;
-      const int64_t blocks = std::min< int64_t >( 4096, ( n + 255 ) / 256 );
-      hipLaunchKernelGGL( ( kColumnGather< T, NR > ), dim3( (unsigned) std::max< int64_t >( 1, blocks ) ), dim3( 256 ), 0,
-                          M.ctx->stream, (const T*) f.ptr( level ), n, col, out );
+      Mesh&      M = *f.mesh;
+      LevelPlan& P = M.plan( level );
+      const dim3 grid( blocksFor( n, 256 ) ), block( 256 );
+      T*         u = (T*) f.ptr( level );
+      if ( upload )
+         hipLaunchKernelGGL( ( kOwnedValues< T, NR, true > ), grid, block, 0, M.ctx->stream, viewOf( P ), M.T.nV(), M.T.nE(),
+                             M.T.nF(), q0, n, col, u, host );
+      else
+         hipLaunchKernelGGL( ( kOwnedValues< T, NR, false > ), grid, block, 0, M.ctx->stream, viewOf( P ), M.T.nV(),
+                             M.T.nE(), M.T.nF(), q0, n, col, u, host );
    }
 };
 
 void launchColumnSelect( Function& f, int level, unsigned keep ) { dispatch< ColumnSelectF >( f.prec, f.nrhs, f, level, keep ); }
 
-void launchColumnGather( Function& f, int level, int col, double* out )
+void launchOwnedValues( Function& f, int level, int64_t q0, int n, int col, double* host, bool upload )
 {
-   dispatch< ColumnGatherF >( f.prec, f.nrhs, f, level, col, out );
+   dispatch< OwnedValuesF >( f.prec, f.nrhs, f, level, q0, n, col, host, upload );
 }
 
 void launchAddFromMasked( Function& x, Function& e, int level, int flag, unsigned mask )

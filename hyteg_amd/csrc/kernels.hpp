@@ -68,8 +68,9 @@ void launchAddFrom( Function& x, Function& e, int level, int flag );
 void launchAddFromMasked( Function& x, Function& e, int level, int flag, unsigned mask );
 // zeroes the columns r without bit r of keep, on every primitive's whole closure array
 void launchColumnSelect( Function& f, int level, unsigned keep );
-// copies column col of the whole level buffer (plan total values) into out (device, FP64)
-void launchColumnGather( Function& f, int level, int col, double* out );
+// n values of owned DoFs from q0 on (every right-hand side, or column col if col >= 0) between the level and host
+// memory that the device can address
+void launchOwnedValues( Function& f, int level, int64_t q0, int n, int col, double* host, bool upload );
 // Residual of iterative refinement: r = b - A x with FP64 x and b; vertex, edge and face values go to r64
 // and, rounded, to rc; cell values go rounded straight to rc; ||r||^2 (FP64, owned DoFs of flag primitives)
 // to scalars[slot].  Needs the column schedule on the level; returns false (nothing launched) otherwise.
