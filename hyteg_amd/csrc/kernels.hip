@@ -2298,6 +2298,217 @@ __global__ __launch_bounds__( 256 ) void kFaceSorFused( LV g, const FaceGeom* __
 }
 
 // --------------------------------------------------------------------------------------------------------
+// fused SOR phases for several right-hand sides (forward sweeps)
+//
+// The columns of an interleaved function do not couple, so a workgroup takes one primitive and RG of its NR columns
+// through a whole phase with barriers between the colours: vertices and edges (with the edges' end copies) in one launch,
+// up to level 5 faces (with the edge-to-face copy) in one, up to level 4 cells (with the face-to-cell copy) in one.  A
+// sweep was thirteen launches, most of them of 4 to 7 us that are latency; it is three (eight at level 5).  Values and
+// expressions are those of the launches they replace; only the vertices' sums (eight slices) and the faces' (off-plane
+// terms first) are ordered anew.  Launches of a sweep, 48 macro-tets, 32 columns, FP32, us, before -> now: vertices and
+// edges 22 -> 10.5; faces 17, 18, 22, 42 at levels 2 to 5 -> 6, 9, 16, 37; cells 18, 21, 25 at levels 2 to 4 -> 7, 11, 14.
+constexpr int kMultiThreads      = 256;
+constexpr int kCellMultiMaxLevel = 4; // 116 points of a colour, 31 KB of LDS per workgroup
+
+// one macro-edge and its two end vertices; LDS (dynamic): 2 w RG values
+template < typename T, int NR, int RG >
+__global__ __launch_bounds__( kMultiThreads ) void kEdgeSorMulti( LV g, const EdgeGeom* __restrict__ eg,
+                                                                  const EdgeTerm* __restrict__ terms,
+                                                                  const T* __restrict__ EW, int flag, T* __restrict__ u,
+                                                                  const T* __restrict__ b, T omega,
+                                                                  const int64_t* __restrict__ vsnap,
+                                                                  const int32_t* __restrict__ ends, const T* __restrict__ VW )
+{
+   constexpr int S = kMultiThreads / ( 2 * RG );
+   static_assert( S >= 1 && NR % RG == 0, "both end vertices' columns fit the workgroup" );
+   extern __shared__ unsigned char smem[];
+   __shared__ T    vpart[S][2][RG];
+   T*              su   = reinterpret_cast< T* >( smem );
+   T*              ts   = su + g.w * RG;
+   const int       edge = (int) blockIdx.x / ( NR / RG ), r0 = (int) blockIdx.x % ( NR / RG ) * RG, w = g.w;
+   const int       tid = (int) threadIdx.x, r = tid % RG;
+   const EdgeGeom& G  = eg[edge]; // edge id = geometry index
+   const int64_t   eo = g.offE + (int64_t) edge * g.eS;
+   for ( int x = tid / RG; x < w; x += kMultiThreads / RG )
+      su[x * RG + r] = u[( eo + x ) * NR + r0 + r];
+   // vertex j's terms from the faces' copies of the edge points (see kEdgeSorFused), in S slices
+   const int      j = tid / RG & 1, sl = tid / ( 2 * RG );
+   const int32_t* en = ends + 10 * (int64_t) edge;
+   const int      v = en[j], vTermOff = en[4 + j], vN = en[6 + j], vType = en[8 + j];
+   const T*       vw = VW + v + vTermOff;
+   T              part = T( 0 );
+   if ( vType & flag )
+      for ( int k = sl; k < vN; k += S )
+         part += vw[1 + k] * u[vsnap[vTermOff + k] * NR + r0 + r];
+   vpart[sl][j][r] = part;
+   __syncthreads();
+   if ( sl == 0 )
+   {
+      const int q  = ( j ? w - 1 : 0 ) * RG + r;
+      T         nv = su[q];
+      if ( vType & flag )
+      {
+         T acc = T( 0 );
+         for ( int k = 0; k < S; k++ )
+            acc += vpart[k][j][r];
+         nv = ( T( 1 ) - omega ) * nv + omega / vw[0] * ( b[(int64_t) v * NR + r0 + r] - acc );
+      }
+      su[q]                                          = nv;
+      u[( eo + ( j ? w - 1 : 0 ) ) * NR + r0 + r]    = nv;
+      if ( en[2 + j] ) u[(int64_t) v * NR + r0 + r] = nv;
+   }
+   if ( !( G.type & flag ) ) return; // uniform over the workgroup
+   const T* ew = EW + 3 * (int64_t) G.edge + G.termOff;
+   for ( int x = 1 + tid / RG; x <= w - 2; x += kMultiThreads / RG )
+      ts[x * RG + r] = edgeTermsSum< T, NR >( g, G, terms, ew + 3, u, x, r0 + r );
+   __syncthreads();
+   for ( int colour = 0; colour < 2; colour++ )
+   {
+      for ( int x = 2 - colour + 2 * ( tid / RG ); x <= w - 2; x += 2 * ( kMultiThreads / RG ) )
+      {
+         T acc = ew[0] * su[( x - 1 ) * RG + r] + ew[2] * su[( x + 1 ) * RG + r];
+         acc += ts[x * RG + r];
+         const int64_t o = ( eo + x ) * NR + r0 + r;
+         const T       nv = ( T( 1 ) - omega ) * su[x * RG + r] + omega / ew[1] * ( b[o] - acc );
+         su[x * RG + r]   = nv;
+         u[o]             = nv;
+      }
+      __syncthreads();
+   }
+}
+
+// one macro-face in LDS (levels <= kFaceFusedMaxLevel): V the whole face, its boundary straight from the edges, Q the
+// right-hand side less the off-plane terms, which read cell points that the phase does not change
+template < typename T, int NR, int RG >
+__global__ __launch_bounds__( 1024 ) void kFaceSorMulti( LV g, const FaceGeom* __restrict__ fg, const E2F* __restrict__ e2f,
+                                                        const T* __restrict__ FW, int flag, T* __restrict__ u,
+                                                        const T* __restrict__ b, T omega )
+{
+   constexpr int wMax = ( 1 << kFaceFusedMaxLevel ) + 1;
+   __shared__ T    V[wMax * ( wMax + 1 ) / 2 * RG], Q[kFaceFusedMaxNp * RG];
+   const FaceGeom& G  = fg[blockIdx.x / ( NR / RG )];
+   const int       rl = (int) threadIdx.x % RG, r = (int) ( blockIdx.x % ( NR / RG ) ) * RG + rl, w = g.w, m = w - 3;
+   const int       t = (int) threadIdx.x / RG, step = (int) blockDim.x / RG, np = m * ( m + 1 ) / 2, nV = w * ( w + 1 ) / 2;
+   const int64_t   fo     = g.offF + (int64_t) G.face * g.fS;
+   const bool      active = ( G.type & flag ) != 0;
+   const T*        fw     = FW + (int64_t) G.face * kFaceW;
+   for ( int p = t; p < 3 * w; p += step )
+   {
+      const E2F e = e2f[3 * G.face + p / w];
+      const int x = p % w, o = fidx( w, e.base[0] + x * e.inc[0], e.base[1] + x * e.inc[1] );
+      V[o * RG + rl] = u[( g.offE + (int64_t) e.edge * g.eS + x ) * NR + r];
+   }
+   for ( int k = t; k < np; k += step )
+   {
+      int i, j;
+      triPos( m, k, i, j );
+      const int     o  = fidx( w, ++i, ++j );
+      const int64_t oo = ( fo + o ) * NR + r;
+      V[o * RG + rl]   = u[oo];
+      if ( active ) Q[k * RG + rl] = b[oo] - faceOffPlaneAdd< T, NR >( g, G, fw, u, i, j, r, T( 0 ) );
+   }
+   __syncthreads();
+   if ( active )
+   {
+      const T relax = omega / fw[0];
+      for ( int colour = 0; colour < 3; colour++ )
+      {
+         for ( int k = t; k < np; k += step )
+         {
+            int i, j;
+            triPos( m, k, i, j );
+            i++, j++;
+            if ( ( i + 2 * j ) % 3 != colour ) continue;
+            // (i, j + 1) and (i, j - 1) are w - j and w - j + 1 places away
+            T*      Z   = V + fidx( w, i, j ) * RG + rl;
+            const T acc = fw[1] * Z[-RG] + fw[2] * Z[RG] + fw[3] * Z[( w - j ) * RG] + fw[4] * Z[-( w - j + 1 ) * RG] +
+                          fw[5] * Z[( w - j - 1 ) * RG] + fw[6] * Z[-( w - j ) * RG];
+            Z[0]        = ( T( 1 ) - omega ) * Z[0] + relax * ( Q[k * RG + rl] - acc );
+         }
+         __syncthreads();
+      }
+   }
+   for ( int o = t; o < nV; o += step )
+      u[( fo + o ) * NR + r] = V[o * RG + rl];
+}
+
+// one macro-cell in LDS (pts: its interior points by colour, as for kCellSorSmall), its boundary planes straight from
+// the faces.  A thread holds the place and right-hand side of its point of each colour (at most one) from the start.  The
+// groups of a cell's columns run on one XCD: they share the lines of its points.
+template < typename T, int NR, int RG >
+__global__ __launch_bounds__( 1024 ) void kCellSorMulti( LV g, const int* __restrict__ pts, ColourStarts cs, int nCells,
+                                                         const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
+                                                         T* __restrict__ u, const T* __restrict__ b, T omega,
+                                                         const F2C* __restrict__ f2c )
+{
+   constexpr int wMax = ( 1 << kCellMultiMaxLevel ) + 1, groups = NR / RG;
+   __shared__ T  V[wMax * ( wMax + 1 ) * ( wMax + 2 ) / 6 * RG];
+   const int     slot = (int) blockIdx.x >> 3, cell = slot / groups * 8 + ( (int) blockIdx.x & 7 );
+   if ( cell >= nCells ) return;
+   const int     rl = (int) threadIdx.x % RG, r = slot % groups * RG + rl, t = (int) threadIdx.x / RG;
+   const int     step = (int) blockDim.x / RG, w = g.w, t0 = tet32( w ), nF = w * ( w + 1 ) >> 1;
+   const int64_t base = g.offC + (int64_t) cell * g.cS;
+   T*            cu   = u + base * NR + r;
+   const T*      cb   = b + base * NR + r;
+   int           o[4], yz[4];
+   T             bv[4];
+#pragma unroll
+   for ( int cc = 0; cc < 4; cc++ )
+   {
+      const int  k  = cs.s[cc] + t;
+      const bool ok = k < cs.s[cc + 1];
+      const int  p = ok ? pts[k] : 0, x = p & 1023, y = ( p >> 10 ) & 1023, z = p >> 20;
+      o[cc]        = ok ? crow32( w, t0, y, z ) + x : -1;
+      yz[cc]       = y | z << 16;
+      bv[cc]       = ok ? cb[o[cc] * NR] : T( 0 );
+      if ( ok ) V[o[cc] * RG + rl] = cu[o[cc] * NR];
+   }
+   for ( int e = t; e < 4 * nF; e += step )
+   {
+      const F2C m = f2c[4 * cell + e / nF];
+      const int p = e % nF, j = triRow32( w, p ), i = p - j * ( 2 * w + 1 - j ) / 2;
+      const int x = m.m.base[0] + i * m.m.a[0] + j * m.m.b[0];
+      const int y = m.m.base[1] + i * m.m.a[1] + j * m.m.b[1];
+      const int z = m.m.base[2] + i * m.m.a[2] + j * m.m.b[2];
+      V[( crow32( w, t0, y, z ) + x ) * RG + rl] = u[( g.offF + (int64_t) m.face * g.fS + p ) * NR + r];
+   }
+   __syncthreads();
+   if ( ctype[cell] & flag ) // uniform over the workgroup
+   {
+      const T* c = W8 + (int64_t) cell * 15;
+      const T cW = c[dW], cE = c[dE], cN = c[dN], cS = c[dS], cNW = c[dNW], cSE = c[dSE];
+      const T cTC = c[dTC], cTW = c[dTW], cTS = c[dTS], cTSE = c[dTSE], cBC = c[dBC], cBN = c[dBN], cBE = c[dBE],
+              cBNW = c[dBNW];
+      const T relax = omega / c[dC];
+#pragma unroll
+      for ( int cc = 0; cc < 4; cc++ )
+      {
+         if ( o[cc] >= 0 )
+         {
+            // slab z has width W; its rows y, y + 1 and the slabs beside it (see kCellFlat)
+            const int y = yz[cc] & 0xffff, W = w - ( yz[cc] >> 16 );
+            T*        Z = V + o[cc] * RG + rl;
+            const int n = W - y, tc = W * ( W + 1 ) / 2 - y, bc = y - ( W + 1 ) * ( W + 2 ) / 2;
+#define U( i ) Z[( i ) * RG]
+            T acc = fma2( cW, U( -1 ), cE, U( 1 ) );
+            acc   = fma2( cN, U( n ), cNW, U( n - 1 ), acc );
+            acc   = fma2( cS, U( -n - 1 ), cSE, U( -n ), acc );
+            T up  = fma2( cTC, U( tc ), cTW, U( tc - 1 ) );
+            up    = fma2( cTS, U( tc - n ), cTSE, U( tc - n + 1 ), up );
+            T dn  = fma2( cBC, U( bc ), cBE, U( bc + 1 ) );
+            dn    = fma2( cBN, U( bc + n + 1 ), cBNW, U( bc + n ), dn );
+            acc   = acc + ( up + dn );
+            U( 0 ) = sorUpdate( omega, relax, U( 0 ), bv[cc], acc );
+#undef U
+         }
+         __syncthreads();
+      }
+   }
+   for ( int k = t; k < t0; k += step )
+      cu[k * NR] = V[k * RG + rl];
+}
+
+// --------------------------------------------------------------------------------------------------------
 // interpolation of a sum of Fourier modes at the micro-vertices (right-hand sides built on the device)
 
 template < typename T, int NR >
@@ -3607,6 +3818,29 @@ bool cellSorIsSmall( const LevelPlan& P )
    }
 }
 
+// The face-to-cell refresh and SOR cell phase of a forward sweep on several right-hand sides in one launch
+// (kCellSorMulti); false (nothing launched) above level 4: a level-5 cell leaves room for 16 bytes of columns per point
+// and one workgroup per CU, and took 79 us against 61 for the refresh and the four colour passes (48 cells, FP32).
+template < typename T, int NR >
+bool cellSorMulti( Mesh& M, LevelPlan& P, const T* CW, int flag, T* u, const T* b, T om )
+{
+   if ( P.L < 2 || P.L > kCellMultiMaxLevel || P.colourStart[4] == 0 ) return false;
+   ColourStarts cs;
+   int          most = 0;
+   for ( int k = 0; k < 5; k++ )
+   {
+      cs.s[k] = P.colourStart[k];
+      if ( k > 0 ) most = std::max( most, cs.s[k] - cs.s[k - 1] );
+   }
+   constexpr int RG      = 32 / (int) sizeof( T );
+   const int     threads = ( most * RG + 63 ) / 64 * 64;
+   if ( threads > 1024 ) throw std::logic_error( "cell SOR: more points of a colour than a workgroup has threads" );
+   hipLaunchKernelGGL( ( kCellSorMulti< T, NR, RG > ), dim3( ( M.T.nC() + 7 ) / 8 * 8 * ( NR / RG ) ), dim3( threads ), 0,
+                       M.ctx->stream, viewOf( P ), P.dColourPts.p, cs, M.T.nC(), CW, P.dCellType.p, flag, u, b, om,
+                       P.dF2C.p );
+   return true;
+}
+
 // withF2C: the one-workgroup-per-cell phase also does the face-to-cell refresh that precedes a forward cell
 // phase (the caller then skips it); ignored by the other forms of the phase.
 template < typename T, int NR >
@@ -3920,7 +4154,47 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
       return;
    }
    if ( backward && NR != 1 ) throw std::invalid_argument( "backward SOR needs one right-hand side" );
+   auto faceColours = [&]() {
+      const int64_t m = P.w - 3;
+      if ( m > 0 && nF > 0 )
+         for ( int c = 0; c < 3; c++ )
+            hipLaunchKernelGGL( ( kFaceSor< T, NR > ), dim3( blocksFor( ( m + 2 ) / 3 * NR, 256 ), m, nF ), dim3( 256 ), 0,
+                                s, g, P.dFaceGeom.p, wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om, c );
+   };
+   auto cellColours = [&]() {
+      for ( int c = 0; c < 4; c++ )
+         cellSorLaunch< T, NR >( M, P, wsel< T >( Wt.cell64, Wt.cell32 ), flag, u, b, om, c );
+   };
    // (closure copies are current: refreshed above when asked for, and every sweep ends with all of them current)
+   if constexpr ( NR > 1 )
+   {
+      // columns of a workgroup: 64 to 128 bytes of an edge point, 32 of a face point
+      constexpr int RE = 16, RF = 32 / (int) sizeof( T );
+      const size_t  edgeLds = 2 * (size_t) P.w * RE * sizeof( T );
+      if ( level >= 1 && edgeLds <= 60 * 1024 ) // beyond (level 8), the launches are long anyway
+      {
+         hipLaunchKernelGGL( ( kEdgeSorMulti< T, NR, RE > ), dim3( nE * ( NR / RE ) ), dim3( kMultiThreads ), edgeLds, s, g,
+                             P.dEdgeGeom.p, P.dEdgeTerms.p, wsel< T >( Wt.edge64, Wt.edge32 ), flag, u, b, om,
+                             P.dVertexSnap.p, P.dEdgeEnds.p, wsel< T >( Wt.vertex64, Wt.vertex32 ) );
+         if ( level >= 2 && level <= kFaceFusedMaxLevel && nF > 0 )
+         {
+            const int threads = std::min( 1024, std::max( 64, ( P.w - 3 ) * ( P.w - 2 ) / 2 * RF / 64 * 64 ) );
+            hipLaunchKernelGGL( ( kFaceSorMulti< T, NR, RF > ), dim3( nF * ( NR / RF ) ), dim3( threads ), 0, s, g,
+                                P.dFaceGeom.p, P.dE2F.p, wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om );
+         }
+         else
+         {
+            refreshT< T, NR >( xf, level, 2 );
+            if ( level >= 2 ) faceColours();
+         }
+         if ( !cellSorMulti< T, NR >( M, P, wsel< T >( Wt.cell64, Wt.cell32 ), flag, u, b, om ) )
+         {
+            refreshT< T, NR >( xf, level, 4 );
+            if ( level >= 2 ) cellColours();
+         }
+         return;
+      }
+   }
    hipLaunchKernelGGL( ( kVertexSor< T, NR > ), dim3( blocksFor( (int64_t) nV * NR, 256 ) ), dim3( 256 ), 0, s, g,
                        P.dVertexGeom.p, P.dVertexTerms.p, nV, wsel< T >( Wt.vertex64, Wt.vertex32 ), flag, u, b, om );
    refreshT< T, NR >( xf, level, 1 );
@@ -3931,14 +4205,9 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
    refreshT< T, NR >( xf, level, 2 );
    if ( level >= 2 )
    {
-      const int64_t m = P.w - 3;
-      if ( m > 0 && nF > 0 )
-         for ( int c = 0; c < 3; c++ )
-            hipLaunchKernelGGL( ( kFaceSor< T, NR > ), dim3( blocksFor( ( m + 2 ) / 3 * NR, 256 ), m, nF ), dim3( 256 ), 0,
-                                s, g, P.dFaceGeom.p, wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om, c );
+      faceColours();
       refreshT< T, NR >( xf, level, 4 );
-      for ( int c = 0; c < 4; c++ )
-         cellSorLaunch< T, NR >( M, P, wsel< T >( Wt.cell64, Wt.cell32 ), flag, u, b, om, c );
+      cellColours();
    }
 }
 
