@@ -1586,6 +1586,13 @@ __global__ __launch_bounds__( 1024 ) void kCellColumn( LV g, const MarchUnit* __
 // --------------------------------------------------------------------------------------------------------
 // macro-face interior
 
+// the in-plane neighbours' terms of a face point (weights 1 .. 6)
+template < typename T >
+__device__ __forceinline__ T faceInPlane( const T* __restrict__ fw, T vW, T vE, T vN, T vS, T vNW, T vSE )
+{
+   return fma2( fw[5], vNW, fw[6], vSE, fma2( fw[3], vN, fw[4], vS, fma2( fw[1], vW, fw[2], vE ) ) );
+}
+
 // acc plus the off-plane terms of face point (i, j) (the cells' points next to the face), in side order
 template < typename T, int NR >
 __device__ __forceinline__ T faceOffPlaneAdd( const LV& g, const FaceGeom& G, const T* __restrict__ fw,
@@ -1603,7 +1610,7 @@ __device__ __forceinline__ T faceOffPlaneAdd( const LV& g, const FaceGeom& G, co
          const int x   = M.base[0] + col * M.a[0] + row * M.b[0] + M.o[0];
          const int y   = M.base[1] + col * M.a[1] + row * M.b[1] + M.o[1];
          const int z   = M.base[2] + col * M.a[2] + row * M.b[2] + M.o[2];
-         acc += fw[7 + 4 * s + k] * u[( cb + cellRel( w, t0, x, y, z ) ) * NR + r];
+         acc         = fmaT( fw[7 + 4 * s + k], u[( cb + cellRel( w, t0, x, y, z ) ) * NR + r], acc );
       }
    }
    return acc;
@@ -2138,9 +2145,9 @@ __global__ __launch_bounds__( kEdgeThreads ) void kEdgeSorFused( LV g, const Edg
             const T* vw   = VW + v + vTermOff;
             T        part = T( 0 );
             for ( int k = lane; k < vN; k += 64 )
-               part += vw[1 + k] * u[vsnap[vTermOff + k]];
+               part = fmaT( vw[1 + k], u[vsnap[vTermOff + k]], part );
             const T acc = waveSum( part );
-            nv          = ( T( 1 ) - omega ) * old + omega / vw[0] * ( b[v] - acc );
+            nv          = sorUpdate( omega, omega / vw[0], old, b[v], acc );
          }
          if ( lane == 0 )
          {
@@ -2210,7 +2217,7 @@ __global__ __launch_bounds__( kEdgeThreads ) void kEdgeSorFused( LV g, const Edg
          }
 #pragma unroll
          for ( int q = 0; q < kEdgeTermBatch; q++ )
-            if ( k0 + q < ke ) acc += sW[k0 + q] * v[q];
+            if ( k0 + q < ke ) acc = fmaT( sW[k0 + q], v[q], acc );
       }
       if ( S == 1 )
          tsum[x] = acc;
@@ -2234,8 +2241,8 @@ __global__ __launch_bounds__( kEdgeThreads ) void kEdgeSorFused( LV g, const Edg
       const int colour = reverse ? 1 - cc : cc;
       for ( int x = 2 - colour + 2 * (int) threadIdx.x; x <= w - 2; x += 2 * blockDim.x )
       {
-         const T acc = tsum[x] + ( eW * su[x - 1] + eE * su[x + 1] );
-         const T nv  = ( T( 1 ) - omega ) * su[x] + rl * ( sb[x] - acc );
+         const T acc = tsum[x] + fma2( eW, su[x - 1], eE, su[x + 1] );
+         const T nv  = sorUpdate( omega, rl, su[x], sb[x], acc );
          su[x]       = nv;
          u[eo + x]   = nv;
       }
@@ -2285,16 +2292,272 @@ __global__ __launch_bounds__( 256 ) void kFaceSorFused( LV g, const FaceGeom* __
          const int bb = triRow32( m, k ), i = k - bb * ( 2 * m + 1 - bb ) / 2 + 1, j = bb + 1;
          if ( ( i + 2 * j ) % 3 != colour ) continue;
 #define UF( ii, jj ) u[fo + fidx( w, ii, jj )]
-         T acc = fw[1] * UF( i - 1, j ) + fw[2] * UF( i + 1, j );
-         acc += fw[3] * UF( i, j + 1 ) + fw[4] * UF( i, j - 1 );
-         acc += fw[5] * UF( i - 1, j + 1 ) + fw[6] * UF( i + 1, j - 1 );
+         const T acc = faceInPlane( fw, UF( i - 1, j ), UF( i + 1, j ), UF( i, j + 1 ), UF( i, j - 1 ), UF( i - 1, j + 1 ),
+                                    UF( i + 1, j - 1 ) ) +
+                       sOff[k];
 #undef UF
-         acc += sOff[k];
          const int64_t o = fo + fidx( w, i, j );
-         u[o]            = ( T( 1 ) - omega ) * u[o] + rl * ( b[o] - acc );
+         u[o]            = sorUpdate( omega, rl, u[o], b[o], acc );
       }
       __syncthreads();
    }
+}
+
+// --------------------------------------------------------------------------------------------------------
+// a forward SOR sweep of a small level in one launch (one right-hand side)
+
+// Workgroup = macro-cell.  The sweep goes from one array (uo) to another (un): everything a phase reads from outside the
+// cell's closure are values from before the sweep (other primitives' points, see the sweep's read rule), and uo keeps
+// them, so a workgroup can run all phases of its cell by itself: its vertices, edges and faces too, which the
+// neighbouring cells' workgroups compute to the same bits (same expressions from the same values), one of them writing
+// each.  Values of uo are read from the primitives that own them (own: element -> owner's element), so no closure copy
+// of uo needs to be current; those of un are when the sweep ends.  The terms of edge and face points from outside are
+// read through tables of owners (edgeNbr, faceNbr), all in flight together, before the phases run in LDS.
+// Three launches (vertices and edges, faces, cells), each a few microseconds of latency at these sizes, become one, and
+// the refresh before the first sweep goes.  The expressions are those of the launches it replaces, bit for bit.  Bound by
+// the latency of two dependent loads and some twelve barriers: 10 us at levels 1 to 3 and 15 us at level 4 (48
+// macro-tets, FP32) against 18 and 20 us for the three launches and their gaps; level-4 V(2,2) of 6 macro-tets 333 -> 240
+// us, level-6 FP32 solve 24.6 -> 21.7 ms, level-7 FP64 V(3,3) 3.45 -> 3.32 ms.  At level 5 a cell took 41 us against 30.
+template < typename T >
+struct SweepCellTables
+{
+   const CellLocal* cells;
+   const int32_t *  own, *edgeNbr, *faceNbr, *pts;
+   const int64_t*   vterms;
+   const T *        VW, *EW, *FW, *CW;
+};
+// v[k] by selects: a lane-dependent index into values that live in scalar registers
+template < int N >
+__device__ __forceinline__ int pick( const int32_t ( &v )[N], int k )
+{
+   int r = v[0];
+#pragma unroll
+   for ( int i = 1; i < N; i++ )
+      r = k == i ? v[i] : r;
+   return r;
+}
+constexpr int kSweepThreads = 1024;
+template < typename T, int LMAX >
+__global__ __launch_bounds__( kSweepThreads ) void kSweepCell( LV g, SweepCellTables< T > S, ColourStarts cs, int flag,
+                                                               const T* __restrict__ uo, T* __restrict__ un,
+                                                               const T* __restrict__ b, T omega )
+{
+   constexpr int wM = ( 1 << LMAX ) + 1, nPE = wM - 2, nPF = ( wM - 3 ) * ( wM - 2 ) / 2;
+   __shared__ T    V[wM * ( wM + 1 ) * ( wM + 2 ) / 6], sPart[6 * kEdgeThreads], eB[6 * nPE], eSum[6 * nPE],
+       fB[4 * nPF], fOff[4 * nPF], sVert[4], sEW[6][3], sFW[4][7];
+   __shared__ int32_t sMap[4][9];
+   constexpr int nt = kSweepThreads;
+   const int w = g.w, t0 = tet32( w ), tid = (int) threadIdx.x, cell = (int) blockIdx.x;
+   const int lane = tid & 63, np = w - 2, m = w - 3, nf = m * ( m + 1 ) / 2;
+   const CellLocal& C    = S.cells[cell];
+   const int64_t    co   = g.offC + (int64_t) cell * g.cS;
+   const bool       cellOn = nf > 0 && ( C.type & flag );
+   // place of point x of the cell's edge le (from the edge's first vertex), of face point (i, j) of local face lf
+   auto edgeAt = [&]( int ends, int x ) {
+      const int f = ends & 3, to = ends >> 2;
+      auto      at = [&]( int d ) { return f == d ? w - 1 - x : to == d ? x : 0; };
+      return cellRel( w, t0, at( 1 ), at( 2 ), at( 3 ) );
+   };
+   auto faceAt = [&]( int lf, int i, int j ) {
+      const int32_t* M = sMap[lf];
+      return cellRel( w, t0, M[0] + i * M[3] + j * M[6], M[1] + i * M[4] + j * M[7], M[2] + i * M[5] + j * M[8] );
+   };
+   // everything from memory first: the parts are given to different waves as far as they go round, so that their chains of
+   // dependent loads (table, then value) run side by side.  share( n ): this thread's first item of a part of n
+   int  given = 0;
+   auto share = [&]( int n ) {
+      const int k = tid - given;
+      given       = ( given + n + 63 ) / 64 * 64 % kSweepThreads;
+      return k < 0 ? k + kSweepThreads : k;
+   };
+   for ( int k = share( t0 ); k < t0; k += nt )
+      V[k] = uo[S.own[co + k]];
+   // the cell's points: at most one of each colour per thread, place, row geometry and right-hand side
+   int o[4], rowY[4], rowW[4];
+   T   bv[4];
+#pragma unroll
+   for ( int cc = 0; cc < 4; cc++ )
+   {
+      const int k = nf > 0 ? cs.s[cc] + share( cs.s[cc + 1] - cs.s[cc] ) : 0;
+      o[cc]       = -1;
+      if ( nf > 0 && k < cs.s[cc + 1] )
+      {
+         const int p = S.pts[k], y = ( p >> 10 ) & 1023, z = p >> 20;
+         rowY[cc]    = y;
+         rowW[cc]    = w - z;
+         o[cc]       = crow32( w, t0, y, z ) + ( p & 1023 );
+         bv[cc]      = b[co + o[cc]];
+      }
+   }
+   // vertices: one wave each, the terms as kVertexSorPush sums them
+   const int v = __builtin_amdgcn_readfirstlane( share( 4 * 64 ) >> 6 );
+   if ( v < 4 )
+   {
+      const T* vw   = S.VW + C.vert[v] + C.vTermOff[v];
+      T        part = T( 0 ), nv = uo[C.vert[v]];
+      if ( C.vType[v] & flag )
+      {
+         for ( int k = lane; k < C.vTerms[v]; k += 64 )
+            part = fmaT( vw[1 + k], uo[S.vterms[C.vTermOff[v] + k]], part );
+         nv = sorUpdate( omega, omega / vw[0], nv, b[C.vert[v]], waveSum( part ) );
+      }
+      if ( lane == 0 ) sVert[v] = nv;
+   }
+   // edges: sums of the terms from outside the edge in the slices of kEdgeSorFused
+   int slices = 1;
+   while ( slices < 8 && 2 * slices * np <= kEdgeThreads )
+      slices *= 2;
+   const int perEdge = np * slices;
+   for ( int k = share( 6 * perEdge ); k < 6 * perEdge; k += nt )
+   {
+      const int le = k / perEdge, q = k % perEdge, x = 1 + q % np, edge = pick( C.edge, le );
+      if ( !( pick( C.eType, le ) & flag ) ) continue;
+      const int      n = pick( C.eTerms, le ), off = pick( C.eTermOff, le );
+      const int      per = ( n + slices - 1 ) / slices, kb = q / np * per, ke = min( n, kb + per );
+      const T*       ew  = S.EW + 3 * edge + off + 3;
+      const int32_t* nbr = S.edgeNbr + off * np + ( x - 1 ) * n;
+      T              acc = T( 0 );
+      for ( int k0 = kb; k0 < ke; k0 += kTermBatch )
+      {
+         T v[kTermBatch], wt[kTermBatch];
+#pragma unroll
+         for ( int j = 0; j < kTermBatch; j++ )
+         {
+            v[j]  = uo[nbr[min( k0 + j, n - 1 )]];
+            wt[j] = ew[min( k0 + j, n - 1 )];
+         }
+#pragma unroll
+         for ( int j = 0; j < kTermBatch; j++ )
+            if ( k0 + j < ke ) acc = fmaT( wt[j], v[j], acc );
+      }
+      sPart[k] = acc;
+      if ( q < np ) eB[le * np + x - 1] = b[g.offE + edge * g.eS + x];
+      if ( q < 3 ) sEW[le][q] = ew[q - 3];
+   }
+   // faces: off-plane sums
+   for ( int k = share( 4 * nf ); k < 4 * nf; k += nt )
+   {
+      const int lf = k / nf, q = k % nf, face = pick( C.face, lf );
+      if ( !( pick( C.fType, lf ) & flag ) ) continue;
+      const T*       fw  = S.FW + face * kFaceW + 7;
+      const int32_t* nbr = S.faceNbr + ( face * nf + q ) * 8;
+      const int      nS  = 4 * pick( C.fSides, lf );
+      T              v[8], wt[8], acc = T( 0 );
+#pragma unroll
+      for ( int j = 0; j < 8; j++ )
+      {
+         v[j]  = uo[max( nbr[j], 0 )];
+         wt[j] = fw[j];
+      }
+#pragma unroll
+      for ( int j = 0; j < 8; j++ )
+         if ( j < nS ) acc = fmaT( wt[j], v[j], acc );
+      int i, j;
+      triPos( m, q, i, j );
+      fOff[k] = acc;
+      fB[k]   = b[g.offF + face * g.fS + fidx( w, i + 1, j + 1 )];
+   }
+   if ( tid < 36 ) sMap[tid / 9][tid % 9] = C.fMap[tid];
+   if ( nf > 0 && tid < 28 ) sFW[tid / 7][tid % 7] = S.FW[pick( C.face, tid / 7 ) * kFaceW + tid % 7];
+   T c[15];
+#pragma unroll
+   for ( int k = 0; k < 15; k++ )
+      c[k] = cellOn ? S.CW[(int64_t) cell * 15 + k] : T( 1 );
+   __syncthreads();
+   for ( int k = tid; k < 6 * np; k += nt )
+   {
+      const int le = k / np, x = k % np;
+      T         acc = sPart[le * perEdge + x];
+      for ( int sl = 1; sl < slices; sl++ )
+         acc += sPart[le * perEdge + sl * np + x];
+      eSum[k] = acc;
+   }
+   if ( tid < 4 ) V[cellRel( w, t0, tid == 1 ? w - 1 : 0, tid == 2 ? w - 1 : 0, tid == 3 ? w - 1 : 0 )] = sVert[tid];
+   __syncthreads();
+   for ( int colour = 0; colour < 2; colour++ )
+   {
+      for ( int k = tid; k < 6 * np; k += nt )
+      {
+         const int le = k / np, x = 1 + k % np, ends = pick( C.ends, le );
+         if ( ( x & 1 ) != colour || !( pick( C.eType, le ) & flag ) ) continue;
+         T&      Z   = V[edgeAt( ends, x )];
+         const T acc = eSum[k] + fma2( sEW[le][0], V[edgeAt( ends, x - 1 )], sEW[le][2], V[edgeAt( ends, x + 1 )] );
+         Z           = sorUpdate( omega, omega / sEW[le][1], Z, eB[k], acc );
+      }
+      __syncthreads();
+   }
+   if ( nf > 0 )
+      for ( int colour = 0; colour < 3; colour++ )
+      {
+         for ( int k = tid; k < 4 * nf; k += nt )
+         {
+            const int lf = k / nf;
+            int       i, j;
+            triPos( m, k % nf, i, j );
+            i++, j++;
+            if ( ( i + 2 * j ) % 3 != colour || !( pick( C.fType, lf ) & flag ) ) continue;
+            const T* fw  = sFW[lf];
+            auto     U   = [&]( int ii, int jj ) { return V[faceAt( lf, ii, jj )]; };
+            const T  acc = faceInPlane( fw, U( i - 1, j ), U( i + 1, j ), U( i, j + 1 ), U( i, j - 1 ), U( i - 1, j + 1 ),
+                                        U( i + 1, j - 1 ) ) +
+                          fOff[k];
+            T& Z = V[faceAt( lf, i, j )];
+            Z    = sorUpdate( omega, omega / fw[0], Z, fB[k], acc );
+         }
+         __syncthreads();
+      }
+   if ( cellOn )
+   {
+      const T cW = c[dW], cE = c[dE], cN = c[dN], cS = c[dS], cNW = c[dNW], cSE = c[dSE];
+      const T cTC = c[dTC], cTW = c[dTW], cTS = c[dTS], cTSE = c[dTSE], cBC = c[dBC], cBN = c[dBN], cBE = c[dBE],
+              cBNW = c[dBNW];
+      const T relax = omega / c[dC];
+#pragma unroll
+      for ( int cc = 0; cc < 4; cc++ )
+      {
+         if ( o[cc] >= 0 )
+         {
+            // offsets of rows y, y + 1 in the slab of width W and of the slabs beside it (see kCellFlat)
+            const int y = rowY[cc], W = rowW[cc], n = W - y, tc = W * ( W + 1 ) / 2 - y, bc = y - ( W + 1 ) * ( W + 2 ) / 2;
+            T*        Z = V + o[cc];
+            T         acc = fma2( cW, Z[-1], cE, Z[1] );
+            acc           = fma2( cN, Z[n], cNW, Z[n - 1], acc );
+            acc           = fma2( cS, Z[-n - 1], cSE, Z[-n], acc );
+            T up          = fma2( cTC, Z[tc], cTW, Z[tc - 1] );
+            up            = fma2( cTS, Z[tc - n], cTSE, Z[tc - n + 1], up );
+            T dn          = fma2( cBC, Z[bc], cBE, Z[bc + 1] );
+            dn            = fma2( cBN, Z[bc + n + 1], cBNW, Z[bc + n], dn );
+            acc           = acc + ( up + dn );
+            Z[0]          = sorUpdate( omega, relax, Z[0], bv[cc], acc );
+         }
+         __syncthreads();
+      }
+   }
+   // the cell with its closure; the faces, edges and vertices that this cell writes
+   for ( int k = tid; k < t0; k += nt )
+      un[co + k] = V[k];
+   const int nV = w * ( w + 1 ) / 2;
+   for ( int k = tid; k < 4 * nV; k += nt )
+   {
+      const int lf = k / nV, q = k % nV;
+      if ( !( C.write >> ( 10 + lf ) & 1 ) ) continue;
+      int i, j;
+      triPos( w, q, i, j );
+      un[g.offF + pick( C.face, lf ) * g.fS + q] = V[faceAt( lf, i, j )];
+   }
+   for ( int k = tid; k < 6 * w; k += nt )
+   {
+      const int le = k / w, x = k % w;
+      if ( C.write >> ( 4 + le ) & 1 ) un[g.offE + pick( C.edge, le ) * g.eS + x] = V[edgeAt( pick( C.ends, le ), x )];
+   }
+   if ( tid < 4 && ( C.write >> tid & 1 ) ) un[pick( C.vert, tid )] = sVert[tid];
+}
+
+template < typename T >
+__global__ __launch_bounds__( 256 ) void kCopyLevel( const T* __restrict__ src, T* __restrict__ dst, int n )
+{
+   const int k = (int) ( blockIdx.x * 256 + threadIdx.x );
+   if ( k < n ) dst[k] = src[k];
 }
 
 // --------------------------------------------------------------------------------------------------------
@@ -4006,6 +4269,46 @@ void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, in
 #undef LAUNCH_MODES
 }
 
+// Whether forward sweeps of the level run as one launch each (kSweepCell): its tables and scratch array exist (levels 1 to
+// kSweepCellMaxLevel, prepared with the solver) and the fused tile phase is not selected for T
+template < typename T >
+bool sweepCellOk( const LevelPlan& P )
+{
+   return P.sweepScratch && !( P.sorTile > 0 && ( P.sorPrecisions & ( std::is_same< T, double >::value ? 1 : 2 ) ) );
+}
+
+// `count` forward sweeps, each from one of x and the level's scratch array to the other; after an odd count, the scratch
+// array is copied back
+template < typename T >
+void sweepCells( Operator& op, Function& xf, const Function& bf, double omega, int level, int flag, int count )
+{
+   Mesh&       M  = *op.mesh;
+   LevelPlan&  P  = M.plan( level );
+   auto&       Wt = op.weights( level );
+   hipStream_t s  = M.ctx->stream;
+   T *         u = (T*) xf.ptr( level ), *other = reinterpret_cast< T* >( P.sweepScratch );
+   const SweepCellTables< T > S{ P.cellLocal, P.own, P.edgeNbr, P.faceNbr, P.dColourPts.p, P.dVertexTerms.p,
+                                 wsel< T >( Wt.vertex64, Wt.vertex32 ), wsel< T >( Wt.edge64, Wt.edge32 ),
+                                 wsel< T >( Wt.face64, Wt.face32 ), wsel< T >( Wt.cell64, Wt.cell32 ) };
+   ColourStarts cs;
+   for ( int k = 0; k < 5; k++ )
+      cs.s[k] = P.colourStart[k];
+   for ( int k = 0; k < count; k++ )
+   {
+      const T* src = k % 2 ? other : u;
+      T*       dst = k % 2 ? u : other;
+      if ( level <= 3 )
+         hipLaunchKernelGGL( ( kSweepCell< T, 3 > ), dim3( M.T.nC() ), dim3( kSweepThreads ), 0, s, viewOf( P ), S, cs, flag, src,
+                             dst, (const T*) bf.ptr( level ), (T) omega );
+      else
+         hipLaunchKernelGGL( ( kSweepCell< T, kSweepCellMaxLevel > ), dim3( M.T.nC() ), dim3( kSweepThreads ), 0, s, viewOf( P ),
+                             S, cs, flag, src, dst, (const T*) bf.ptr( level ), (T) omega );
+   }
+   if ( count % 2 )
+      hipLaunchKernelGGL( ( kCopyLevel< T > ), dim3( blocksFor( P.total, 256 ) ), dim3( 256 ), 0, s, (const T*) other, u,
+                          (int) P.total );
+}
+
 // One SOR sweep.  Forward (P1Operator.hpp:341-420): V -> E -> F -> C, each class reading the lower classes'
 // new values through closure copies refreshed in between and the higher classes' start-of-sweep values.
 // Backward (the same function with backwards = true): C -> F -> E -> V with the colours of every primitive
@@ -4032,6 +4335,8 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
    const T*    b  = (const T*) bf.ptr( level );
    const T     om = (T) omega;
    const int   nV = M.T.nV(), nE = M.T.nE(), nF = M.T.nF();
+   if constexpr ( NR == 1 )
+      if ( !backward && !pp && sweepCellOk< T >( P ) ) return sweepCells< T >( op, xf, bf, omega, level, flag, 1 );
    // a ping-pong pair reads no macro-cell closure point beyond distance 1 of the faces' edges before its final
    // face-to-cell copy
    if ( refreshFirst ) refreshT< T, NR >( xf, level, pp == 1 ? 1 | 2 | 8 : 7 );
@@ -4219,6 +4524,8 @@ void sorSweepsT( Operator& op, Function& xf, const Function& bf, double omega, i
 {
    Mesh&      M = *op.mesh;
    LevelPlan& P = M.plan( level );
+   if constexpr ( NR == 1 )
+      if ( count > 0 && sweepCellOk< T >( P ) ) return sweepCells< T >( op, xf, bf, omega, level, flag, count );
    if ( count >= 2 && pingPongOk< T, NR >( M, P, flag ) )
    {
       M.prepareCellSor( P );

@@ -146,6 +146,19 @@ struct CellFaceRead
    int32_t c[4][6];
 };
 
+// One macro-cell for the one-launch sweep of a small level: its edges (id, the cell-local vertices each runs between as
+// from | to << 2, term offset and count, type), vertices, faces (with their maps to the cell: base, a, b of F2C), its own
+// type, and which of its vertices (bits 0 .. 3), edges (4 .. 9) and faces (10 .. 13) it writes back (each primitive's
+// first cell does)
+struct CellLocal
+{
+   int32_t edge[6], ends[6], eTermOff[6], eTerms[6], eType[6];
+   int32_t vert[4], vTermOff[4], vTerms[4], vType[4];
+   int32_t face[4], fType[4], fSides[4], fMap[36];
+   int32_t type, write;
+};
+constexpr int kSweepCellMaxLevel = 4;
+
 // Operator weights aligned with the geometry tables.
 //   face: 15 per face: in-plane C, W, E, N, S, NW, SE (summed over sides), then side0 off[4], side1 off[4]
 //   edge: 3 (W, C, E) per edge followed by one weight per EdgeTerm

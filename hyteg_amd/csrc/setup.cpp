@@ -8,6 +8,7 @@
 // point (1,1) (P1Operator.hpp:2031-2042), edge weights at the edge point 1 (P1Elements.hpp:829-964) and
 // vertex weights from the single corner micro-tetrahedron of every neighbour cell (P1Elements.hpp:601-683).
 #include <algorithm>
+#include <cstring>
 #include <cmath>
 #include <stdexcept>
 
@@ -906,10 +907,105 @@ void Mesh::selectCellSor( int level, int tile, int precisions )
 
 bool Mesh::cellSorReady( const LevelPlan& P ) const { return P.sorTile == 0 || ctx->hostOnly || P.sorUnits != nullptr; }
 
+void Mesh::prepareSweepCell( LevelPlan& P )
+{
+   if ( P.L < 1 || P.L > kSweepCellMaxLevel || P.sweepScratch || ctx->hostOnly ) return;
+   const int              w = P.w, m = w - 3, nf = m * ( m + 1 ) / 2;
+   std::vector< int32_t > own( (size_t) P.total );
+   for ( int64_t k = 0; k < P.total; k++ )
+      own[k] = (int32_t) k;
+   for ( int e = 0; e < T.nE(); e++ )
+   {
+      own[P.edgeOff( e )]         = T.ev[e][0];
+      own[P.edgeOff( e ) + w - 1] = T.ev[e][1];
+   }
+   for ( int f = 0; f < T.nF(); f++ )
+      for ( int le = 0; le < 3; le++ )
+         for ( int x = 0; x < w; x++ )
+         {
+            int p[2];
+            faceEdgePoint( T, f, le, w, x, 0, p );
+            own[P.faceOff( f ) + faceIndex( w, p[0], p[1] )] = own[P.edgeOff( T.fe[f][le] ) + x];
+         }
+   auto cellAt = [&]( int c, const FaceCellMap& M, int i, int j, int layer ) {
+      return P.cellOff( c ) + cellIndex( w, M.base[0] + i * M.a[0] + j * M.b[0] + layer * M.o[0],
+                                         M.base[1] + i * M.a[1] + j * M.b[1] + layer * M.o[1],
+                                         M.base[2] + i * M.a[2] + j * M.b[2] + layer * M.o[2] );
+   };
+   std::vector< CellLocal > cells( T.nC() );
+   for ( int c = 0; c < T.nC(); c++ )
+   {
+      CellLocal& C = cells[c];
+      C.type       = T.cType[c];
+      for ( int lf = 0; lf < 4; lf++ )
+      {
+         const int         f = T.cf[c][lf];
+         const FaceCellMap M = numericMap( T, c, lf, w );
+         for ( int j = 0; j < w; j++ )
+            for ( int i = 0; i + j < w; i++ )
+               own[cellAt( c, M, i, j, 0 )] = own[P.faceOff( f ) + faceIndex( w, i, j )];
+         const VertexGeom& v = P.hVertexGeom[T.cv[c][lf]];
+         C.vert[lf]          = T.cv[c][lf];
+         C.vTermOff[lf] = v.termOff, C.vTerms[lf] = v.nTerms, C.vType[lf] = v.type;
+         C.face[lf] = f, C.fType[lf] = T.fType[f], C.fSides[lf] = P.hFaceGeom[f].nSides;
+         for ( int d = 0; d < 3; d++ )
+            C.fMap[9 * lf + d] = M.base[d], C.fMap[9 * lf + 3 + d] = M.a[d], C.fMap[9 * lf + 6 + d] = M.b[d];
+         C.write |= ( T.vCells[T.cv[c][lf]][0] == c ? 1 : 0 ) << lf | ( T.fCells[f][0] == c ? 1 : 0 ) << ( 10 + lf );
+      }
+      for ( int le = 0; le < 6; le++ )
+      {
+         const EdgeGeom& e = P.hEdgeGeom[T.ce[c][le]];
+         C.edge[le]        = T.ce[c][le];
+         C.eTermOff[le] = e.termOff, C.eTerms[le] = e.nTerms, C.eType[le] = e.type;
+         C.ends[le] = T.cemap[c][2 * le] | T.cemap[c][2 * le + 1] << 2;
+         C.write |= ( T.eCells[T.ce[c][le]][0] == c ? 1 : 0 ) << ( 4 + le );
+      }
+   }
+   std::vector< int32_t > edgeNbr, faceNbr;
+   edgeNbr.reserve( P.hEdgeTerms.size() * (size_t) ( w - 2 ) );
+   for ( const EdgeGeom& G : P.hEdgeGeom )
+      for ( int x = 1; x <= w - 2; x++ )
+         for ( int k = 0; k < G.nTerms; k++ )
+         {
+            const EdgeTerm& t = P.hEdgeTerms[G.termOff + k];
+            const int       q[3] = { t.base[0] + x * t.inc[0], t.base[1] + x * t.inc[1], t.base[2] + x * t.inc[2] };
+            edgeNbr.push_back( own[t.kind == 0 ? P.faceOff( t.prim ) + faceIndex( w, q[0], q[1] )
+                                               : P.cellOff( t.prim ) + cellIndex( w, q[0], q[1], q[2] )] );
+         }
+   faceNbr.reserve( (size_t) T.nF() * nf * 8 );
+   for ( const FaceGeom& G : P.hFaceGeom )
+      for ( int j = 1; j <= m; j++ )
+         for ( int i = 1; i + j <= w - 2; i++ )
+            for ( int sd = 0; sd < 2; sd++ )
+               for ( int k = 0; k < 4; k++ )
+                  faceNbr.push_back( sd < G.nSides ? own[cellAt( G.side[sd].cell, G.side[sd], i + G.offCol[sd][k],
+                                                                 j + G.offRow[sd][k], 1 )]
+                                                   : -1 );
+   // one allocation and one copy: the scratch array (cleared: its padding is copied with it), then the tables
+   const size_t           nScratch = 2 * (size_t) P.total, nCells = cells.size() * ( sizeof( CellLocal ) / 4 );
+   std::vector< int32_t > all( nCells );
+   std::memcpy( all.data(), cells.data(), 4 * nCells );
+   for ( const auto* t : { &own, &edgeNbr, &faceNbr } )
+      all.insert( all.end(), t->begin(), t->end() );
+   P.sweepTables.alloc( nScratch + all.size() );
+   {
+      HYMI_LEGACY_LOCK;
+      HYMI_HIP( hipMemsetAsync( P.sweepTables.p, 0, 4 * nScratch, ctx->stream ) );
+      HYMI_HIP( hipMemcpyAsync( P.sweepTables.p + nScratch, all.data(), 4 * all.size(), hipMemcpyHostToDevice, ctx->stream ) );
+   }
+   HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
+   P.cellLocal    = reinterpret_cast< const CellLocal* >( P.sweepTables.p + nScratch );
+   P.own          = P.sweepTables.p + nScratch + nCells;
+   P.edgeNbr      = P.own + own.size();
+   P.faceNbr      = P.edgeNbr + edgeNbr.size();
+   P.sweepScratch = reinterpret_cast< double* >( P.sweepTables.p );
+}
+
 // Work units and scratch arrays of the fused SOR cell phase selected on P (nothing if the passes are selected or
 // they exist already).  Called outside graph capture: by the entry points that sweep and by solver creation.
 void Mesh::prepareCellSor( LevelPlan& P )
 {
+   prepareSweepCell( P );
    if ( P.sorTile == 0 || P.sorUnits ) return;
    const int tile = P.sorTile;
    std::vector< MarchUnit > v;
