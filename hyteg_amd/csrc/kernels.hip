@@ -991,10 +991,13 @@ __global__ __launch_bounds__( 256 ) void kCellTile( LV g, const MarchUnit* __res
    if ( z < zb ) step( z, stB, stA );
 }
 
-// The whole SOR cell phase of a small level in one launch: one workgroup per macro-cell runs the four colours
-// in order, with a barrier between colours (cells do not couple within the phase: their boundary values are
-// closure copies that no kernel of the phase writes).  pts lists the cell's interior points by colour; every
-// point is computed with the expression of the march kernels, so the result equals four colour passes.
+// The whole SOR cell phase of a small level in one launch: one workgroup per macro-cell holds the cell in LDS (52 KB at
+// level 5 in FP64) and runs the four colours in order, with a barrier between colours (cells do not couple within the
+// phase: their boundary values are closure copies that no kernel of the phase writes).  pts lists the cell's interior
+// points by colour; a thread has the places and right-hand sides of its points of every colour (two at most) in registers
+// before the first.  Every point is computed with the expression of the march kernels, so the result equals four colour
+// passes.  With the colours reading global memory, and points of a colour in every fourth word of LDS, four symmetric
+// sweeps of level 5 (36 macro-tets, FP64) took 151 and 145 us, now 141 (the faces' LDS form included).
 struct ColourStarts
 {
    int s[5];
@@ -1002,62 +1005,95 @@ struct ColourStarts
 // With F2C = true (forward sweeps) the workgroup first copies its four faces' closures into the cell's closure
 // (the face-to-cell refresh of the sweep, as kF2C does it for this cell): the faces are final once the face
 // phase is done, and the cell's copies are read by no other workgroup.  Cells the flag leaves alone copy too.
+constexpr int kCellSmallWidth = ( 1 << kCellSmallMaxLevel ) + 1, kCellSmallIter = 2;
 template < typename T, bool F2C_ >
 __global__ __launch_bounds__( 1024 ) void kCellSorSmall( LV g, const int* __restrict__ pts, ColourStarts cs,
                                                         const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
                                                         T* __restrict__ u, const T* __restrict__ b, T omega, int reverse,
                                                         const F2C* __restrict__ f2c )
 {
-   const int     cell = blockIdx.x;
+   constexpr int wM = kCellSmallWidth;
+   constexpr int Q = ( wM * ( wM + 1 ) * ( wM + 2 ) / 6 + 3 ) / 4;
+   __shared__ T  V[4 * Q];
+   // point i of the cell lies at at( i ): the points of a colour are 4 apart in a row, so the four residues of i are kept
+   // apart and the lanes of a wave read consecutive words (with V[i] only every fourth bank pair is used)
+   auto          at = [&]( int i ) -> T& { return V[( i & 3 ) * Q + ( i >> 2 )]; };
+   const int     cell = blockIdx.x, tid = (int) threadIdx.x, nt = (int) blockDim.x;
    const int     w = g.w, t0 = tet32( w );
    const int64_t base = g.offC + (int64_t) cell * g.cS;
+   T*            cu   = u + base;
+   const T*      cb   = b + base;
+   const bool    on   = ( ctype[cell] & flag ) != 0; // uniform over the workgroup
+   if ( !F2C_ && !on ) return;
+   // the colours in the order of the sweep (a backward one takes them in reverse): places (-1: none), row and slab width,
+   // right-hand sides
+   int o[4][kCellSmallIter], rw[4][kCellSmallIter];
+   T   bv[4][kCellSmallIter];
+#pragma unroll
+   for ( int cc = 0; cc < 4; cc++ )
+#pragma unroll
+      for ( int it = 0; it < kCellSmallIter; it++ )
+      {
+         const int colour = reverse ? 3 - cc : cc, k = cs.s[colour] + tid + it * nt;
+         o[cc][it]        = -1;
+         if ( k < cs.s[colour + 1] )
+         {
+            const int p = pts[k], y = ( p >> 10 ) & 1023, z = p >> 20;
+            o[cc][it]  = crow32( w, t0, y, z ) + ( p & 1023 );
+            rw[cc][it] = y | ( w - z ) << 16;
+            bv[cc][it] = cb[o[cc][it]];
+            if ( F2C_ ) at( o[cc][it] ) = cu[o[cc][it]];
+         }
+      }
    if constexpr ( F2C_ )
    {
       const int nF = w * ( w + 1 ) >> 1;
-      for ( int e = (int) threadIdx.x; e < 4 * nF; e += blockDim.x )
+      for ( int e = tid; e < 4 * nF; e += nt )
       {
          const F2C m = f2c[4 * cell + e / nF];
          const int p = e % nF, j = triRow32( w, p ), i = p - j * ( 2 * w + 1 - j ) / 2;
          const int x = m.m.base[0] + i * m.m.a[0] + j * m.m.b[0];
          const int y = m.m.base[1] + i * m.m.a[1] + j * m.m.b[1];
          const int z = m.m.base[2] + i * m.m.a[2] + j * m.m.b[2];
-         u[base + crow32( w, t0, y, z ) + x] = u[g.offF + (int64_t) m.face * g.fS + p];
+         at( crow32( w, t0, y, z ) + x ) = u[g.offF + (int64_t) m.face * g.fS + p];
       }
-      __syncthreads();
    }
-   if ( !( ctype[cell] & flag ) ) return; // uniform over the workgroup
-   T*            cu   = u + base;
-   const T*      cb   = b + base;
-   const T*      c    = W8 + (int64_t) cell * 15;
+   else
+      for ( int k = tid; k < t0; k += nt )
+         at( k ) = cu[k];
+   const T* c = W8 + (int64_t) cell * 15;
    const T cE = c[dE], cW = c[dW], cN = c[dN], cS = c[dS], cNW = c[dNW], cSE = c[dSE];
    const T cTC = c[dTC], cTW = c[dTW], cTS = c[dTS], cTSE = c[dTSE], cBC = c[dBC], cBN = c[dBN], cBE = c[dBE],
            cBNW = c[dBNW];
    const T relax = omega / c[dC];
+   __syncthreads();
+#pragma unroll
    for ( int cc = 0; cc < 4; cc++ )
    {
-      const int colour = reverse ? 3 - cc : cc; // a backward sweep takes the colours in reverse
-      for ( int k = cs.s[colour] + (int) threadIdx.x; k < cs.s[colour + 1]; k += blockDim.x )
-      {
-         const int p = pts[k], x = p & 1023, y = ( p >> 10 ) & 1023, z = p >> 20;
-         const int r0 = crow32( w, t0, y, z ) + x, rN = crow32( w, t0, y + 1, z ) + x, rS = crow32( w, t0, y - 1, z ) + x;
-         const int rT = crow32( w, t0, y, z + 1 ) + x, rTS = crow32( w, t0, y - 1, z + 1 ) + x;
-         const int rB = crow32( w, t0, y, z - 1 ) + x, rBN = crow32( w, t0, y + 1, z - 1 ) + x;
-         const T   Z0 = cu[r0], Z0l = cu[r0 - 1], Z0r = cu[r0 + 1], Zp = cu[rN], Zpl = cu[rN - 1], Zm = cu[rS],
-                 Zmr = cu[rS + 1];
-         const T T0 = cu[rT], T0l = cu[rT - 1], Tm = cu[rTS], Tmr = cu[rTS + 1];
-         const T B0 = cu[rB], B0r = cu[rB + 1], Bp = cu[rBN], Bpl = cu[rBN - 1];
-         T       acc = fma2( cW, Z0l, cE, Z0r );
-         acc   = fma2( cN, Zp, cNW, Zpl, acc );
-         acc   = fma2( cS, Zm, cSE, Zmr, acc );
-         T up  = fma2( cTC, T0, cTW, T0l );
-         up    = fma2( cTS, Tm, cTSE, Tmr, up );
-         T dn  = fma2( cBC, B0, cBE, B0r );
-         dn    = fma2( cBN, Bp, cBNW, Bpl, dn );
-         acc   = acc + ( up + dn );
-         cu[r0] = sorUpdate( omega, relax, Z0, cb[r0], acc );
-      }
+#pragma unroll
+      for ( int it = 0; it < kCellSmallIter; it++ )
+         if ( on && o[cc][it] >= 0 )
+         {
+            // offsets of rows y, y + 1 in the slab of width W and of the slabs beside it (see kCellFlat)
+            const int y = rw[cc][it] & 0xffff, W = rw[cc][it] >> 16, n = W - y, tc = W * ( W + 1 ) / 2 - y,
+                      bc = y - ( W + 1 ) * ( W + 2 ) / 2;
+            const int q = o[cc][it];
+#define Z( d ) at( q + ( d ) )
+            T acc = fma2( cW, Z( -1 ), cE, Z( 1 ) );
+            acc   = fma2( cN, Z( n ), cNW, Z( n - 1 ), acc );
+            acc   = fma2( cS, Z( -n - 1 ), cSE, Z( -n ), acc );
+            T up  = fma2( cTC, Z( tc ), cTW, Z( tc - 1 ) );
+            up    = fma2( cTS, Z( tc - n ), cTSE, Z( tc - n + 1 ), up );
+            T dn  = fma2( cBC, Z( bc ), cBE, Z( bc + 1 ) );
+            dn    = fma2( cBN, Z( bc + n + 1 ), cBNW, Z( bc + n ), dn );
+            acc   = acc + ( up + dn );
+            Z( 0 ) = sorUpdate( omega, relax, Z( 0 ), bv[cc][it], acc );
+#undef Z
+         }
       __syncthreads(); // the next colour reads this colour's values
    }
+   for ( int k = tid; k < t0; k += nt )
+      cu[k] = at( k );
 }
 
 // The whole SOR cell phase of a level in one launch, for levels above the one-workgroup-per-cell phase.
@@ -2250,56 +2286,70 @@ __global__ __launch_bounds__( kEdgeThreads ) void kEdgeSorFused( LV g, const Edg
    }
 }
 
+// The face lives in LDS: its boundary from the final edge values, its interior, the right-hand side and the sums of the
+// off-plane terms, which read cell points that the phase does not change, all loaded together.  Every face copies its
+// edges, also one whose own points the flag leaves alone.  With the boundary copied in memory first and the colours
+// reading it from there, 36 macro-tets took 9.5 us at level 5 in FP64, now 7.4.
+constexpr int kFaceFusedThreads = 512;
 template < typename T >
-__global__ __launch_bounds__( 256 ) void kFaceSorFused( LV g, const FaceGeom* __restrict__ fg, const E2F* __restrict__ e2f,
-                                                        const T* __restrict__ FW, int flag, T* __restrict__ u,
-                                                        const T* __restrict__ b, T omega, int reverse )
+__global__ __launch_bounds__( kFaceFusedThreads ) void kFaceSorFused( LV g, const FaceGeom* __restrict__ fg,
+                                                                      const E2F* __restrict__ e2f,
+                                                                      const T* __restrict__ FW, int flag,
+                                                                      T* __restrict__ u, const T* __restrict__ b, T omega,
+                                                                      int reverse )
 {
+   constexpr int   wM = ( 1 << kFaceFusedMaxLevel ) + 1;
+   __shared__ T    V[wM * ( wM + 1 ) / 2], sOff[kFaceFusedMaxNp], sB[kFaceFusedMaxNp];
    const FaceGeom& G  = fg[blockIdx.x];
+   const int       w = g.w, m = w - 3, np = m * ( m + 1 ) / 2, nV = w * ( w + 1 ) / 2; // np <= kFaceFusedMaxNp
+   const int       tid = (int) threadIdx.x, nt = (int) blockDim.x;
    const int64_t   fo = g.offF + (int64_t) G.face * g.fS;
-   // own boundary <- final edge values (the E2F table holds the three edges of face f at 3f .. 3f+2); the
-   // three edges' values are loaded before any is stored, so their loads are in flight together.  Every face
-   // copies, also one whose own points the flag leaves alone: its edges may have been updated.
-   E2F m3[3];
-   for ( int le = 0; le < 3; le++ )
-      m3[le] = e2f[3 * G.face + le];
-   for ( int p = threadIdx.x; p < g.w; p += blockDim.x )
+   const bool      on = ( G.type & flag ) != 0; // uniform over the workgroup
+   const T*        fw = FW + (int64_t) G.face * kFaceW;
+   // the last waves take the edges (the E2F table holds the three edges of face f at 3f .. 3f+2), the first the interior
+   for ( int k = nt - 1 - tid; k < 3 * w; k += nt )
    {
-      T ev[3];
-      for ( int le = 0; le < 3; le++ )
-         ev[le] = u[g.offE + (int64_t) m3[le].edge * g.eS + p];
-      for ( int le = 0; le < 3; le++ )
-         u[fo + fidx( g.w, m3[le].base[0] + p * m3[le].inc[0], m3[le].base[1] + p * m3[le].inc[1] )] = ev[le];
+      const E2F e = e2f[3 * G.face + k / w];
+      const int x = k % w;
+      V[fidx( w, e.base[0] + x * e.inc[0], e.base[1] + x * e.inc[1] )] = u[g.offE + (int64_t) e.edge * g.eS + x];
    }
-   if ( !( G.type & flag ) ) return; // uniform over the workgroup: no barrier is skipped by part of it
-   // The off-plane terms read cell points, which the face phase does not change: their sums are formed once
-   // for all points (LDS), next to the edge copies above, and each colour pass adds only the in-plane terms.
-   __shared__ T  sOff[kFaceFusedMaxNp];
-   const int     w  = g.w, m = w - 3, np = m * ( m + 1 ) / 2; // np <= kFaceFusedMaxNp (levels <= kFaceFusedMaxLevel)
-   const T*      fw = FW + (int64_t) G.face * kFaceW;
-   const T       rl = omega / fw[0];
-   for ( int k = threadIdx.x; k < np; k += blockDim.x )
-   {
-      const int bb = triRow32( m, k ), i = k - bb * ( 2 * m + 1 - bb ) / 2 + 1, j = bb + 1;
-      sOff[k]      = faceOffPlaneAdd< T, 1 >( g, G, fw, u, i, j, 0, T( 0 ) );
-   }
-   __syncthreads();
-   for ( int cc = 0; cc < 3; cc++ )
-   {
-      const int colour = reverse ? 2 - cc : cc; // a backward sweep takes the colours in reverse
-      for ( int k = threadIdx.x; k < np; k += blockDim.x )
+   if ( on )
+      for ( int k = tid; k < np; k += nt )
       {
-         const int bb = triRow32( m, k ), i = k - bb * ( 2 * m + 1 - bb ) / 2 + 1, j = bb + 1;
-         if ( ( i + 2 * j ) % 3 != colour ) continue;
-#define UF( ii, jj ) u[fo + fidx( w, ii, jj )]
-         const T acc = faceInPlane( fw, UF( i - 1, j ), UF( i + 1, j ), UF( i, j + 1 ), UF( i, j - 1 ), UF( i - 1, j + 1 ),
-                                    UF( i + 1, j - 1 ) ) +
-                       sOff[k];
-#undef UF
-         const int64_t o = fo + fidx( w, i, j );
-         u[o]            = sorUpdate( omega, rl, u[o], b[o], acc );
+         int i, j;
+         triPos( m, k, i, j );
+         const int o = fidx( w, ++i, ++j );
+         V[o]        = u[fo + o];
+         sB[k]       = b[fo + o];
+         sOff[k]     = faceOffPlaneAdd< T, 1 >( g, G, fw, u, i, j, 0, T( 0 ) );
       }
-      __syncthreads();
+   __syncthreads();
+   if ( on )
+   {
+      const T rl = omega / fw[0];
+      for ( int cc = 0; cc < 3; cc++ )
+      {
+         const int colour = reverse ? 2 - cc : cc; // a backward sweep takes the colours in reverse
+         for ( int k = tid; k < np; k += nt )
+         {
+            int i, j;
+            triPos( m, k, i, j );
+            i++, j++;
+            if ( ( i + 2 * j ) % 3 != colour ) continue;
+            // (i, j + 1) and (i, j - 1) are w - j and w - j + 1 places away
+            T*      Z   = V + fidx( w, i, j );
+            const T acc = faceInPlane( fw, Z[-1], Z[1], Z[w - j], Z[-( w - j + 1 )], Z[w - j - 1], Z[-( w - j )] ) + sOff[k];
+            Z[0]        = sorUpdate( omega, rl, Z[0], sB[k], acc );
+         }
+         __syncthreads();
+      }
+   }
+   // all of it, or (a face left alone) its boundary
+   for ( int k = tid; k < nV; k += nt )
+   {
+      int i, j;
+      triPos( w, k, i, j );
+      if ( on || i == 0 || j == 0 || i + j == w - 1 ) u[fo + k] = V[k];
    }
 }
 
@@ -4125,6 +4175,9 @@ void cellSorPhase( Mesh& M, LevelPlan& P, const T* CW, int flag, T* u, const T* 
       // threads: about one point of a colour each, from 64 (level 2) up to 1024 (level 5: 1124 per colour)
       const int perColour = ( P.colourStart[4] + 3 ) / 4;
       const int threads   = std::min( 1024, std::max( 64, ( perColour + 63 ) / 64 * 64 ) );
+      for ( int k = 0; k < 4; k++ )
+         if ( cs.s[k + 1] - cs.s[k] > kCellSmallIter * threads )
+            throw std::logic_error( "cell SOR: more points of a colour than its threads take" );
       if ( withF2C )
          hipLaunchKernelGGL( ( kCellSorSmall< T, true > ), dim3( M.T.nC() ), dim3( threads ), 0, M.ctx->stream, viewOf( P ),
                              P.dColourPts.p, cs, CW, P.dCellType.p, flag, u, b, om, rev, P.dF2C.p );
@@ -4368,7 +4421,7 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
       auto facePhase = [&]() {
          if ( nF == 0 ) return;
          if ( level <= kFaceFusedMaxLevel )
-            hipLaunchKernelGGL( ( kFaceSorFused< T > ), dim3( nF ), dim3( 256 ), 0, s, g, P.dFaceGeom.p, P.dE2F.p,
+            hipLaunchKernelGGL( ( kFaceSorFused< T > ), dim3( nF ), dim3( kFaceFusedThreads ), 0, s, g, P.dFaceGeom.p, P.dE2F.p,
                                 wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om, rev );
          else
          {
