@@ -1200,6 +1200,7 @@ static int makeOperator( hymi_mesh mesh, int minL, int maxL, int form, hymi_oper
       {
          h->op.lw.push_back( std::make_unique< Operator::LevelWeights >() );
          buildOperatorWeights( h->op, L );
+         mesh->m.prepareSweepCell( mesh->m.plan( L ) );
       }
       *out = h.release();
    } );

@@ -1658,10 +1658,9 @@ __device__ __forceinline__ T faceStencilSum( const LV& g, const FaceGeom& G, con
 {
    const int w = g.w;
 #define UF( ii, jj ) u[( fo + fidx( w, ii, jj ) ) * NR + r]
-   T acc = fw[1] * UF( i - 1, j ) + fw[2] * UF( i + 1, j );
-   acc += fw[3] * UF( i, j + 1 ) + fw[4] * UF( i, j - 1 );
-   acc += fw[5] * UF( i - 1, j + 1 ) + fw[6] * UF( i + 1, j - 1 );
-   if ( withCentre ) acc += fw[0] * UF( i, j );
+   T acc = faceInPlane( fw, UF( i - 1, j ), UF( i + 1, j ), UF( i, j + 1 ), UF( i, j - 1 ), UF( i - 1, j + 1 ),
+                        UF( i + 1, j - 1 ) );
+   if ( withCentre ) acc = fmaT( fw[0], UF( i, j ), acc );
 #undef UF
    return faceOffPlaneAdd< T, NR >( g, G, fw, u, i, j, r, acc );
 }
@@ -1923,7 +1922,7 @@ __device__ __forceinline__ T edgeTermsSum( const LV& g, const EdgeGeom& G, const
       }
 #pragma unroll
       for ( int q = 0; q < kTermBatch; q++ )
-         if ( k0 + q < n ) acc += wt[q] * v[q];
+         if ( k0 + q < n ) acc = fmaT( wt[q], v[q], acc );
    }
    return acc;
 }
@@ -1941,7 +1940,8 @@ __device__ __forceinline__ void kEdgeApply_b( const Blk& B, LV g, const EdgeGeom
    if ( x > g.w - 2 ) return;
    const T*      ew  = EW + 3 * (int64_t) G.edge + G.termOff;
    const int64_t eo  = g.offE + (int64_t) G.edge * g.eS;
-   T             acc = ew[0] * u[( eo + x - 1 ) * NR + r] + ew[1] * u[( eo + x ) * NR + r] + ew[2] * u[( eo + x + 1 ) * NR + r];
+   T             acc = fmaT( ew[1], u[( eo + x ) * NR + r],
+                             fma2( ew[0], u[( eo + x - 1 ) * NR + r], ew[2], u[( eo + x + 1 ) * NR + r] ) );
    acc += edgeTermsSum< T, NR >( g, G, terms, ew + 3, u, x, r );
    const int64_t o = ( eo + x ) * NR + r;
    if ( MODE == kReplace )
@@ -2000,7 +2000,7 @@ __device__ __forceinline__ void kVertexApply_b( const Blk& B, LV g, const Vertex
       }
 #pragma unroll
       for ( int q = 0; q < kTermBatch; q++ )
-         if ( k0 + q < G.nTerms ) acc += wt[q] * v[q];
+         if ( k0 + q < G.nTerms ) acc = fmaT( wt[q], v[q], acc );
    }
    const int64_t o = (int64_t) G.vertex * NR + r;
    if ( MODE == kReplace )
@@ -2601,6 +2601,118 @@ __global__ __launch_bounds__( kSweepThreads ) void kSweepCell( LV g, SweepCellTa
       if ( C.write >> ( 4 + le ) & 1 ) un[g.offE + pick( C.edge, le ) * g.eS + x] = V[edgeAt( pick( C.ends, le ), x )];
    }
    if ( tid < 4 && ( C.write >> tid & 1 ) ) un[pick( C.vert, tid )] = sVert[tid];
+}
+
+// Apply or residual of a small level in one launch, without a refresh of src's closure copies: a workgroup per
+// macro-cell reads the cell's closure from the owners into LDS and computes the cell's interior and the faces, edges and
+// vertices that it writes (CellLocal), their outside terms through the owner tables of kSweepCell.  Launch latency bounds
+// it: refresh and apply took 8.9 us at level 3 (6 macro-tets, FP64), this 4.3.
+constexpr int kApplyCellThreads = 512;
+template < typename T, int LMAX, int MODE >
+__global__ __launch_bounds__( kApplyCellThreads ) void kApplyCell( LV g, SweepCellTables< T > S, ColourStarts cs, int flag,
+                                                                   const T* __restrict__ u, T* __restrict__ y,
+                                                                   const T* __restrict__ b )
+{
+   constexpr int wM = ( 1 << LMAX ) + 1, nt = kApplyCellThreads;
+   __shared__ T       V[wM * ( wM + 1 ) * ( wM + 2 ) / 6];
+   const int          w = g.w, t0 = tet32( w ), tid = (int) threadIdx.x, cell = (int) blockIdx.x;
+   const int          lane = tid & 63, np = w - 2, m = w - 3, nf = m * ( m + 1 ) / 2, ni = nf > 0 ? cs.s[4] : 0;
+   const CellLocal&   C  = S.cells[cell];
+   const int64_t      co = g.offC + (int64_t) cell * g.cS;
+   auto put = [&]( int64_t o, T acc ) { y[o] = MODE == kReplace ? acc : MODE == kAdd ? y[o] + acc : b[o] - acc; };
+   for ( int k = tid; k < t0; k += nt )
+      V[k] = u[S.own[co + k]];
+   __syncthreads();
+   if ( C.type & flag )
+   {
+      const T* c = S.CW + (int64_t) cell * 15;
+      const T cC = c[dC], cW = c[dW], cE = c[dE], cN = c[dN], cS = c[dS], cNW = c[dNW], cSE = c[dSE];
+      const T cTC = c[dTC], cTW = c[dTW], cTS = c[dTS], cTSE = c[dTSE], cBC = c[dBC], cBN = c[dBN], cBE = c[dBE],
+              cBNW = c[dBNW];
+      for ( int k = tid; k < ni; k += nt )
+      {
+         const int p = S.pts[k], yy = ( p >> 10 ) & 1023, z = p >> 20, r0 = crow32( w, t0, yy, z ) + ( p & 1023 );
+         // offsets of rows y, y + 1 in the slab of width W and of the slabs beside it (see kCellFlat)
+         const int W = w - z, n = W - yy, tc = W * ( W + 1 ) / 2 - yy, bc = yy - ( W + 1 ) * ( W + 2 ) / 2;
+         const T*  Z   = V + r0;
+         T         acc = cC * Z[0];
+         acc           = fma2( cW, Z[-1], cE, Z[1], acc );
+         acc           = fma2( cN, Z[n], cNW, Z[n - 1], acc );
+         acc           = fma2( cS, Z[-n - 1], cSE, Z[-n], acc );
+         T up          = fma2( cTC, Z[tc], cTW, Z[tc - 1] );
+         up            = fma2( cTS, Z[tc - n], cTSE, Z[tc - n + 1], up );
+         T dn          = fma2( cBC, Z[bc], cBE, Z[bc + 1] );
+         dn            = fma2( cBN, Z[bc + n + 1], cBNW, Z[bc + n], dn );
+         put( co + r0, acc + ( up + dn ) );
+      }
+   }
+   // the last threads take the faces, the ones before them the edges, so that the parts' loads run side by side
+   for ( int k = nt - 1 - tid; k < 4 * nf; k += nt )
+   {
+      const int lf = k / nf, q = k % nf, face = pick( C.face, lf );
+      if ( !( C.write >> ( 10 + lf ) & 1 ) || !( pick( C.fType, lf ) & flag ) ) continue;
+      const T*       fw  = S.FW + face * kFaceW;
+      const int32_t *nbr = S.faceNbr + ( face * nf + q ) * 8, *M = C.fMap + 9 * lf;
+      T              v[8];
+#pragma unroll
+      for ( int j = 0; j < 8; j++ )
+         v[j] = u[max( nbr[j], 0 )];
+      int i, j;
+      triPos( m, q, i, j );
+      i++, j++;
+      auto U = [&]( int ii, int jj ) {
+         return V[cellRel( w, t0, M[0] + ii * M[3] + jj * M[6], M[1] + ii * M[4] + jj * M[7], M[2] + ii * M[5] + jj * M[8] )];
+      };
+      T acc = faceInPlane( fw, U( i - 1, j ), U( i + 1, j ), U( i, j + 1 ), U( i, j - 1 ), U( i - 1, j + 1 ), U( i + 1, j - 1 ) );
+      acc   = fmaT( fw[0], U( i, j ), acc );
+#pragma unroll
+      for ( int t = 0; t < 8; t++ )
+         if ( t < 4 * pick( C.fSides, lf ) ) acc = fmaT( fw[7 + t], v[t], acc );
+      put( g.offF + face * g.fS + fidx( w, i, j ), acc );
+   }
+   for ( int k = ( tid + nt / 2 ) % nt; k < 6 * np; k += nt )
+   {
+      const int le = k / np, x = 1 + k % np, edge = pick( C.edge, le ), ends = pick( C.ends, le );
+      if ( !( C.write >> ( 4 + le ) & 1 ) || !( pick( C.eType, le ) & flag ) ) continue;
+      const int      n = pick( C.eTerms, le ), off = pick( C.eTermOff, le ), from = ends & 3, to = ends >> 2;
+      const T*       ew  = S.EW + 3 * edge + off;
+      const int32_t* nbr = S.edgeNbr + off * np + ( x - 1 ) * n;
+      auto           U   = [&]( int xx ) {
+         auto at = [&]( int d ) { return from == d ? w - 1 - xx : to == d ? xx : 0; };
+         return V[cellRel( w, t0, at( 1 ), at( 2 ), at( 3 ) )];
+      };
+      T acc = fmaT( ew[1], U( x ), fma2( ew[0], U( x - 1 ), ew[2], U( x + 1 ) ) ), sum = T( 0 );
+      for ( int k0 = 0; k0 < n; k0 += 2 * kTermBatch )
+      {
+         T v[2 * kTermBatch], wt[2 * kTermBatch];
+#pragma unroll
+         for ( int j = 0; j < 2 * kTermBatch; j++ )
+         {
+            v[j]  = u[nbr[min( k0 + j, n - 1 )]];
+            wt[j] = ew[3 + min( k0 + j, n - 1 )];
+         }
+#pragma unroll
+         for ( int j = 0; j < 2 * kTermBatch; j++ )
+            if ( k0 + j < n ) sum = fmaT( wt[j], v[j], sum );
+      }
+      put( g.offE + edge * g.eS + x, acc + sum );
+   }
+   const int v = __builtin_amdgcn_readfirstlane( tid >> 6 );
+   if ( v < 4 && ( C.write >> v & 1 ) && ( C.vType[v] & flag ) )
+   {
+      // the lanes load the terms, summed in their order
+      const T*  vw  = S.VW + C.vert[v] + C.vTermOff[v];
+      const int n   = C.vTerms[v];
+      T         acc = vw[0] * u[C.vert[v]];
+      for ( int k0 = 0; k0 < n; k0 += 64 )
+      {
+         const int k  = min( k0 + lane, n - 1 );
+         const T   wt = vw[1 + k], x = u[S.vterms[C.vTermOff[v] + k]];
+         for ( int q = 0; q < min( 64, n - k0 ); q++ )
+            acc = fmaT( __shfl( wt, q, 64 ), __shfl( x, q, 64 ), acc );
+      }
+      if ( lane == 0 ) put( C.vert[v], acc );
+   }
 }
 
 template < typename T >
@@ -4236,6 +4348,21 @@ void refreshT( Function& f, int level, int mask )
                           dim3( 256 ), 0, s, g, P.dF2C.p, u, (T*) nullptr );
 }
 
+template < typename T >
+SweepCellTables< T > sweepCellTables( const LevelPlan& P, Operator::LevelWeights& Wt )
+{
+   return { P.cellLocal, P.own, P.edgeNbr, P.faceNbr, P.dColourPts.p, P.dVertexTerms.p,
+            wsel< T >( Wt.vertex64, Wt.vertex32 ), wsel< T >( Wt.edge64, Wt.edge32 ), wsel< T >( Wt.face64, Wt.face32 ),
+            wsel< T >( Wt.cell64, Wt.cell32 ) };
+}
+ColourStarts colourStarts( const LevelPlan& P )
+{
+   ColourStarts cs;
+   for ( int k = 0; k < 5; k++ )
+      cs.s[k] = P.colourStart[k];
+   return cs;
+}
+
 // cells = false leaves out the macro-cell interiors (the fused residual-and-restriction pass computes those)
 template < typename T, int NR >
 void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, int level, int flag, int mode,
@@ -4249,6 +4376,30 @@ void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, in
    const T*    u  = (const T*) src.ptr( level );
    T*          y  = (T*) dst.ptr( level );
    const T*    b  = rhs ? (const T*) rhs->ptr( level ) : nullptr;
+   if constexpr ( NR == 1 )
+      if ( cells && P.sweepScratch ) // small levels, their tables prepared with the operator
+      {
+         const SweepCellTables< T > S  = sweepCellTables< T >( P, Wt );
+         const ColourStarts         cs = colourStarts( P );
+#define HYMI_APPLY( LMAX, MODE )                                                                                     \
+   hipLaunchKernelGGL( ( kApplyCell< T, LMAX, MODE > ), dim3( M.T.nC() ), dim3( kApplyCellThreads ), 0, s, g, S, cs, \
+                       flag, u, y, b )
+         auto go = [&]( auto lmax ) {
+            constexpr int LMAX = decltype( lmax )::value;
+            if ( mode == kReplace )
+               HYMI_APPLY( LMAX, kReplace );
+            else if ( mode == kAdd )
+               HYMI_APPLY( LMAX, kAdd );
+            else
+               HYMI_APPLY( LMAX, kResidual );
+         };
+#undef HYMI_APPLY
+         if ( level <= 3 )
+            go( std::integral_constant< int, 3 >{} );
+         else
+            go( std::integral_constant< int, kSweepCellMaxLevel >{} );
+         return;
+      }
    if ( refreshSrc ) refreshT< T, NR >( src, level, 7 );
    const T* VW = wsel< T >( Wt.vertex64, Wt.vertex32 );
    const T* EW = wsel< T >( Wt.edge64, Wt.edge32 );
@@ -4340,12 +4491,8 @@ void sweepCells( Operator& op, Function& xf, const Function& bf, double omega, i
    auto&       Wt = op.weights( level );
    hipStream_t s  = M.ctx->stream;
    T *         u = (T*) xf.ptr( level ), *other = reinterpret_cast< T* >( P.sweepScratch );
-   const SweepCellTables< T > S{ P.cellLocal, P.own, P.edgeNbr, P.faceNbr, P.dColourPts.p, P.dVertexTerms.p,
-                                 wsel< T >( Wt.vertex64, Wt.vertex32 ), wsel< T >( Wt.edge64, Wt.edge32 ),
-                                 wsel< T >( Wt.face64, Wt.face32 ), wsel< T >( Wt.cell64, Wt.cell32 ) };
-   ColourStarts cs;
-   for ( int k = 0; k < 5; k++ )
-      cs.s[k] = P.colourStart[k];
+   const SweepCellTables< T > S  = sweepCellTables< T >( P, Wt );
+   const ColourStarts         cs = colourStarts( P );
    for ( int k = 0; k < count; k++ )
    {
       const T* src = k % 2 ? other : u;

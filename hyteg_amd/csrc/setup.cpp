@@ -927,10 +927,14 @@ void Mesh::prepareSweepCell( LevelPlan& P )
             faceEdgePoint( T, f, le, w, x, 0, p );
             own[P.faceOff( f ) + faceIndex( w, p[0], p[1] )] = own[P.edgeOff( T.fe[f][le] ) + x];
          }
-   auto cellAt = [&]( int c, const FaceCellMap& M, int i, int j, int layer ) {
-      return P.cellOff( c ) + cellIndex( w, M.base[0] + i * M.a[0] + j * M.b[0] + layer * M.o[0],
-                                         M.base[1] + i * M.a[1] + j * M.b[1] + layer * M.o[1],
-                                         M.base[2] + i * M.a[2] + j * M.b[2] + layer * M.o[2] );
+   // cell-relative index from a table of the slabs' starts (this runs once per table entry)
+   std::vector< int > slab( w + 1 );
+   for ( int z = 0; z <= w; z++ )
+      slab[z] = (int) cellIndex( w, 0, 0, z );
+   auto inCellAt = [&]( int x, int y, int z ) { return slab[z] + y * ( w - z + 1 ) - y * ( y + 1 ) / 2 + x; };
+   auto cellAt   = [&]( const FaceCellMap& M, int i, int j, int layer ) {
+      return inCellAt( M.base[0] + i * M.a[0] + j * M.b[0] + layer * M.o[0], M.base[1] + i * M.a[1] + j * M.b[1] + layer * M.o[1],
+                         M.base[2] + i * M.a[2] + j * M.b[2] + layer * M.o[2] );
    };
    std::vector< CellLocal > cells( T.nC() );
    for ( int c = 0; c < T.nC(); c++ )
@@ -943,7 +947,7 @@ void Mesh::prepareSweepCell( LevelPlan& P )
          const FaceCellMap M = numericMap( T, c, lf, w );
          for ( int j = 0; j < w; j++ )
             for ( int i = 0; i + j < w; i++ )
-               own[cellAt( c, M, i, j, 0 )] = own[P.faceOff( f ) + faceIndex( w, i, j )];
+               own[P.cellOff( c ) + cellAt( M, i, j, 0 )] = own[P.faceOff( f ) + faceIndex( w, i, j )];
          const VertexGeom& v = P.hVertexGeom[T.cv[c][lf]];
          C.vert[lf]          = T.cv[c][lf];
          C.vTermOff[lf] = v.termOff, C.vTerms[lf] = v.nTerms, C.vType[lf] = v.type;
@@ -970,7 +974,7 @@ void Mesh::prepareSweepCell( LevelPlan& P )
             const EdgeTerm& t = P.hEdgeTerms[G.termOff + k];
             const int       q[3] = { t.base[0] + x * t.inc[0], t.base[1] + x * t.inc[1], t.base[2] + x * t.inc[2] };
             edgeNbr.push_back( own[t.kind == 0 ? P.faceOff( t.prim ) + faceIndex( w, q[0], q[1] )
-                                               : P.cellOff( t.prim ) + cellIndex( w, q[0], q[1], q[2] )] );
+                                               : P.cellOff( t.prim ) + inCellAt( q[0], q[1], q[2] )] );
          }
    faceNbr.reserve( (size_t) T.nF() * nf * 8 );
    for ( const FaceGeom& G : P.hFaceGeom )
@@ -978,27 +982,31 @@ void Mesh::prepareSweepCell( LevelPlan& P )
          for ( int i = 1; i + j <= w - 2; i++ )
             for ( int sd = 0; sd < 2; sd++ )
                for ( int k = 0; k < 4; k++ )
-                  faceNbr.push_back( sd < G.nSides ? own[cellAt( G.side[sd].cell, G.side[sd], i + G.offCol[sd][k],
-                                                                 j + G.offRow[sd][k], 1 )]
+                  faceNbr.push_back( sd < G.nSides ? own[P.cellOff( G.side[sd].cell ) + cellAt( G.side[sd], i + G.offCol[sd][k],
+                                                                                                j + G.offRow[sd][k], 1 )]
                                                    : -1 );
-   // one allocation and one copy: the scratch array (cleared: its padding is copied with it), then the tables
+   // one allocation: the tables, then the scratch array (cleared: its padding is copied with it; copied with the tables
+   // where that is shorter than a fill's launch)
    const size_t           nScratch = 2 * (size_t) P.total, nCells = cells.size() * ( sizeof( CellLocal ) / 4 );
    std::vector< int32_t > all( nCells );
    std::memcpy( all.data(), cells.data(), 4 * nCells );
    for ( const auto* t : { &own, &edgeNbr, &faceNbr } )
       all.insert( all.end(), t->begin(), t->end() );
-   P.sweepTables.alloc( nScratch + all.size() );
+   const size_t nTables = ( all.size() + 63 ) / 64 * 64;
+   const bool   fill    = nScratch > 50000;
+   all.resize( nTables + ( fill ? 0 : nScratch ), 0 );
+   P.sweepTables.alloc( nTables + nScratch );
    {
       HYMI_LEGACY_LOCK;
-      HYMI_HIP( hipMemsetAsync( P.sweepTables.p, 0, 4 * nScratch, ctx->stream ) );
-      HYMI_HIP( hipMemcpyAsync( P.sweepTables.p + nScratch, all.data(), 4 * all.size(), hipMemcpyHostToDevice, ctx->stream ) );
+      if ( fill ) HYMI_HIP( hipMemsetAsync( P.sweepTables.p + nTables, 0, 4 * nScratch, ctx->stream ) );
+      HYMI_HIP( hipMemcpyAsync( P.sweepTables.p, all.data(), 4 * all.size(), hipMemcpyHostToDevice, ctx->stream ) );
    }
    HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
-   P.cellLocal    = reinterpret_cast< const CellLocal* >( P.sweepTables.p + nScratch );
-   P.own          = P.sweepTables.p + nScratch + nCells;
+   P.cellLocal    = reinterpret_cast< const CellLocal* >( P.sweepTables.p );
+   P.own          = P.sweepTables.p + nCells;
    P.edgeNbr      = P.own + own.size();
    P.faceNbr      = P.edgeNbr + edgeNbr.size();
-   P.sweepScratch = reinterpret_cast< double* >( P.sweepTables.p );
+   P.sweepScratch = reinterpret_cast< double* >( P.sweepTables.p + nTables );
 }
 
 // Work units and scratch arrays of the fused SOR cell phase selected on P (nothing if the passes are selected or
