@@ -304,19 +304,10 @@ __global__ __launch_bounds__( 256 ) void kF2C( LV g, const F2C* __restrict__ tab
    }
 }
 
-// Face-to-cell copy of the points within distance 1 of a face's boundary only (rows 0 and 1, and the first two and
-// last two points of every other row: 6w - 9 points), from the faces of u into the cell closures of dst.  These are
-// the closure points that the edge terms and the face ghost layers of the next sweep read from a macro-cell (the
-// fused cell phase reads closure points from the faces themselves).  Block = (chunk of 256 points, cell face).
-template < typename T >
-__global__ __launch_bounds__( 256 ) void kF2CBand( LV g, const F2C* __restrict__ tab, const T* __restrict__ u,
-                                                   T* __restrict__ dst )
+// the e-th point (i, j) within distance 1 of a face's boundary (e < 6w - 9); false where there is none
+__device__ __forceinline__ bool f2cBandPoint( int w, int e, int& i, int& j )
 {
-   const F2C m  = tab[blockIdx.y];
-   const int w  = g.w, nb = 6 * w - 9;
-   const int e  = (int) blockIdx.x * 256 + (int) threadIdx.x;
-   if ( e >= nb ) return;
-   int i, j;
+   if ( e >= 6 * w - 9 ) return false;
    if ( e < w )
       j = 0, i = e;
    else if ( e < 2 * w - 1 )
@@ -327,7 +318,21 @@ __global__ __launch_bounds__( 256 ) void kF2CBand( LV g, const F2C* __restrict__
       j           = 2 + ( ( e - ( 2 * w - 1 ) ) >> 2 );
       i           = k < 2 ? k : w - j - 4 + k;
    }
-   if ( i < 0 || i > w - 1 - j ) return; // short rows near the top corner
+   return i >= 0 && i <= w - 1 - j; // short rows near the top corner
+}
+
+// Face-to-cell copy of the points within distance 1 of a face's boundary only (rows 0 and 1, and the first two and
+// last two points of every other row: 6w - 9 points), from the faces of u into the cell closures of dst.  These are
+// the closure points that the edge terms and the face ghost layers of the next sweep read from a macro-cell (the
+// fused cell phase reads closure points from the faces themselves).  Block = (chunk of 256 points, cell face).
+template < typename T >
+__global__ __launch_bounds__( 256 ) void kF2CBand( LV g, const F2C* __restrict__ tab, const T* __restrict__ u,
+                                                   T* __restrict__ dst )
+{
+   const F2C m = tab[blockIdx.y];
+   const int w = g.w;
+   int       i, j;
+   if ( !f2cBandPoint( w, (int) blockIdx.x * 256 + (int) threadIdx.x, i, j ) ) return;
    const int x = m.m.base[0] + i * m.m.a[0] + j * m.m.b[0];
    const int y = m.m.base[1] + i * m.m.a[1] + j * m.m.b[1];
    const int z = m.m.base[2] + i * m.m.a[2] + j * m.m.b[2];
@@ -352,7 +357,7 @@ __device__ __forceinline__ int64_t refreshEdgeSrc( const LV& g, const V2E* __res
 template < typename T, int NR >
 __global__ __launch_bounds__( 256 ) void kRefresh( LV g, const V2E* __restrict__ v2e, int nE, const E2F* __restrict__ e2f,
                                                   int nF, const F2C* __restrict__ f2c, int nPairs, int mask, int nA,
-                                                  int nB, int chunks, T* __restrict__ u )
+                                                  int nB, int chunks, int band, T* __restrict__ u )
 {
    const int  w = g.w, blk = (int) blockIdx.x;
    const bool fromVertex = ( mask & 1 ) != 0, fromEdge = ( mask & 2 ) != 0;
@@ -384,31 +389,40 @@ __global__ __launch_bounds__( 256 ) void kRefresh( LV g, const V2E* __restrict__
    const int     t0 = tet32( w ), nV = ( w * ( w + 1 ) >> 1 ) * NR;
    const int64_t fo = g.offF + (int64_t) m.face * g.fS;
    T*            cu = u + ( g.offC + (int64_t) m.m.cell * g.cS ) * NR;
-   const int     e0 = ( q - pair * chunks ) * 256 * kF2CBatch + (int) threadIdx.x;
-   T             v[kF2CBatch];
-   int           o[kF2CBatch];
-#pragma unroll
-   for ( int k = 0; k < kF2CBatch; k++ )
-   {
-      const int e = e0 + 256 * k, ec = e < nV ? e : 0, p = ec / NR, r = ec % NR;
-      const int j = triRow32( w, p ), i = p - j * ( 2 * w + 1 - j ) / 2;
+   auto          cellPoint = [&]( int i, int j ) {
       const int x = m.m.base[0] + i * m.m.a[0] + j * m.m.b[0];
       const int y = m.m.base[1] + i * m.m.a[1] + j * m.m.b[1];
       const int z = m.m.base[2] + i * m.m.a[2] + j * m.m.b[2];
-      o[k]        = ( crow32( w, t0, y, z ) + x ) * NR + r;
-      int64_t src = fo + p;                     // face interior, or the face's own copy of its boundary
+      return crow32( w, t0, y, z ) + x;
+   };
+   auto source = [&]( int i, int j, int p ) -> int64_t { // where face point (i, j), index p, is read
       if ( fromEdge && ( i == 0 || j == 0 || i + j == w - 1 ) )
          for ( int le = 0; le < 3; le++ ) // the face edge through (i, j); corners lie on two, same owner value
          {
             const E2F me = e2f[3 * m.face + le];
             const int te = me.inc[0] != 0 ? ( i - me.base[0] ) * me.inc[0] : ( j - me.base[1] ) * me.inc[1];
             if ( te >= 0 && te <= w - 1 && me.base[0] + te * me.inc[0] == i && me.base[1] + te * me.inc[1] == j )
-            {
-               src = refreshEdgeSrc< T, NR >( g, v2e, me.edge, te, fromVertex );
-               break;
-            }
+               return refreshEdgeSrc< T, NR >( g, v2e, me.edge, te, fromVertex );
          }
-      v[k] = u[src * NR + r];
+      return fo + p; // face interior, or the face's own copy of its boundary
+   };
+   if ( band ) // only the points within distance 1 of the face's boundary (one right-hand side, see kF2CBand)
+   {
+      int i, j;
+      if ( f2cBandPoint( w, ( q - pair * chunks ) * 256 + (int) threadIdx.x, i, j ) )
+         cu[cellPoint( i, j )] = u[source( i, j, fidx( w, i, j ) )];
+      return;
+   }
+   const int e0 = ( q - pair * chunks ) * 256 * kF2CBatch + (int) threadIdx.x;
+   T         v[kF2CBatch];
+   int       o[kF2CBatch];
+#pragma unroll
+   for ( int k = 0; k < kF2CBatch; k++ )
+   {
+      const int e = e0 + 256 * k, ec = e < nV ? e : 0, p = ec / NR, r = ec % NR;
+      const int j = triRow32( w, p ), i = p - j * ( 2 * w + 1 - j ) / 2;
+      o[k]        = cellPoint( i, j ) * NR + r;
+      v[k]        = u[source( i, j, p ) * NR + r];
    }
 #pragma unroll
    for ( int k = 0; k < kF2CBatch; k++ )
@@ -3250,7 +3264,7 @@ __global__ __launch_bounds__( 64 * ( 2 * kResBandY + 1 ), 8 ) void kResidualRest
 
 template < typename T, int NR >
 __device__ __forceinline__ void kRestrictFace_b( const Blk& B, LV gc, LV gf, const FaceGeom* __restrict__ fgFine, int flag, const T* __restrict__ uf,
-                               T* __restrict__ uc )
+                               T* __restrict__ uc, const int32_t* __restrict__ own )
 {
    const FaceGeom& G = fgFine[B.y];
    if ( !( G.type & flag ) ) return;
@@ -3280,7 +3294,8 @@ __device__ __forceinline__ void kRestrictFace_b( const Blk& B, LV gc, LV gf, con
          const int x   = M.base[0] + col * M.a[0] + row * M.b[0] + M.o[0];
          const int y   = M.base[1] + col * M.a[1] + row * M.b[1] + M.o[1];
          const int z   = M.base[2] + col * M.a[2] + row * M.b[2] + M.o[2];
-         acc += uf[( cb + cellRel( w, tet32( w ), x, y, z ) ) * NR + r];
+         const int64_t o = cb + cellRel( w, tet32( w ), x, y, z );
+         acc += uf[( own ? own[o] : o ) * NR + r];
       }
    }
    const int64_t co = gc.offF + (int64_t) G.face * gc.fS;
@@ -3289,7 +3304,7 @@ __device__ __forceinline__ void kRestrictFace_b( const Blk& B, LV gc, LV gf, con
 
 template < typename T, int NR >
 __device__ __forceinline__ void kRestrictEdge_b( const Blk& B, LV gc, LV gf, const EdgeGeom* __restrict__ egFine, const EdgeTerm* __restrict__ terms,
-                               int flag, const T* __restrict__ uf, T* __restrict__ uc )
+                               int flag, const T* __restrict__ uf, T* __restrict__ uc, const int32_t* __restrict__ own )
 {
    const EdgeGeom& G = egFine[B.y];
    if ( !( G.type & flag ) ) return;
@@ -3311,7 +3326,8 @@ __device__ __forceinline__ void kRestrictEdge_b( const Blk& B, LV gc, LV gf, con
       {
          const EdgeTerm& e = terms[G.termOff + min( k0 + q, n - 1 )];
          wr[q]             = e.wr;
-         v[q]              = uf[edgeTermIndex< T, NR >( gf, e, x, t0 ) * NR + r];
+         const int64_t o   = edgeTermIndex< T, NR >( gf, e, x, t0 );
+         v[q]              = uf[( own ? own[o] : o ) * NR + r];
       }
 #pragma unroll
       for ( int q = 0; q < kTermBatch; q++ )
@@ -3355,7 +3371,8 @@ __device__ __forceinline__ void kZeroRanges_b( const Blk& B, const Range* __rest
 }
 
 // a restriction in one launch (LowGrid): vertex, edge and face parts, the macro-cell part (one right-hand side:
-// kRestrictFlat_b over the coarse level's transfer units) and the zeroing of the coarse level of another function (ranges zr)
+// kRestrictFlat_b over the coarse level's transfer units) and the zeroing of the coarse level of another function (ranges
+// zr).  own (small levels, else null): the fine level's owners, read in place of closure copies, which then need no refresh
 template < typename T, int NR >
 __global__ __launch_bounds__( 256 ) void kLowRestrict( LowGrid L, LV gc, LV gf, const VertexGeom* __restrict__ vgFine,
                                                        const int64_t* __restrict__ vtermsFine, int nV,
@@ -3365,16 +3382,16 @@ __global__ __launch_bounds__( 256 ) void kLowRestrict( LowGrid L, LV gc, LV gf, 
                                                        const T* __restrict__ uf, T* __restrict__ uc,
                                                        const MarchUnit* __restrict__ cellUnits, int64_t nCellUnits,
                                                        const int* __restrict__ ctypeC, const Range* __restrict__ zr,
-                                                       T* __restrict__ zdst )
+                                                       T* __restrict__ zdst, const int32_t* __restrict__ own )
 {
    Blk       B;
    const int part = lowPart( L, B );
    if ( part == 0 )
       kRestrictVertex_b< T, NR >( B, vgFine, vtermsFine, nV, flag, uf, uc );
    else if ( part == 1 )
-      kRestrictEdge_b< T, NR >( B, gc, gf, egFine, etermsFine, flag, uf, uc );
+      kRestrictEdge_b< T, NR >( B, gc, gf, egFine, etermsFine, flag, uf, uc, own );
    else if ( part == 2 )
-      kRestrictFace_b< T, NR >( B, gc, gf, fgFine, flag, uf, uc );
+      kRestrictFace_b< T, NR >( B, gc, gf, fgFine, flag, uf, uc, own );
    else if ( part == 3 )
    {
       if constexpr ( NR == 1 ) kRestrictFlat_b< T >( B, gc, gf, cellUnits, nCellUnits, ctypeC, flag, uf, uc );
@@ -4311,28 +4328,22 @@ void refreshT( Function& f, int level, int mask )
    hipStream_t s = M.ctx->stream;
    T*          u = (T*) f.ptr( level );
    if ( M.T.nC() == 0 ) mask &= 3;
-   // bit 8: of the face-to-cell step only the points within distance 1 of the faces' edges (kF2CBand), for
-   // readers that take no other cell closure point (one right-hand side; else the whole copy)
-   if ( mask & 8 )
-   {
-      refreshT< T, NR >( f, level, mask & 3 );
-      if ( NR == 1 )
-         hipLaunchKernelGGL( ( kF2CBand< T > ), dim3( (unsigned) ( ( 6 * P.w - 9 + 255 ) / 256 ), 4 * M.T.nC() ),
-                             dim3( 256 ), 0, s, g, P.dF2C.p, (const T*) u, u );
-      else
-         refreshT< T, NR >( f, level, 4 );
-      return;
-   }
+   // bit 8: of the face-to-cell step only the points within distance 1 of the faces' edges (see kF2CBand), for readers
+   // that take no other cell closure point (one right-hand side; else the whole copy).  In the same launch as the other
+   // steps (two launches before: 4 us of every residual, restriction and ping-pong pair)
+   const bool band = ( mask & 8 ) != 0 && NR == 1;
+   if ( mask & 8 ) mask = ( mask & 3 ) | ( M.T.nC() > 0 ? 4 : 0 );
    if ( mask == 3 || mask == 5 || mask == 6 || mask == 7 ) // several steps: one launch reading the owners
    {
       const int     nA = ( mask & 1 ) ? (int) blocksFor( 2 * (int64_t) M.T.nE() * NR, 256 ) : 0;
       const int     nB = ( mask & 2 ) ? (int) blocksFor( 3 * (int64_t) M.T.nF() * P.w * NR, 256 ) : 0;
-      const int     chunks = (int) ( ( (int64_t) P.w * ( P.w + 1 ) / 2 * NR + 256 * kF2CBatch - 1 ) / ( 256 * kF2CBatch ) );
+      const int     chunks = band ? ( 6 * P.w - 9 + 255 ) / 256
+                                  : (int) ( ( (int64_t) P.w * ( P.w + 1 ) / 2 * NR + 256 * kF2CBatch - 1 ) / ( 256 * kF2CBatch ) );
       const int     nPairs = ( mask & 4 ) ? 4 * M.T.nC() : 0;
       const int64_t nBlk   = (int64_t) nA + nB + (int64_t) nPairs * chunks;
       if ( nBlk > 0 )
          hipLaunchKernelGGL( ( kRefresh< T, NR > ), dim3( (unsigned) nBlk ), dim3( 256 ), 0, s, g, P.dV2E.p, M.T.nE(),
-                             P.dE2F.p, M.T.nF(), P.dF2C.p, nPairs, mask, nA, nB, chunks, u );
+                             P.dE2F.p, M.T.nF(), P.dF2C.p, nPairs, mask, nA, nB, chunks, band ? 1 : 0, u );
       return;
    }
    if ( mask & 1 )
@@ -4743,13 +4754,10 @@ void sorSweepsT( Operator& op, Function& xf, const Function& bf, double omega, i
       sorT< T, NR >( op, xf, bf, omega, level, flag, refreshFirst && k == 0, false, k );
 }
 
-// bandOnly: the source's cell closures are refreshed only within distance 1 of the faces' edges, which is all
-// the restriction reads of them (the cell-interior part gathers interior fine points only); for a scratch source
-// whose other closure points nobody reads afterwards
 // cells = false leaves out the macro-cell interiors of the coarse level; zeroCoarse (may be null): a function whose
 // coarse level (all primitives) is set to zero in the same launch
 template < typename T, int NR >
-void restrictT( Function& f, Function& dst, int srcLevel, int flag, bool bandOnly = false, bool cells = true,
+void restrictT( Function& f, Function& dst, int srcLevel, int flag, bool cells = true,
                 Function* zeroCoarse = nullptr )
 {
    Mesh&       M  = *f.mesh;
@@ -4759,7 +4767,10 @@ void restrictT( Function& f, Function& dst, int srcLevel, int flag, bool bandOnl
    hipStream_t s  = M.ctx->stream;
    const T*    uf = (const T*) f.ptr( srcLevel );
    T*          uc = (T*) dst.ptr( srcLevel - 1 );
-   refreshT< T, NR >( f, srcLevel, bandOnly && NR == 1 ? 1 | 2 | 8 : 7 );
+   // of the cells' closures the restriction reads points within distance 1 of the faces' edges only (the cell-interior part
+   // gathers interior fine points); on small levels it reads the owners instead
+   const int32_t* own = NR == 1 ? Pf.own : nullptr;
+   if ( !own ) refreshT< T, NR >( f, srcLevel, NR == 1 ? 1 | 2 | 8 : 7 );
    const int nV = M.T.nV(), nE = M.T.nE(), nF = M.T.nF();
    // coarse vertices, edge interiors, face interiors and (one right-hand side) macro-cell interiors in one launch,
    // with the zeroing of zeroCoarse
@@ -4787,7 +4798,7 @@ void restrictT( Function& f, Function& dst, int srcLevel, int flag, bool bandOnl
    T* zdst         = zeroCoarse ? (T*) zeroCoarse->ptr( srcLevel - 1 ) : nullptr;
    hipLaunchKernelGGL( ( kLowRestrict< T, NR > ), dim3( lowBlocks( lg ) ), dim3( 256 ), 0, s, lg, gc, gf, Pf.dVertexGeom.p,
                        Pf.dVertexTerms.p, nV, Pf.dEdgeGeom.p, Pf.dEdgeTerms.p, Pf.dFaceGeom.p, flag, uf, uc, mu, nu,
-                       Pc.dCellType.p, zr, zdst );
+                       Pc.dCellType.p, zr, zdst, own );
    if ( !cells || NR == 1 ) return;
    int64_t        nseg = 0;
    rowSegFits< NR >( Pf );
@@ -4810,7 +4821,7 @@ void residualRestrictT( Operator& op, Function& x, Function& r, Function& b, int
    if ( NR > 1 || !M.residualRestrictOn( L ) )
    {
       applyT< T, NR >( op, x, r, &b, L, flag, kResidual, refreshSrc );
-      restrictT< T, NR >( r, b, L, flag, true, true, zeroCoarse );
+      restrictT< T, NR >( r, b, L, flag, true, zeroCoarse );
       return;
    }
    LevelPlan&       Pc = M.plan( L - 1 );
@@ -4824,7 +4835,7 @@ void residualRestrictT( Operator& op, Function& x, Function& r, Function& b, int
                           M.ctx->stream, viewOf( Pf ), viewOf( Pc ), mu, n, extra, wsel< T >( Wt.cell64, Wt.cell32 ),
                           Pf.dCellType.p, flag, (const T*) x.ptr( L ), (const T*) b.ptr( L ), (T*) r.ptr( L ),
                           (T*) b.ptr( L - 1 ) );
-   restrictT< T, NR >( r, b, L, flag, true, false, zeroCoarse );
+   restrictT< T, NR >( r, b, L, flag, false, zeroCoarse );
 }
 
 template < typename T, int NR, bool REPL >
@@ -5018,9 +5029,9 @@ struct SorSweepsF
 template < typename T, int NR >
 struct RestrictF
 {
-   static void run( Function& f, Function& d, int L, int flag, bool bandOnly )
+   static void run( Function& f, Function& d, int L, int flag )
    {
-      restrictT< T, NR >( f, d, L, flag, bandOnly );
+      restrictT< T, NR >( f, d, L, flag );
    }
 };
 template < typename T, int NR >
@@ -5137,11 +5148,11 @@ void launchSorSweeps( Operator& op, Function& x, const Function& b, double omega
    dispatch< SorSweepsF >( x.prec, x.nrhs, op, x, b, omega, level, flag, count, refreshFirst );
 }
 
-void launchRestrict( Function& f, Function& dst, int srcLevel, int flag, bool bandOnly )
+void launchRestrict( Function& f, Function& dst, int srcLevel, int flag )
 {
    if ( dst.prec != f.prec || dst.nrhs != f.nrhs || dst.mesh != f.mesh )
       throw std::runtime_error( "restrict: source and destination must share mesh, precision and nrhs" );
-   dispatch< RestrictF >( f.prec, f.nrhs, f, dst, srcLevel, flag, bandOnly );
+   dispatch< RestrictF >( f.prec, f.nrhs, f, dst, srcLevel, flag );
 }
 
 void launchResidualRestrict( Operator& op, Function& x, Function& r, Function& b, int level, int flag, bool refreshSrc,

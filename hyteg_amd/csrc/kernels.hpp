@@ -29,8 +29,7 @@ void launchSor( Operator& op, Function& x, const Function& b, double omega, int 
 void launchSorSweeps( Operator& op, Function& x, const Function& b, double omega, int level, int flag, int count,
                       bool refreshFirst = true );
 // coarse level of dst <- restriction of the fine level of f (dst may be f)
-// bandOnly: refresh the source's cell closures only where the restriction reads them (a scratch source)
-void launchRestrict( Function& f, Function& dst, int srcLevel, int flag, bool bandOnly = false );
+void launchRestrict( Function& f, Function& dst, int srcLevel, int flag );
 // r = b - A x on `level`, restricted into b on level - 1 (flag DoFs); r is scratch afterwards (of its macro-cell
 // interiors only the points next to the faces are written where the level fuses the two passes).  zeroCoarse (may
 // be null): a function whose level - 1 is set to zero on every primitive in the restriction's launch
