@@ -1308,7 +1308,7 @@ int hymi_smooth_sor( hymi_operator op, hymi_function x, hymi_function b, double 
       require( x != b, "x and b must differ" );
       require( x->f.prec == b->f.prec && x->f.nrhs == b->f.nrhs, "functions must share precision and nrhs" );
       op->op.mesh->prepareCellSor( op->op.mesh->plan( level ) );
-      launchSor( op->op, x->f, b->f, omega, level, flag );
+      launchSorSweeps( op->op, x->f, b->f, omega, level, flag, 1 );
    } );
 }
 

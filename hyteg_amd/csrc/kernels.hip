@@ -2729,6 +2729,20 @@ __global__ __launch_bounds__( kApplyCellThreads ) void kApplyCell( LV g, SweepCe
    }
 }
 
+// copy of 16 bytes per thread and step, kCopyBatch steps in flight
+constexpr int kCopyBatch = 4;
+__global__ __launch_bounds__( 256 ) void kCopy16( const uint4* __restrict__ src, uint4* __restrict__ dst, int64_t n )
+{
+   const int64_t k0 = (int64_t) blockIdx.x * ( 256 * kCopyBatch ) + threadIdx.x;
+   uint4         v[kCopyBatch];
+#pragma unroll
+   for ( int q = 0; q < kCopyBatch; q++ )
+      v[q] = src[min( k0 + 256 * q, n - 1 )];
+#pragma unroll
+   for ( int q = 0; q < kCopyBatch; q++ )
+      if ( k0 + 256 * q < n ) dst[k0 + 256 * q] = v[q];
+}
+
 template < typename T >
 __global__ __launch_bounds__( 256 ) void kCopyLevel( const T* __restrict__ src, T* __restrict__ dst, int n )
 {
@@ -4224,6 +4238,15 @@ void cellSorPingPong( Mesh& M, LevelPlan& P, const T* CW, int flag, const T* src
                        (const T*) nullptr, faces, P.dCellFaceRead.p, b, omega, 0 );
 }
 
+// the macro-cell arrays of src to dst (both laid out as the level; the cells start at a multiple of 64 elements)
+template < typename T >
+void copyCells( Mesh& M, const LevelPlan& P, const T* src, T* dst )
+{
+   const int64_t n = (int64_t) M.T.nC() * P.cStride * (int64_t) sizeof( T ) / 16;
+   hipLaunchKernelGGL( kCopy16, dim3( blocksFor( n, 256 * kCopyBatch ) ), dim3( 256 ), 0, M.ctx->stream,
+                       (const uint4*) ( src + P.offC ), (uint4*) ( dst + P.offC ), n );
+}
+
 // Whether a forward smoothing sequence on this level can run its sweeps in ping-pong pairs: the fused cell phase
 // is selected for T (one right-hand side), the face phase reads the cells through ghost layers (levels above the
 // one-workgroup-per-face phase), and every macro-cell is updated (a cell the flag leaves alone would leave the
@@ -4527,7 +4550,8 @@ void sweepCells( Operator& op, Function& xf, const Function& bf, double omega, i
 // values from closure copies, which are refreshed only after the sweep.  Either way every closure copy is
 // current when the sweep ends.
 // pp (forward sweeps on levels where pingPongOk holds): 0 in place; 1 = the macro-cell interiors are read from
-// u and their new values written to the level's ping-pong array B (sorBand); 2 = read from B and written to u.
+// u and their new values written to the level's ping-pong array B (sorBand); 2 = read from B and written to u; 3 = a
+// sweep by itself: the cells of u are copied to B before the cell phase, which reads B and writes u.
 // Within the sweep every kernel that reads macro-cell interiors (edge terms, face ghost layers) reads the array
 // that holds them at that point, and the cell phase reads the closure points from the face arrays, so the
 // interiors of B are at every point what those of u would be in place.  Of the macro-cell closures, the second
@@ -4550,7 +4574,7 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
       if ( !backward && !pp && sweepCellOk< T >( P ) ) return sweepCells< T >( op, xf, bf, omega, level, flag, 1 );
    // a ping-pong pair reads no macro-cell closure point beyond distance 1 of the faces' edges before its final
    // face-to-cell copy
-   if ( refreshFirst ) refreshT< T, NR >( xf, level, pp == 1 ? 1 | 2 | 8 : 7 );
+   if ( refreshFirst ) refreshT< T, NR >( xf, level, pp == 1 || pp == 3 ? 1 | 2 | 8 : 7 );
    if ( NR == 1 && level >= 1 )
    {
       if ( pp && ( backward || !pingPongOk< T, NR >( M, P, flag ) ) )
@@ -4637,6 +4661,7 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
                }
                else
                {
+                  if ( pp == 3 ) copyCells< T >( M, P, u, ppArr );
                   cellSorPingPong< T >( M, P, CW, flag, ppArr, u, u, b, om );
                   hipLaunchKernelGGL( ( kF2C< T, 1 > ),
                                       dim3( (unsigned) ( ( (int64_t) P.w * ( P.w + 1 ) / 2 + 256 * kF2CBatch - 1 ) /
@@ -4727,8 +4752,14 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
    }
 }
 
-// One smoothing sequence of `count` forward sweeps.  Where pingPongOk holds, the sweeps run in pairs (u -> B,
-// B -> u), after one in-place sweep if count is odd; otherwise sweep k is chained to sweep k - 1.
+// One smoothing sequence of `count` forward sweeps.  Where pingPongOk holds, the sweeps run in pairs (u -> B, B -> u), after
+// one by itself (pp 3) if count is odd; otherwise sweep k is chained to sweep k - 1.  A sweep by itself in place needs
+// the band copy (43 % of the points at level 7, gathered row by row) and both face-to-cell copies; a plain copy of the
+// cells is shorter, unless there are fewer tiles than CUs: the sweep then takes as long as its longest tile, whose steps
+// are shorter in place (they choose between no two arrays).  One sweep, us, in place -> by itself: 48 macro-tets FP32
+// level 7 219 -> 199, level 8 1682 -> 1421, FP64 level 7 365 -> 343; 6 macro-tets FP64 level 8 (396 tiles) 416 -> 372,
+// FP32 level 7 (126 tiles) 131 -> 141.
+constexpr int64_t kSorAloneUnits = 256;
 template < typename T, int NR >
 void sorSweepsT( Operator& op, Function& xf, const Function& bf, double omega, int level, int flag, int count,
                  bool refreshFirst )
@@ -4737,12 +4768,13 @@ void sorSweepsT( Operator& op, Function& xf, const Function& bf, double omega, i
    LevelPlan& P = M.plan( level );
    if constexpr ( NR == 1 )
       if ( count > 0 && sweepCellOk< T >( P ) ) return sweepCells< T >( op, xf, bf, omega, level, flag, count );
-   if ( count >= 2 && pingPongOk< T, NR >( M, P, flag ) )
+   if ( pingPongOk< T, NR >( M, P, flag ) )
    {
       M.prepareCellSor( P );
       int k = 0;
       if ( count % 2 == 1 )
-         sorT< T, NR >( op, xf, bf, omega, level, flag, refreshFirst, false, 0 ), k = 1;
+         sorT< T, NR >( op, xf, bf, omega, level, flag, refreshFirst, false, 0, P.sorUnitCount >= kSorAloneUnits ? 3 : 0 ),
+             k = 1;
       for ( ; k < count; k += 2 )
       {
          sorT< T, NR >( op, xf, bf, omega, level, flag, refreshFirst && k == 0, false, 0, 1 );
