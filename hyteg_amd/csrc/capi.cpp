@@ -1200,7 +1200,6 @@ static int makeOperator( hymi_mesh mesh, int minL, int maxL, int form, hymi_oper
       {
          h->op.lw.push_back( std::make_unique< Operator::LevelWeights >() );
          buildOperatorWeights( h->op, L );
-         mesh->m.prepareSweepCell( mesh->m.plan( L ) );
       }
       *out = h.release();
    } );
@@ -1275,6 +1274,12 @@ static void checkOpFunc( hymi_operator op, hymi_function f, int level )
    requireLevel( f->f, level );
 }
 
+// the tables of the one-launch kernels of levels 1 to 4 (one right-hand side), on their first use
+static void prepareSmallLevel( Function& f, int level )
+{
+   if ( f.nrhs == 1 ) f.mesh->prepareSweepCells( level, level );
+}
+
 int hymi_apply( hymi_operator op, hymi_function src, hymi_function dst, int level, int flag, int update )
 {
    return guarded( [&] {
@@ -1283,6 +1288,7 @@ int hymi_apply( hymi_operator op, hymi_function src, hymi_function dst, int leve
       require( src != dst, "src and dst must differ" );
       require( src->f.prec == dst->f.prec && src->f.nrhs == dst->f.nrhs, "src and dst must share precision and nrhs" );
       require( update == HYMI_REPLACE || update == HYMI_ADD, "bad update type" );
+      prepareSmallLevel( src->f, level );
       launchApply( op->op, src->f, dst->f, nullptr, level, flag, update == HYMI_ADD ? kAdd : kReplace );
    } );
 }
@@ -1296,6 +1302,7 @@ int hymi_residual( hymi_operator op, hymi_function x, hymi_function b, hymi_func
       require( x != r, "x and r must differ" );
       require( x->f.prec == r->f.prec && x->f.prec == b->f.prec && x->f.nrhs == r->f.nrhs && x->f.nrhs == b->f.nrhs,
                "functions must share precision and nrhs" );
+      prepareSmallLevel( x->f, level );
       launchApply( op->op, x->f, r->f, &b->f, level, flag, kResidual );
    } );
 }
@@ -1308,6 +1315,7 @@ int hymi_smooth_sor( hymi_operator op, hymi_function x, hymi_function b, double 
       require( x != b, "x and b must differ" );
       require( x->f.prec == b->f.prec && x->f.nrhs == b->f.nrhs, "functions must share precision and nrhs" );
       op->op.mesh->prepareCellSor( op->op.mesh->plan( level ) );
+      prepareSmallLevel( x->f, level );
       launchSorSweeps( op->op, x->f, b->f, omega, level, flag, 1 );
    } );
 }
@@ -1406,6 +1414,7 @@ int hymi_gmg_create( hymi_operator op, hymi_function xt, int minL, int maxL, int
       g->cg.r   = makeFunction( M, minL, minL, g->prec, g->nrhs );
       g->cg.ap  = makeFunction( M, minL, minL, g->prec, g->nrhs );
       // build every table a V-cycle uses now, so that a V-cycle never allocates (graph capture)
+      if ( g->nrhs == 1 ) M.prepareSweepCells( minL, maxL );
       const int segLen = 64 / g->nrhs;
       for ( int L = minL; L <= maxL; L++ )
       {

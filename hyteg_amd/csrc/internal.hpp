@@ -122,11 +122,11 @@ struct LevelPlan
    DevBuf< int64_t >    dVertexSnap;
    DevBuf< int32_t >    dEdgeEnds;
    DevBuf< int32_t >    dCellType;
-   // one-launch sweeps (levels 1 .. kSweepCellMaxLevel; Mesh::prepareSweepCell): per element the element of the primitive
+   // one-launch sweeps (levels 1 .. kSweepCellMaxLevel; Mesh::prepareSweepCells): per element the element of the primitive
    // that owns the value; per edge term and edge point, and per face point and off-plane neighbour (-1: none), the element
    // the term reads, at its owner; the cells; the array that sweeps go to and from (FP64-sized)
-   // (pointers into sweepTables)
-   DevBuf< int32_t > sweepTables;
+   // (pointers into sweepTables, which the levels prepared together share)
+   std::shared_ptr< DevBuf< int32_t > > sweepTables;
    const int32_t *   own = nullptr, *edgeNbr = nullptr, *faceNbr = nullptr;
    const CellLocal*  cellLocal    = nullptr;
    double*           sweepScratch = nullptr;
@@ -212,8 +212,9 @@ struct Mesh
    // the selection alone (no allocation), and the allocation of what the selection needs (outside capture)
    void selectCellSor( int level, int tile, int precisions );
    void prepareCellSor( LevelPlan& P );
-   // tables and scratch array of the one-launch sweep (levels 1 .. kSweepCellMaxLevel; outside capture)
-   void prepareSweepCell( LevelPlan& P );
+   // tables and scratch arrays of the one-launch sweep on the levels of 1 .. kSweepCellMaxLevel in [minL, maxL] (outside
+   // capture)
+   void prepareSweepCells( int minL, int maxL );
    bool cellSorReady( const LevelPlan& P ) const;
    // fused residual and restriction from `level` (one right-hand side): -1 default, 0 off, 1 on (level >= 3);
    // bumps scheduleEpoch like setSchedule

@@ -907,9 +907,10 @@ void Mesh::selectCellSor( int level, int tile, int precisions )
 
 bool Mesh::cellSorReady( const LevelPlan& P ) const { return P.sorTile == 0 || ctx->hostOnly || P.sorUnits != nullptr; }
 
-void Mesh::prepareSweepCell( LevelPlan& P )
+namespace {
+// the tables of one level, in the order cells, own, edgeNbr, faceNbr; start: where the last three begin
+void sweepCellTables( const Topology& T, const LevelPlan& P, std::vector< int32_t >& all, size_t ( &start )[4] )
 {
-   if ( P.L < 1 || P.L > kSweepCellMaxLevel || P.sweepScratch || ctx->hostOnly ) return;
    const int              w = P.w, m = w - 3, nf = m * ( m + 1 ) / 2;
    std::vector< int32_t > own( (size_t) P.total );
    for ( int64_t k = 0; k < P.total; k++ )
@@ -985,35 +986,66 @@ void Mesh::prepareSweepCell( LevelPlan& P )
                   faceNbr.push_back( sd < G.nSides ? own[P.cellOff( G.side[sd].cell ) + cellAt( G.side[sd], i + G.offCol[sd][k],
                                                                                                 j + G.offRow[sd][k], 1 )]
                                                    : -1 );
-   // one allocation: the tables, then the scratch array (cleared: its padding is copied with it; copied with the tables
-   // where that is shorter than a fill's launch)
-   const size_t           nScratch = 2 * (size_t) P.total, nCells = cells.size() * ( sizeof( CellLocal ) / 4 );
-   std::vector< int32_t > all( nCells );
-   std::memcpy( all.data(), cells.data(), 4 * nCells );
-   for ( const auto* t : { &own, &edgeNbr, &faceNbr } )
-      all.insert( all.end(), t->begin(), t->end() );
+   start[0] = all.size();
+   all.resize( start[0] + cells.size() * ( sizeof( CellLocal ) / 4 ) );
+   std::memcpy( all.data() + start[0], cells.data(), cells.size() * sizeof( CellLocal ) );
+   const std::vector< int32_t >* tables[3] = { &own, &edgeNbr, &faceNbr };
+   for ( int k = 0; k < 3; k++ )
+   {
+      start[k + 1] = all.size();
+      all.insert( all.end(), tables[k]->begin(), tables[k]->end() );
+   }
+}
+} // namespace
+
+void Mesh::prepareSweepCells( int minL, int maxL )
+{
+   if ( ctx->hostOnly ) return;
+   std::vector< LevelPlan* > levels;
+   for ( int L = std::max( 1, minL ); L <= std::min( maxL, kSweepCellMaxLevel ); L++ )
+      if ( LevelPlan& P = plan( L ); !P.sweepScratch ) levels.push_back( &P );
+   if ( levels.empty() ) return;
+   // one allocation for all of them: the tables, then the scratch arrays (cleared, since their padding is copied with them;
+   // as part of the tables' copy where that is shorter than a fill's launch)
+   std::vector< int32_t >    all;
+   std::vector< size_t >     starts;
+   size_t                    nScratch = 0;
+   for ( const LevelPlan* P : levels )
+   {
+      size_t start[4];
+      sweepCellTables( T, *P, all, start );
+      starts.insert( starts.end(), start, start + 4 );
+      nScratch += 2 * (size_t) P->total; // FP64; a level's total is a multiple of 64
+   }
    const size_t nTables = ( all.size() + 63 ) / 64 * 64;
    const bool   fill    = nScratch > 50000;
    all.resize( nTables + ( fill ? 0 : nScratch ), 0 );
-   P.sweepTables.alloc( nTables + nScratch );
+   auto buf = std::make_shared< DevBuf< int32_t > >();
+   buf->alloc( nTables + nScratch );
    {
       HYMI_LEGACY_LOCK;
-      if ( fill ) HYMI_HIP( hipMemsetAsync( P.sweepTables.p + nTables, 0, 4 * nScratch, ctx->stream ) );
-      HYMI_HIP( hipMemcpyAsync( P.sweepTables.p, all.data(), 4 * all.size(), hipMemcpyHostToDevice, ctx->stream ) );
+      if ( fill ) HYMI_HIP( hipMemsetAsync( buf->p + nTables, 0, 4 * nScratch, ctx->stream ) );
+      HYMI_HIP( hipMemcpyAsync( buf->p, all.data(), 4 * all.size(), hipMemcpyHostToDevice, ctx->stream ) );
    }
    HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
-   P.cellLocal    = reinterpret_cast< const CellLocal* >( P.sweepTables.p );
-   P.own          = P.sweepTables.p + nCells;
-   P.edgeNbr      = P.own + own.size();
-   P.faceNbr      = P.edgeNbr + edgeNbr.size();
-   P.sweepScratch = reinterpret_cast< double* >( P.sweepTables.p + nTables );
+   size_t scratch = nTables;
+   for ( size_t k = 0; k < levels.size(); k++ )
+   {
+      LevelPlan& P   = *levels[k];
+      P.sweepTables  = buf;
+      P.cellLocal    = reinterpret_cast< const CellLocal* >( buf->p + starts[4 * k] );
+      P.own          = buf->p + starts[4 * k + 1];
+      P.edgeNbr      = buf->p + starts[4 * k + 2];
+      P.faceNbr      = buf->p + starts[4 * k + 3];
+      P.sweepScratch = reinterpret_cast< double* >( buf->p + scratch );
+      scratch += 2 * (size_t) P.total;
+   }
 }
 
 // Work units and scratch arrays of the fused SOR cell phase selected on P (nothing if the passes are selected or
 // they exist already).  Called outside graph capture: by the entry points that sweep and by solver creation.
 void Mesh::prepareCellSor( LevelPlan& P )
 {
-   prepareSweepCell( P );
    if ( P.sorTile == 0 || P.sorUnits ) return;
    const int tile = P.sorTile;
    std::vector< MarchUnit > v;
