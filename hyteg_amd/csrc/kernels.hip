@@ -4921,7 +4921,11 @@ void dotInto( Function& a, Function& b, int level, int flag, double* partials, i
    LevelPlan&  P   = M.plan( level );
    LV          g   = viewOf( P );
    hipStream_t s   = ctx.stream;
-   const int64_t nbLow = 64;
+   // Several right-hand sides: at most 1024 workgroups for the cells and 256 for the rest, fewer where each would have
+   // less than 1024 values.  With 2048 and 64 on every level the lower-dimensional part took 71 us at level 5 (48
+   // macro-tets, now 22) and the final sum, one workgroup over all partials, 65 us (now 39).
+   const int64_t lowValues = ( (int64_t) M.T.nF() * ( P.w - 3 ) * ( P.w - 2 ) / 2 + (int64_t) M.T.nE() * ( P.w - 2 ) + M.T.nV() ) * NR;
+   const int64_t nbLow     = NR == 1 ? 64 : std::min< int64_t >( 256, ( lowValues + 1023 ) / 1024 );
    int64_t       nbC   = 0;
    auto          noTables = []() {
       throw std::runtime_error( "dot: work-unit tables of the level are not prepared (a function of the level "
@@ -4948,7 +4952,7 @@ void dotInto( Function& a, Function& b, int level, int flag, double* partials, i
       if ( !mayBuild && P.segs.find( segLen< NR >() ) == P.segs.end() ) noTables();
       int64_t        nseg   = 0;
       const CellSeg* sg     = M.segments( P, segLen< NR >(), &nseg );
-      const int64_t  nbCell = std::min< int64_t >( kDotBlocks, ( nseg + 3 ) / 4 );
+      const int64_t  nbCell = std::min< int64_t >( 1024, ( nseg + 3 ) / 4 );
       nbC                   = nbCell > 0 ? nbCell : 0;
       if ( ( nbC + nbLow ) * NR > cap ) throw std::logic_error( "dot: partial-sum buffer too small" );
       if ( nbC > 0 )
