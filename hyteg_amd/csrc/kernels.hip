@@ -3033,7 +3033,73 @@ __global__ void kModesCell( LV g, const CellSeg* __restrict__ segs, int64_t nseg
                       fr + 12 * ( (int64_t) frameOff + sg.cell ), 1.0 / ( g.w - 1 ), x, sg.y, sg.z, modes, nModes );
 }
 
-
+// The macro-cell interiors for one right-hand side and at most kModesMax modes.  A point's coordinates are those of its
+// row's start plus x steps along the first edge, so by the addition theorem sin( k pi p ) = s0 cx + c0 sx with (s0, c0)
+// of the row and (sx, cx) of the x step: two fused operations in place of a sine, which bound the direct form (24 sines of
+// some 50 instructions per point and 8 modes: 7.1 ms a function at level 8, 48 macro-tets, 1.8 now).  Workgroup (part, chunk
+// of 64 x, cell): the step factors of its x in LDS, then each wave takes kModesRows rows of a slab at a time, computes
+// their factors lane by lane (LDS) and sums the modes of 64 points per row.  The parts take the slabs in turn.  Against
+// 64-bit values the error is that of the direct form, whose arguments are rounded as often.
+constexpr int kModesMax = 8, kModesRows = 4, kModesThreads = 512;
+template < typename T >
+__global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const int* __restrict__ ctype, int frameOff, int flag,
+                                                                   const double* __restrict__ fr,
+                                                                   const double* __restrict__ modes, int nModes,
+                                                                   T* __restrict__ u )
+{
+   constexpr int CM = 3 * kModesMax, NW = kModesThreads / 64;
+   __shared__ double2 sx[CM][64], sr[NW][kModesRows][CM];
+   __shared__ double  amp[kModesMax];
+   const int cell = (int) blockIdx.z, tid = (int) threadIdx.x, wave = tid >> 6, lane = tid & 63, nc = 3 * nModes;
+   if ( !( ctype[cell] & flag ) ) return;
+   const int     w = g.w, t0 = tet32( w ), x0 = 1 + 64 * (int) blockIdx.y, x = x0 + lane;
+   const double* f = fr + 12 * ( (int64_t) frameOff + cell );
+   const double  h = 1.0 / ( w - 1 ), pi = 3.141592653589793;
+   for ( int k = tid; k < nc * 64; k += kModesThreads )
+   {
+      const int c = k >> 6, d = c % 3;
+      double    s, cs;
+      sincos( modes[4 * ( c / 3 ) + 1 + d] * pi * ( h * ( x0 + ( k & 63 ) ) * f[3 + d] ), &s, &cs );
+      sx[c][k & 63] = make_double2( s, cs );
+   }
+   if ( tid < nModes ) amp[tid] = modes[4 * tid];
+   __syncthreads();
+   T* cu = u + g.offC + (int64_t) cell * g.cS;
+   for ( int z = 1 + (int) blockIdx.x; z <= w - 3 - x0; z += (int) gridDim.x )
+   {
+      const int last = w - 2 - z - x0; // rows 1 .. last hold an interior point at x0
+      for ( int y0 = 1 + wave * kModesRows; y0 <= last; y0 += NW * kModesRows )
+      {
+         for ( int k = lane; k < kModesRows * nc; k += 64 )
+         {
+            const int r = k / nc, c = k % nc, d = c % 3;
+            double    s, cs;
+            sincos( modes[4 * ( c / 3 ) + 1 + d] * pi * ( f[d] + h * ( ( y0 + r ) * f[6 + d] + z * f[9 + d] ) ), &s, &cs );
+            sr[wave][r][c] = make_double2( s, cs );
+         }
+         __builtin_amdgcn_wave_barrier(); // the wave's own writes, read below by its other lanes
+         double acc[kModesRows];
+#pragma unroll
+         for ( int r = 0; r < kModesRows; r++ )
+            acc[r] = 0.0;
+         for ( int m = 0; m < nModes; m++ )
+         {
+            const double2 X = sx[3 * m][lane], Y = sx[3 * m + 1][lane], Z = sx[3 * m + 2][lane];
+            const double  a = amp[m];
+#pragma unroll
+            for ( int r = 0; r < kModesRows; r++ )
+            {
+               const double2 *q = sr[wave][r] + 3 * m;
+               acc[r] += a * ( q[0].x * X.y + q[0].y * X.x ) * ( q[1].x * Y.y + q[1].y * Y.x ) * ( q[2].x * Z.y + q[2].y * Z.x );
+            }
+         }
+#pragma unroll
+         for ( int r = 0; r < kModesRows; r++ )
+            if ( x + y0 + r + z <= w - 2 ) cu[crow32( w, t0, y0 + r, z ) + x] = (T) acc[r];
+         __builtin_amdgcn_wave_barrier();
+      }
+   }
+}
 
 // --------------------------------------------------------------------------------------------------------
 // restriction (coarse owned point <- fine neighbourhood of 2p, weights 1 and 1/2)
@@ -5570,7 +5636,14 @@ void launchInterpolateModes( Function& f, int level, int flag, int nModes, const
       if ( m > 0 && nF > 0 )
          hipLaunchKernelGGL( ( kModesFace< T, NR > ), dim3( blocksFor( m * ( m + 1 ) / 2 * NR, 128 ), nF ), dim3( 128 ), 0, s,
                              g, P.dFaceGeom.p, nV + nE, flag, fr, dModes, nModes, u );
-      if ( nseg > 0 )
+      if ( NR == 1 && nseg > 0 && nModes <= kModesMax )
+      {
+         // slabs in parts, so that about 2048 workgroups share the cells' rows
+         const int chunks = ( P.w - 4 + 63 ) / 64, parts = std::max( 1, std::min( P.w - 4, 2048 / ( nC * chunks ) ) );
+         hipLaunchKernelGGL( ( kModesRowsCell< T > ), dim3( parts, chunks, nC ), dim3( kModesThreads ), 0, s, g,
+                             P.dCellType.p, nV + nE + nF, flag, fr, dModes, nModes, u );
+      }
+      else if ( nseg > 0 )
          hipLaunchKernelGGL( ( kModesCell< T, NR > ), dim3( (unsigned) ( ( nseg + 3 ) / 4 ), NR ), dim3( 256 ), 0, s, g, sg,
                              nseg, P.dCellType.p, nV + nE + nF, flag, fr, dModes, nModes, u );
    };
