@@ -452,7 +452,8 @@ struct hymi_gmg_s
          HYMI_HIP( hipGraphLaunch( it->second.exec, s ) );
    }
 
-   void recurse( Function& x, Function& b, int L )
+   // stale: x's closure copies on level L are not current (W-cycle's second visit after no post-smoothing)
+   void recurse( Function& x, Function& b, int L, bool stale = false )
    {
       const int flag = kInner | kNeumann;
       if ( L == minL )
@@ -463,7 +464,7 @@ struct hymi_gmg_s
       }
       // ghost copies of x are current after a sweep and after the coarse-level reset; only the caller's x on
       // the finest level, x after prolongation and x after the coarse solver need a refresh
-      const bool finest = ( L == maxL_invoked );
+      const bool finest = ( L == maxL_invoked ) || stale;
       // smoothIncrementOnCoarserGrids (GeometricMultigridSolver.hpp:156,218): smoothInc more steps per level
       // below the invoked one
       const int  extra  = smoothInc * ( maxL_invoked - L );
@@ -473,10 +474,12 @@ struct hymi_gmg_s
       // is zeroed (all primitives) in the restriction's launch
       launchResidualRestrict( *A, x, *tmp, b, L, flag, nu1 + extra == 0 && finest, &x );
       recurse( x, b, L - 1 );
+      // the coarse x ends with a sweep, which leaves its copies current, or (no post-smoothing) with a prolongation
+      const bool coarseStale = nu2 + smoothInc * ( maxL_invoked - ( L - 1 ) ) == 0;
       // W-cycle (GeometricMultigridSolver.hpp:201-204): the coarse correction is visited again, from its
       // result and with the same coarse right-hand side
-      if ( wcycle ) recurse( x, b, L - 1 );
-      launchProlongateAdd( x, L - 1, flag, L - 1 == minL );
+      if ( wcycle ) recurse( x, b, L - 1, coarseStale );
+      launchProlongateAdd( x, L - 1, flag, L - 1 == minL || coarseStale );
       smooth( x, b, L, flag, nu2 + extra, true );
    }
 
