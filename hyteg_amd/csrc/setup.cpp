@@ -1003,7 +1003,12 @@ void Mesh::prepareSweepCells( int minL, int maxL )
    if ( ctx->hostOnly ) return;
    std::vector< LevelPlan* > levels;
    for ( int L = std::max( 1, minL ); L <= std::min( maxL, kSweepCellMaxLevel ); L++ )
-      if ( LevelPlan& P = plan( L ); !P.sweepScratch ) levels.push_back( &P );
+   {
+      LevelPlan&    P  = plan( L );
+      const int64_t w  = P.w, most = int64_t( 1 ) << 30; // the kernels index elements and tables in 32 bits
+      const bool    ok = P.total < most && T.nF() * ( w - 3 ) * ( w - 2 ) / 2 * 8 < most && (int64_t) P.hEdgeTerms.size() * ( w - 2 ) < most;
+      if ( ok && !P.sweepScratch ) levels.push_back( &P );
+   }
    if ( levels.empty() ) return;
    // one allocation for all of them: the tables, then the scratch arrays (cleared, since their padding is copied with them;
    // as part of the tables' copy where that is shorter than a fill's launch)
