@@ -561,14 +561,9 @@ const CellSeg* Mesh::segments( LevelPlan& P, int len, int64_t* count )
 }
 
 // Default launch schedule of the macro-cell kernels, from a sweep of kind x rows x waves x block on MI355X
-// (48 macro-cells, levels 5-7, FP64 apply and SOR colour pass): flat slab windows (they keep ~90 % of the
-// lanes busy where row windows keep ~50 %); two windows per unit from level 6 up, one below, where more
-// waves are needed to fill the GPU.  The column march (kind 3) is faster from level 5 up (level 7 FP64
-// apply 81 us against 105 us) but is selected explicitly, not by default: a serving run of many concurrent
-// hierarchies with it as the default ended in a GPU fault whose cause has not been found.
-// Measured per-level defaults (MI355X, FP64 and FP32 alike): the column march from level 5 up, 16 slabs per
-// unit and 4 waves per workgroup from level 7, 8 and 4 on level 6, 4 and 2 on level 5, loads one slab ahead;
-// flat slab windows below, where a cell is too thin for columns to pay.
+// (48 macro-cells, FP64 and FP32 alike): the column march from level 5 up (level 7 FP64 apply 81 us against 105 us
+// of flat slab windows), 16 slabs per unit and 4 waves per workgroup from level 7, 8 and 4 on level 6, 4 and 2 on
+// level 5, loads one slab ahead; flat slab windows below, where a cell is too thin for columns to pay.
 MarchSchedule defaultSchedule( int level )
 {
    MarchSchedule S;

@@ -242,7 +242,8 @@ int hymi_time_kernel( hymi_operator op, hymi_gmg gmg, hymi_function x, hymi_func
  * marches a wave's 64 (x, y) positions up through `rows` slabs with loads issued `block` slabs ahead (block
  * 1, 2 or 4); waves per workgroup 1, 2 or 4; rows 1..4096.  kind -1 and zeros select the level default (the
  * column march with 16 / 8 / 4 slabs per unit on levels >= 7 / 6 / 5, flat windows below).  A schedule the level
- * cannot run (a kind-2 band too large for LDS) is refused.  Results do not depend on the schedule.  Setting a
+ * cannot run (a kind-2 band too large for LDS) is refused.  Results do not depend on the schedule; the apply
+ * and residual of one right-hand side on levels 1 to 4 run without one (a workgroup per macro-cell).  Setting a
  * schedule waits for the context stream; V-cycle graphs captured before it are captured again on their
  * next replay.  out = {rows, waves, block, kind}. */
 int hymi_mesh_set_schedule( hymi_mesh mesh, int level, int kind, int rows, int waves, int block );
