@@ -3380,21 +3380,43 @@ __device__ __forceinline__ void kRestrictFace_b( const Blk& B, LV gc, LV gf, con
    T acc = UF( i - 1, j ) + UF( i + 1, j ) + UF( i, j + 1 ) + UF( i, j - 1 ) + UF( i - 1, j + 1 ) + UF( i + 1, j - 1 );
    const T centre = UF( i, j );
 #undef UF
-   for ( int s = 0; s < G.nSides; s++ )
+   // all eight places first, then their owners, then the values: two trips to memory instead of one per term
+   int64_t o[2][4];
+#pragma unroll
+   for ( int s = 0; s < 2; s++ )
    {
-      const FaceCellMap& M  = G.side[s];
+      const int          sc = min( s, G.nSides - 1 );
+      const FaceCellMap& M  = G.side[sc];
       const int64_t      cb = gf.offC + (int64_t) M.cell * gf.cS;
 #pragma unroll
       for ( int q = 0; q < 4; q++ )
       {
-         const int col = i + G.offCol[s][q], row = j + G.offRow[s][q];
+         const int col = i + G.offCol[sc][q], row = j + G.offRow[sc][q];
          const int x   = M.base[0] + col * M.a[0] + row * M.b[0] + M.o[0];
          const int y   = M.base[1] + col * M.a[1] + row * M.b[1] + M.o[1];
          const int z   = M.base[2] + col * M.a[2] + row * M.b[2] + M.o[2];
-         const int64_t o = cb + cellRel( w, tet32( w ), x, y, z );
-         acc += uf[( own ? own[o] : o ) * NR + r];
+         o[s][q]       = cb + cellRel( w, tet32( w ), x, y, z );
       }
    }
+   if ( own )
+   {
+#pragma unroll
+      for ( int s = 0; s < 2; s++ )
+#pragma unroll
+         for ( int q = 0; q < 4; q++ )
+            o[s][q] = own[o[s][q]];
+   }
+   T v[2][4];
+#pragma unroll
+   for ( int s = 0; s < 2; s++ )
+#pragma unroll
+      for ( int q = 0; q < 4; q++ )
+         v[s][q] = uf[o[s][q] * NR + r];
+#pragma unroll
+   for ( int s = 0; s < 2; s++ )
+#pragma unroll
+      for ( int q = 0; q < 4; q++ )
+         if ( s < G.nSides ) acc += v[s][q];
    const int64_t co = gc.offF + (int64_t) G.face * gc.fS;
    uc[( co + fidx( gc.w, I, J ) ) * NR + r] = centre + T( 0.5 ) * acc;
 }
@@ -3416,16 +3438,25 @@ __device__ __forceinline__ void kRestrictEdge_b( const Blk& B, LV gc, LV gf, con
    const int t0 = tet32( gf.w ), n = G.nTerms;
    for ( int k0 = 0; k0 < n; k0 += kTermBatch )
    {
-      T     v[kTermBatch];
-      float wr[kTermBatch];
+      T       v[kTermBatch];
+      float   wr[kTermBatch];
+      int64_t o[kTermBatch];
 #pragma unroll
       for ( int q = 0; q < kTermBatch; q++ )
       {
          const EdgeTerm& e = terms[G.termOff + min( k0 + q, n - 1 )];
          wr[q]             = e.wr;
-         const int64_t o   = edgeTermIndex< T, NR >( gf, e, x, t0 );
-         v[q]              = uf[( own ? own[o] : o ) * NR + r];
+         o[q]              = edgeTermIndex< T, NR >( gf, e, x, t0 );
       }
+      if ( own )
+      {
+#pragma unroll
+         for ( int q = 0; q < kTermBatch; q++ )
+            o[q] = own[o[q]];
+      }
+#pragma unroll
+      for ( int q = 0; q < kTermBatch; q++ )
+         v[q] = uf[o[q] * NR + r];
 #pragma unroll
       for ( int q = 0; q < kTermBatch; q++ )
          if ( k0 + q < n && wr[q] != 0.0f ) acc += T( wr[q] ) * v[q];
