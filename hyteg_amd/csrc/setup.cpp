@@ -995,7 +995,8 @@ void sweepCellTables( const Topology& T, const LevelPlan& P, std::vector< int32_
 
 void Mesh::prepareSweepCells( int minL, int maxL )
 {
-   if ( ctx->hostOnly ) return;
+   // the one-launch kernels run a workgroup per macro-cell: a vertex of no cell would be left out by all of them
+   if ( ctx->hostOnly || T.loneVertices ) return;
    std::vector< LevelPlan* > levels;
    for ( int L = std::max( 1, minL ); L <= std::min( maxL, kSweepCellMaxLevel ); L++ )
    {

@@ -140,6 +140,7 @@ Topology Topology::fromCells( const std::vector< std::array< double, 3 > >& coor
    }
    for ( auto& l : T.eFaces )
       std::sort( l.begin(), l.end() );
+   T.loneVertices = std::any_of( T.vCells.begin(), T.vCells.end(), []( const auto& l ) { return l.empty(); } );
 
    T.vType.assign( T.nV(), kInner );
    T.eType.assign( T.nE(), kInner );

@@ -43,6 +43,7 @@ struct Topology
    std::vector< std::array< int, 12 > >   cemap; // [localEdge*2 + edgeLocalVertex] = cellLocalVertex
    std::vector< std::vector< int > >      vEdges, vFaces, vCells, eFaces, eCells, fCells;
    std::vector< int >                     vType, eType, fType, cType;
+   bool                                   loneVertices = false; // some vertex belongs to no cell (an unused mesh node)
 
    int nV() const { return (int) vx.size(); }
    int nE() const { return (int) ev.size(); }
