@@ -122,9 +122,9 @@ struct LevelPlan
    DevBuf< int64_t >    dVertexSnap;
    DevBuf< int32_t >    dEdgeEnds;
    DevBuf< int32_t >    dCellType;
-   // one-launch sweeps (levels 1 .. kSweepCellMaxLevel; Mesh::prepareSweepCells): per element the element of the primitive
-   // that owns the value; per edge term and edge point, and per face point and off-plane neighbour (-1: none), the element
-   // the term reads, at its owner; the cells; the array that sweeps go to and from (FP64-sized)
+   // one-launch sweeps (levels 1 .. kSweepCellMaxLevel; Mesh::prepareSweepCells): per macro-cell element the element of the
+   // primitive that owns the value; per edge term and edge point, and per face point and off-plane neighbour (-1: none), the
+   // element the term reads, at its owner; the cells; the array that sweeps go to and from (FP64-sized)
    // (pointers into sweepTables, which the levels prepared together share)
    std::shared_ptr< DevBuf< int32_t > > sweepTables;
    const int32_t *   own = nullptr, *edgeNbr = nullptr, *faceNbr = nullptr;

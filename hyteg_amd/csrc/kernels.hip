@@ -354,6 +354,21 @@ __device__ __forceinline__ int64_t refreshEdgeSrc( const LV& g, const V2E* __res
    return g.offE + (int64_t) edge * g.eS + t;
 }
 
+// the edge of a face through its boundary point (i, j) and the point's place t on it (a corner lies on two: either edge
+// leads to the same owner); false for an interior point
+__device__ __forceinline__ bool faceEdgeThrough( int w, const E2F* __restrict__ e2f, int face, int i, int j, int& edge, int& t )
+{
+   if ( i == 0 || j == 0 || i + j == w - 1 )
+      for ( int le = 0; le < 3; le++ )
+      {
+         const E2F m = e2f[3 * face + le];
+         t           = m.inc[0] != 0 ? ( i - m.base[0] ) * m.inc[0] : ( j - m.base[1] ) * m.inc[1];
+         edge        = m.edge;
+         if ( t >= 0 && t <= w - 1 && m.base[0] + t * m.inc[0] == i && m.base[1] + t * m.inc[1] == j ) return true;
+      }
+   return false;
+}
+
 template < typename T, int NR >
 __global__ __launch_bounds__( 256 ) void kRefresh( LV g, const V2E* __restrict__ v2e, int nE, const E2F* __restrict__ e2f,
                                                   int nF, const F2C* __restrict__ f2c, int nPairs, int mask, int nA,
@@ -396,14 +411,9 @@ __global__ __launch_bounds__( 256 ) void kRefresh( LV g, const V2E* __restrict__
       return crow32( w, t0, y, z ) + x;
    };
    auto source = [&]( int i, int j, int p ) -> int64_t { // where face point (i, j), index p, is read
-      if ( fromEdge && ( i == 0 || j == 0 || i + j == w - 1 ) )
-         for ( int le = 0; le < 3; le++ ) // the face edge through (i, j); corners lie on two, same owner value
-         {
-            const E2F me = e2f[3 * m.face + le];
-            const int te = me.inc[0] != 0 ? ( i - me.base[0] ) * me.inc[0] : ( j - me.base[1] ) * me.inc[1];
-            if ( te >= 0 && te <= w - 1 && me.base[0] + te * me.inc[0] == i && me.base[1] + te * me.inc[1] == j )
-               return refreshEdgeSrc< T, NR >( g, v2e, me.edge, te, fromVertex );
-         }
+      int edge, t;
+      if ( fromEdge && faceEdgeThrough( w, e2f, m.face, i, j, edge, t ) )
+         return refreshEdgeSrc< T, NR >( g, v2e, edge, t, fromVertex );
       return fo + p; // face interior, or the face's own copy of its boundary
    };
    if ( band ) // only the points within distance 1 of the face's boundary (one right-hand side, see kF2CBand)
@@ -2419,6 +2429,152 @@ __device__ __forceinline__ int pick( const int32_t ( &v )[N], int k )
    return r;
 }
 constexpr int kSweepThreads = 1024;
+
+// The tables, built where they are read: with loops over all elements on the host and an upload, the first call on a mesh
+// took 0.2 to 200 ms (6 to 10368 macro-tets, level 4).  Workgroups: the elements of all macro-cells, then the edges (one
+// wave each), the face points, the cells, and the clearing of the scratch array.
+struct SweepTableIn
+{
+   const V2E*          v2e;
+   const E2F*          e2f;
+   const F2C*          f2c;
+   const CellFaceRead* cfr;
+   const VertexGeom*   vg;
+   const int64_t*      vterms;
+   const EdgeGeom*     eg;
+   const EdgeTerm*     eterms;
+   const FaceGeom*     fg;
+   const int*          ctype;
+   int                 nC, nE, nF;
+};
+struct SweepTableOut
+{
+   CellLocal* cells;
+   int32_t *  own, *edgeNbr, *faceNbr;
+   uint4*     scratch;
+   int64_t    nScratch; // in uint4
+};
+struct SweepTableGrid
+{
+   int own, edges, faces, cells, scratch;
+};
+__device__ __forceinline__ int ownerOnFace( const LV& g, const SweepTableIn& S, int face, int i, int j )
+{
+   int edge, t;
+   return (int) ( faceEdgeThrough( g.w, S.e2f, face, i, j, edge, t ) ?
+                      refreshEdgeSrc< float, 1 >( g, S.v2e, edge, t, true ) :
+                      g.offF + (int64_t) face * g.fS + fidx( g.w, i, j ) );
+}
+__device__ __forceinline__ int ownerInCell( const LV& g, const SweepTableIn& S, int cell, int x, int y, int z )
+{
+   const int q = z == 0 ? 0 : y == 0 ? 1 : x == 0 ? 2 : x + y + z == g.w - 1 ? 3 : -1;
+   if ( q < 0 ) return (int) ( g.offC + (int64_t) cell * g.cS ) + cellRel( g.w, tet32( g.w ), x, y, z );
+   const CellFaceRead& R = S.cfr[cell];
+   const int *         c = R.c[q], u = q == 2 ? y : x, v = q == 0 || q == 3 ? y : z;
+   return ownerOnFace( g, S, R.face[q], c[0] + c[1] * u + c[2] * v, c[3] + c[4] * u + c[5] * v );
+}
+__global__ __launch_bounds__( 256 ) void kSweepTables( LV g, SweepTableIn S, SweepTableOut D, SweepTableGrid N )
+{
+   const int w = g.w, t0 = tet32( w ), np = w - 2, m = w - 3, nf = m * ( m + 1 ) / 2, tid = (int) threadIdx.x;
+   int       blk = (int) blockIdx.x;
+   if ( blk < N.own )
+   {
+      const int k = blk * 256 + tid, cell = k / t0;
+      if ( cell >= S.nC ) return;
+      const int p = k - cell * t0;
+      int       z = 0, x, y; // the slab of place p: the last that starts at or before it
+      while ( t0 - tet32( w - z - 1 ) <= p )
+         z++;
+      triPos( w - z, p - ( t0 - tet32( w - z ) ), x, y );
+      D.own[(int64_t) cell * g.cS + p] = ownerInCell( g, S, cell, x, y, z );
+      return;
+   }
+   blk -= N.own;
+   if ( blk < N.edges )
+   {
+      const int e = 4 * blk + ( tid >> 6 );
+      if ( e >= S.nE ) return;
+      const EdgeGeom G = S.eg[e];
+      for ( int k = tid & 63; k < np * G.nTerms; k += 64 )
+      {
+         const EdgeTerm& t = S.eterms[G.termOff + k % G.nTerms];
+         const int       x = 1 + k / G.nTerms;
+         const int       q[3] = { t.base[0] + x * t.inc[0], t.base[1] + x * t.inc[1], t.base[2] + x * t.inc[2] };
+         D.edgeNbr[G.termOff * np + k] =
+             t.kind == 0 ? ownerOnFace( g, S, t.prim, q[0], q[1] ) : ownerInCell( g, S, t.prim, q[0], q[1], q[2] );
+      }
+      return;
+   }
+   blk -= N.edges;
+   if ( blk < N.faces )
+   {
+      const int k = blk * 256 + tid, q = k >> 3, face = nf > 0 ? q / nf : S.nF, s = k >> 2 & 1;
+      if ( face >= S.nF ) return;
+      const FaceGeom& G = S.fg[face];
+      int             i, j, owner = -1;
+      triPos( m, q - face * nf, i, j );
+      if ( s < G.nSides )
+      {
+         const FaceCellMap& M = G.side[s];
+         const int          c = i + 1 + G.offCol[s][k & 3], r = j + 1 + G.offRow[s][k & 3];
+         owner = ownerInCell( g, S, M.cell, M.base[0] + c * M.a[0] + r * M.b[0] + M.o[0],
+                              M.base[1] + c * M.a[1] + r * M.b[1] + M.o[1], M.base[2] + c * M.a[2] + r * M.b[2] + M.o[2] );
+      }
+      D.faceNbr[k] = owner;
+      return;
+   }
+   blk -= N.faces;
+   if ( blk < N.cells )
+   {
+      const int cell = blk * 256 + tid;
+      if ( cell >= S.nC ) return;
+      CellLocal& C         = D.cells[cell];
+      int        write     = 0, vert[4];
+      auto       firstCell = [&]( int edge ) { // of an edge's neighbour cells, whose terms follow those of its faces
+         int k = S.eg[edge].termOff;
+         while ( S.eterms[k].kind == 0 )
+            k++;
+         return S.eterms[k].prim;
+      };
+#pragma unroll
+      for ( int k = 0; k < 4; k++ )
+      {
+         const int          v = ownerInCell( g, S, cell, k == 1 ? w - 1 : 0, k == 2 ? w - 1 : 0, k == 3 ? w - 1 : 0 );
+         const VertexGeom   V = S.vg[v];
+         const F2C&         f = S.f2c[4 * cell + k];
+         const FaceGeom&    F = S.fg[f.face];
+         // a vertex is written by the first cell of its first edge
+         write |= ( firstCell( (int) ( ( S.vterms[V.termOff] - g.offE ) / g.eS ) ) == cell ? 1 : 0 ) << k;
+         write |= ( F.side[0].cell == cell ? 1 : 0 ) << ( 10 + k );
+         vert[k] = C.vert[k] = v;
+         C.vTermOff[k] = V.termOff, C.vTerms[k] = V.nTerms, C.vType[k] = V.type;
+         C.face[k] = f.face, C.fType[k] = F.type, C.fSides[k] = F.nSides;
+#pragma unroll
+         for ( int d = 0; d < 3; d++ )
+            C.fMap[9 * k + d] = f.m.base[d], C.fMap[9 * k + 3 + d] = f.m.a[d], C.fMap[9 * k + 6 + d] = f.m.b[d];
+      }
+      constexpr int from[6] = { 0, 0, 1, 0, 1, 2 }, to[6] = { 1, 2, 2, 3, 3, 3 };
+#pragma unroll
+      for ( int k = 0; k < 6; k++ )
+      {
+         // the edge through the point one step from one corner towards the other
+         auto      at   = [&]( int d ) { return to[k] == d ? 1 : from[k] == d ? w - 2 : 0; };
+         const int edge = (int) ( ( ownerInCell( g, S, cell, at( 1 ), at( 2 ), at( 3 ) ) - g.offE ) / g.eS );
+         const EdgeGeom G = S.eg[edge];
+         C.edge[k] = edge;
+         C.ends[k] = S.v2e[edge].v0 == vert[from[k]] ? from[k] | to[k] << 2 : to[k] | from[k] << 2;
+         C.eTermOff[k] = G.termOff, C.eTerms[k] = G.nTerms, C.eType[k] = G.type;
+         write |= ( firstCell( edge ) == cell ? 1 : 0 ) << ( 4 + k );
+      }
+      C.type  = S.ctype[cell];
+      C.write = write;
+      return;
+   }
+   blk -= N.cells;
+   for ( int64_t k = (int64_t) blk * 256 + tid; k < D.nScratch; k += (int64_t) N.scratch * 256 )
+      D.scratch[k] = make_uint4( 0, 0, 0, 0 );
+}
+
 template < typename T, int LMAX >
 __global__ __launch_bounds__( kSweepThreads ) void kSweepCell( LV g, SweepCellTables< T > S, ColourStarts cs, int flag,
                                                                const T* __restrict__ uo, T* __restrict__ un,
@@ -2453,7 +2609,7 @@ __global__ __launch_bounds__( kSweepThreads ) void kSweepCell( LV g, SweepCellTa
       return k < 0 ? k + kSweepThreads : k;
    };
    for ( int k = share( t0 ); k < t0; k += nt )
-      V[k] = uo[S.own[co + k]];
+      V[k] = uo[S.own[(int64_t) cell * g.cS + k]];
    // the cell's points: at most one of each colour per thread, place, row geometry and right-hand side
    int o[4], rowY[4], rowW[4];
    T   bv[4];
@@ -2653,7 +2809,7 @@ __global__ __launch_bounds__( kApplyCellThreads ) void kApplyCell( LV g, SweepCe
    const int64_t      co = g.offC + (int64_t) cell * g.cS;
    auto put = [&]( int64_t o, T acc ) { y[o] = MODE == kReplace ? acc : MODE == kAdd ? y[o] + acc : b[o] - acc; };
    for ( int k = tid; k < t0; k += nt )
-      V[k] = u[S.own[co + k]];
+      V[k] = u[S.own[(int64_t) cell * g.cS + k]];
    __syncthreads();
    if ( C.type & flag )
    {
@@ -5276,6 +5432,20 @@ bool launchCgVertexOnly( Operator& op, Function& x, const Function& b, int level
                           Wt.vertex32.p, flag, (float*) x.ptr( level ), (const float*) b.ptr( level ), maxIter,
                           tol * tol );
    return true;
+}
+
+void launchSweepTables( Mesh& M, LevelPlan& P, CellLocal* cells, int32_t* own, int32_t* edgeNbr, int32_t* faceNbr,
+                        double* scratch )
+{
+   const int            w = P.w, t0 = (int) tetSize( w ), nf = ( w - 3 ) * ( w - 2 ) / 2;
+   const SweepTableIn   S{ P.dV2E.p, P.dE2F.p, P.dF2C.p, P.dCellFaceRead.p, P.dVertexGeom.p, P.dVertexTerms.p, P.dEdgeGeom.p,
+                           P.dEdgeTerms.p, P.dFaceGeom.p, P.dCellType.p, M.T.nC(), M.T.nE(), M.T.nF() };
+   const SweepTableOut  D{ cells, own, edgeNbr, faceNbr, (uint4*) scratch, P.total / 2 };
+   const SweepTableGrid N{ (int) blocksFor( (int64_t) M.T.nC() * t0, 256 ), ( M.T.nE() + 3 ) / 4,
+                           (int) blocksFor( (int64_t) M.T.nF() * nf * 8, 256 ), ( M.T.nC() + 255 ) / 256,
+                           (int) std::min< int64_t >( 1024, blocksFor( D.nScratch, 256 ) ) };
+   hipLaunchKernelGGL( kSweepTables, dim3( N.own + N.edges + N.faces + N.cells + N.scratch ), dim3( 256 ), 0, M.ctx->stream,
+                       viewOf( P ), S, D, N );
 }
 
 void launchRefresh( Function& f, int level, int mask ) { dispatch< RefreshF >( f.prec, f.nrhs, f, level, mask ); }

@@ -28,6 +28,9 @@ void launchSor( Operator& op, Function& x, const Function& b, double omega, int 
 // `count` SOR sweeps (refreshFirst applies to the first)
 void launchSorSweeps( Operator& op, Function& x, const Function& b, double omega, int level, int flag, int count,
                       bool refreshFirst = true );
+// the tables of the one-launch kernels of a small level (LevelPlan::own and the following) and the cleared scratch array
+void launchSweepTables( Mesh& M, LevelPlan& P, CellLocal* cells, int32_t* own, int32_t* edgeNbr, int32_t* faceNbr,
+                        double* scratch );
 // coarse level of dst <- restriction of the fine level of f (dst may be f)
 void launchRestrict( Function& f, Function& dst, int srcLevel, int flag );
 // r = b - A x on `level`, restricted into b on level - 1 (flag DoFs); r is scratch afterwards (of its macro-cell

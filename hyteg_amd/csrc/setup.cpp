@@ -8,11 +8,11 @@
 // point (1,1) (P1Operator.hpp:2031-2042), edge weights at the edge point 1 (P1Elements.hpp:829-964) and
 // vertex weights from the single corner micro-tetrahedron of every neighbour cell (P1Elements.hpp:601-683).
 #include <algorithm>
-#include <cstring>
 #include <cmath>
 #include <stdexcept>
 
 #include "internal.hpp"
+#include "kernels.hpp"
 
 namespace hymi {
 
@@ -902,97 +902,6 @@ void Mesh::selectCellSor( int level, int tile, int precisions )
 
 bool Mesh::cellSorReady( const LevelPlan& P ) const { return P.sorTile == 0 || ctx->hostOnly || P.sorUnits != nullptr; }
 
-namespace {
-// the tables of one level, in the order cells, own, edgeNbr, faceNbr; start: where the last three begin
-void sweepCellTables( const Topology& T, const LevelPlan& P, std::vector< int32_t >& all, size_t ( &start )[4] )
-{
-   const int              w = P.w, m = w - 3, nf = m * ( m + 1 ) / 2;
-   std::vector< int32_t > own( (size_t) P.total );
-   for ( int64_t k = 0; k < P.total; k++ )
-      own[k] = (int32_t) k;
-   for ( int e = 0; e < T.nE(); e++ )
-   {
-      own[P.edgeOff( e )]         = T.ev[e][0];
-      own[P.edgeOff( e ) + w - 1] = T.ev[e][1];
-   }
-   for ( int f = 0; f < T.nF(); f++ )
-      for ( int le = 0; le < 3; le++ )
-         for ( int x = 0; x < w; x++ )
-         {
-            int p[2];
-            faceEdgePoint( T, f, le, w, x, 0, p );
-            own[P.faceOff( f ) + faceIndex( w, p[0], p[1] )] = own[P.edgeOff( T.fe[f][le] ) + x];
-         }
-   // cell-relative index from a table of the slabs' starts (this runs once per table entry)
-   std::vector< int > slab( w + 1 );
-   for ( int z = 0; z <= w; z++ )
-      slab[z] = (int) cellIndex( w, 0, 0, z );
-   auto inCellAt = [&]( int x, int y, int z ) { return slab[z] + y * ( w - z + 1 ) - y * ( y + 1 ) / 2 + x; };
-   auto cellAt   = [&]( const FaceCellMap& M, int i, int j, int layer ) {
-      return inCellAt( M.base[0] + i * M.a[0] + j * M.b[0] + layer * M.o[0], M.base[1] + i * M.a[1] + j * M.b[1] + layer * M.o[1],
-                         M.base[2] + i * M.a[2] + j * M.b[2] + layer * M.o[2] );
-   };
-   std::vector< CellLocal > cells( T.nC() );
-   for ( int c = 0; c < T.nC(); c++ )
-   {
-      CellLocal& C = cells[c];
-      C.type       = T.cType[c];
-      for ( int lf = 0; lf < 4; lf++ )
-      {
-         const int         f = T.cf[c][lf];
-         const FaceCellMap M = numericMap( T, c, lf, w );
-         for ( int j = 0; j < w; j++ )
-            for ( int i = 0; i + j < w; i++ )
-               own[P.cellOff( c ) + cellAt( M, i, j, 0 )] = own[P.faceOff( f ) + faceIndex( w, i, j )];
-         const VertexGeom& v = P.hVertexGeom[T.cv[c][lf]];
-         C.vert[lf]          = T.cv[c][lf];
-         C.vTermOff[lf] = v.termOff, C.vTerms[lf] = v.nTerms, C.vType[lf] = v.type;
-         C.face[lf] = f, C.fType[lf] = T.fType[f], C.fSides[lf] = P.hFaceGeom[f].nSides;
-         for ( int d = 0; d < 3; d++ )
-            C.fMap[9 * lf + d] = M.base[d], C.fMap[9 * lf + 3 + d] = M.a[d], C.fMap[9 * lf + 6 + d] = M.b[d];
-         C.write |= ( T.vCells[T.cv[c][lf]][0] == c ? 1 : 0 ) << lf | ( T.fCells[f][0] == c ? 1 : 0 ) << ( 10 + lf );
-      }
-      for ( int le = 0; le < 6; le++ )
-      {
-         const EdgeGeom& e = P.hEdgeGeom[T.ce[c][le]];
-         C.edge[le]        = T.ce[c][le];
-         C.eTermOff[le] = e.termOff, C.eTerms[le] = e.nTerms, C.eType[le] = e.type;
-         C.ends[le] = T.cemap[c][2 * le] | T.cemap[c][2 * le + 1] << 2;
-         C.write |= ( T.eCells[T.ce[c][le]][0] == c ? 1 : 0 ) << ( 4 + le );
-      }
-   }
-   std::vector< int32_t > edgeNbr, faceNbr;
-   edgeNbr.reserve( P.hEdgeTerms.size() * (size_t) ( w - 2 ) );
-   for ( const EdgeGeom& G : P.hEdgeGeom )
-      for ( int x = 1; x <= w - 2; x++ )
-         for ( int k = 0; k < G.nTerms; k++ )
-         {
-            const EdgeTerm& t = P.hEdgeTerms[G.termOff + k];
-            const int       q[3] = { t.base[0] + x * t.inc[0], t.base[1] + x * t.inc[1], t.base[2] + x * t.inc[2] };
-            edgeNbr.push_back( own[t.kind == 0 ? P.faceOff( t.prim ) + faceIndex( w, q[0], q[1] )
-                                               : P.cellOff( t.prim ) + inCellAt( q[0], q[1], q[2] )] );
-         }
-   faceNbr.reserve( (size_t) T.nF() * nf * 8 );
-   for ( const FaceGeom& G : P.hFaceGeom )
-      for ( int j = 1; j <= m; j++ )
-         for ( int i = 1; i + j <= w - 2; i++ )
-            for ( int sd = 0; sd < 2; sd++ )
-               for ( int k = 0; k < 4; k++ )
-                  faceNbr.push_back( sd < G.nSides ? own[P.cellOff( G.side[sd].cell ) + cellAt( G.side[sd], i + G.offCol[sd][k],
-                                                                                                j + G.offRow[sd][k], 1 )]
-                                                   : -1 );
-   start[0] = all.size();
-   all.resize( start[0] + cells.size() * ( sizeof( CellLocal ) / 4 ) );
-   std::memcpy( all.data() + start[0], cells.data(), cells.size() * sizeof( CellLocal ) );
-   const std::vector< int32_t >* tables[3] = { &own, &edgeNbr, &faceNbr };
-   for ( int k = 0; k < 3; k++ )
-   {
-      start[k + 1] = all.size();
-      all.insert( all.end(), tables[k]->begin(), tables[k]->end() );
-   }
-}
-} // namespace
-
 void Mesh::prepareSweepCells( int minL, int maxL )
 {
    // the one-launch kernels run a workgroup per macro-cell: a vertex of no cell would be left out by all of them
@@ -1006,40 +915,50 @@ void Mesh::prepareSweepCells( int minL, int maxL )
       if ( ok && !P.sweepScratch ) levels.push_back( &P );
    }
    if ( levels.empty() ) return;
-   // one allocation for all of them: the tables, then the scratch arrays (cleared, since their padding is copied with them;
-   // as part of the tables' copy where that is shorter than a fill's launch)
-   std::vector< int32_t >    all;
-   std::vector< size_t >     starts;
-   size_t                    nScratch = 0;
+   // one allocation for all of them, filled on the device (in 32-bit words; every table starts on 256 bytes)
+   auto   padded = []( int64_t words ) { return (size_t) ( words + 63 ) / 64 * 64; };
+   auto   sizes  = [&]( const LevelPlan& P, size_t ( &n )[5] ) {
+      const int64_t w = P.w;
+      n[0] = padded( (int64_t) T.nC() * ( sizeof( CellLocal ) / 4 ) );
+      n[1] = padded( (int64_t) T.nC() * P.cStride );
+      n[2] = padded( (int64_t) P.hEdgeTerms.size() * ( w - 2 ) );
+      n[3] = padded( (int64_t) T.nF() * ( ( w - 3 ) * ( w - 2 ) / 2 ) * 8 );
+      n[4] = padded( 2 * P.total ); // the scratch array, FP64
+   };
+   size_t words = 0;
    for ( const LevelPlan* P : levels )
    {
-      size_t start[4];
-      sweepCellTables( T, *P, all, start );
-      starts.insert( starts.end(), start, start + 4 );
-      nScratch += 2 * (size_t) P->total; // FP64; a level's total is a multiple of 64
+      size_t n[5];
+      sizes( *P, n );
+      words += n[0] + n[1] + n[2] + n[3] + n[4];
    }
-   const size_t nTables = ( all.size() + 63 ) / 64 * 64;
-   const bool   fill    = nScratch > 50000;
-   all.resize( nTables + ( fill ? 0 : nScratch ), 0 );
    auto buf = std::make_shared< DevBuf< int32_t > >();
-   buf->alloc( nTables + nScratch );
+   try
    {
-      HYMI_LEGACY_LOCK;
-      if ( fill ) HYMI_HIP( hipMemsetAsync( buf->p + nTables, 0, 4 * nScratch, ctx->stream ) );
-      HYMI_HIP( hipMemcpyAsync( buf->p, all.data(), 4 * all.size(), hipMemcpyHostToDevice, ctx->stream ) );
+      buf->alloc( words );
+   } catch ( const HipError& e )
+   {
+      if ( e.code != hipErrorOutOfMemory ) throw;
+      (void) hipGetLastError();
+      return; // no room: the separate launches need no tables
    }
-   HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
-   size_t scratch = nTables;
-   for ( size_t k = 0; k < levels.size(); k++ )
+   int32_t* at = buf->p;
+   for ( LevelPlan* P : levels )
    {
-      LevelPlan& P   = *levels[k];
-      P.sweepTables  = buf;
-      P.cellLocal    = reinterpret_cast< const CellLocal* >( buf->p + starts[4 * k] );
-      P.own          = buf->p + starts[4 * k + 1];
-      P.edgeNbr      = buf->p + starts[4 * k + 2];
-      P.faceNbr      = buf->p + starts[4 * k + 3];
-      P.sweepScratch = reinterpret_cast< double* >( buf->p + scratch );
-      scratch += 2 * (size_t) P.total;
+      size_t n[5];
+      sizes( *P, n );
+      int32_t* part[5];
+      for ( int k = 0; k < 5; k++ )
+         part[k] = at, at += n[k];
+      launchSweepTables( *this, *P, reinterpret_cast< CellLocal* >( part[0] ), part[1], part[2], part[3],
+                         reinterpret_cast< double* >( part[4] ) );
+      HYMI_HIP( hipGetLastError() );
+      P->sweepTables  = buf;
+      P->cellLocal    = reinterpret_cast< const CellLocal* >( part[0] );
+      P->own          = part[1];
+      P->edgeNbr      = part[2];
+      P->faceNbr      = part[3];
+      P->sweepScratch = reinterpret_cast< double* >( part[4] );
    }
 }
 
