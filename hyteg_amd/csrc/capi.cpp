@@ -1318,7 +1318,7 @@ int hymi_smooth_sor( hymi_operator op, hymi_function x, hymi_function b, double 
       require( x != b, "x and b must differ" );
       require( x->f.prec == b->f.prec && x->f.nrhs == b->f.nrhs, "functions must share precision and nrhs" );
       op->op.mesh->prepareCellSor( op->op.mesh->plan( level ) );
-      prepareSmallLevel( x->f, level );
+      if ( sweepsInOneLaunch( level, x->f.mesh->T.nC() ) ) prepareSmallLevel( x->f, level );
       launchSorSweeps( op->op, x->f, b->f, omega, level, flag, 1 );
    } );
 }

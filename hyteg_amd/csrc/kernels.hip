@@ -4681,7 +4681,7 @@ void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, in
    T*          y  = (T*) dst.ptr( level );
    const T*    b  = rhs ? (const T*) rhs->ptr( level ) : nullptr;
    if constexpr ( NR == 1 )
-      if ( cells && P.sweepScratch ) // small levels, once their tables are prepared
+      if ( cells && P.cellLocal ) // small levels, once their tables are prepared
       {
          const SweepCellTables< T > S  = sweepCellTables< T >( P, Wt );
          const ColourStarts         cs = colourStarts( P );
@@ -5440,7 +5440,7 @@ void launchSweepTables( Mesh& M, LevelPlan& P, CellLocal* cells, int32_t* own, i
    const int            w = P.w, t0 = (int) tetSize( w ), nf = ( w - 3 ) * ( w - 2 ) / 2;
    const SweepTableIn   S{ P.dV2E.p, P.dE2F.p, P.dF2C.p, P.dCellFaceRead.p, P.dVertexGeom.p, P.dVertexTerms.p, P.dEdgeGeom.p,
                            P.dEdgeTerms.p, P.dFaceGeom.p, P.dCellType.p, M.T.nC(), M.T.nE(), M.T.nF() };
-   const SweepTableOut  D{ cells, own, edgeNbr, faceNbr, (uint4*) scratch, P.total / 2 };
+   const SweepTableOut  D{ cells, own, edgeNbr, faceNbr, (uint4*) scratch, scratch ? P.total / 2 : 0 };
    const SweepTableGrid N{ (int) blocksFor( (int64_t) M.T.nC() * t0, 256 ), ( M.T.nE() + 3 ) / 4,
                            (int) blocksFor( (int64_t) M.T.nF() * nf * 8, 256 ), ( M.T.nC() + 255 ) / 256,
                            (int) std::min< int64_t >( 1024, blocksFor( D.nScratch, 256 ) ) };

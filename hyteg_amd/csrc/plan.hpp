@@ -158,6 +158,20 @@ struct CellLocal
    int32_t type, write;
 };
 constexpr int kSweepCellMaxLevel = 4;
+// Whether forward sweeps of a small level run as one launch each, a workgroup per macro-cell.  Every cell recomputes the
+// edges, faces and vertices around it, which is free while the workgroups run side by side: the time of a sweep is a
+// staircase with steps at one and two workgroups per CU, that of the separate launches grows slowly.  FP64, us a sweep of
+// a pair (alone), separate launches -> one launch:
+//             216 macro-tets          288                   480                   750
+//   level 1   12.3 -> 6.2             13.0 -> 9.3           14.8 -> 9.8           16.8 -> 13.4
+//   level 2   16.7 -> 10.8            17.9 -> 17.8          20.6 -> 18.8          23.5 -> 26.8
+//             (23.2 -> 13.2)          (22.3 -> 20.2)        (27.1 -> 21.1)        (31.6 -> 29.3)
+//   level 3   18.6 -> 12.3            18.9 -> 22.4          23.0 -> 22.2          26.3 -> 32.0
+//   level 4   22.2 -> 17.4            23.6 -> 29.3          28.8 -> 32.8          37.2 -> 48.8
+// (level 4, 3072 macro-tets, alone: 131 -> 205).  FP32 lies alike.  The one-launch apply and the restriction's owner
+// tables write every point once and win at any size (level 4, 10368 macro-tets, FP64: apply 278 -> 199, restriction
+// 196 -> 65).
+bool sweepsInOneLaunch( int level, int nCells );
 
 // Operator weights aligned with the geometry tables.
 //   face: 15 per face: in-plane C, W, E, N, S, NW, SE (summed over sides), then side0 off[4], side1 off[4]

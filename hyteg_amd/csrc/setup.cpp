@@ -902,6 +902,12 @@ void Mesh::selectCellSor( int level, int tile, int precisions )
 
 bool Mesh::cellSorReady( const LevelPlan& P ) const { return P.sorTile == 0 || ctx->hostOnly || P.sorUnits != nullptr; }
 
+bool sweepsInOneLaunch( int level, int nCells )
+{
+   constexpr int cus = 256;
+   return level >= 1 && level <= kSweepCellMaxLevel && ( level == 1 || nCells <= ( level == 2 ? 2 : 1 ) * cus );
+}
+
 void Mesh::prepareSweepCells( int minL, int maxL )
 {
    // the one-launch kernels run a workgroup per macro-cell: a vertex of no cell would be left out by all of them
@@ -912,7 +918,7 @@ void Mesh::prepareSweepCells( int minL, int maxL )
       LevelPlan&    P  = plan( L );
       const int64_t w  = P.w, most = int64_t( 1 ) << 30; // the kernels index elements and tables in 32 bits
       const bool    ok = P.total < most && T.nF() * ( w - 3 ) * ( w - 2 ) / 2 * 8 < most && (int64_t) P.hEdgeTerms.size() * ( w - 2 ) < most;
-      if ( ok && !P.sweepScratch ) levels.push_back( &P );
+      if ( ok && !P.cellLocal ) levels.push_back( &P );
    }
    if ( levels.empty() ) return;
    // one allocation for all of them, filled on the device (in 32-bit words; every table starts on 256 bytes)
@@ -923,7 +929,7 @@ void Mesh::prepareSweepCells( int minL, int maxL )
       n[1] = padded( (int64_t) T.nC() * P.cStride );
       n[2] = padded( (int64_t) P.hEdgeTerms.size() * ( w - 2 ) );
       n[3] = padded( (int64_t) T.nF() * ( ( w - 3 ) * ( w - 2 ) / 2 ) * 8 );
-      n[4] = padded( 2 * P.total ); // the scratch array, FP64
+      n[4] = sweepsInOneLaunch( P.L, T.nC() ) ? padded( 2 * P.total ) : 0; // the scratch array, FP64
    };
    size_t words = 0;
    for ( const LevelPlan* P : levels )
@@ -951,14 +957,14 @@ void Mesh::prepareSweepCells( int minL, int maxL )
       for ( int k = 0; k < 5; k++ )
          part[k] = at, at += n[k];
       launchSweepTables( *this, *P, reinterpret_cast< CellLocal* >( part[0] ), part[1], part[2], part[3],
-                         reinterpret_cast< double* >( part[4] ) );
+                         n[4] ? reinterpret_cast< double* >( part[4] ) : nullptr );
       HYMI_HIP( hipGetLastError() );
       P->sweepTables  = buf;
       P->cellLocal    = reinterpret_cast< const CellLocal* >( part[0] );
       P->own          = part[1];
       P->edgeNbr      = part[2];
       P->faceNbr      = part[3];
-      P->sweepScratch = reinterpret_cast< double* >( part[4] );
+      P->sweepScratch = n[4] ? reinterpret_cast< double* >( part[4] ) : nullptr;
    }
 }
 
