@@ -1047,14 +1047,17 @@ struct ColourStarts
 // With F2C = true (forward sweeps) the workgroup first copies its four faces' closures into the cell's closure
 // (the face-to-cell refresh of the sweep, as kF2C does it for this cell): the faces are final once the face
 // phase is done, and the cell's copies are read by no other workgroup.  Cells the flag leaves alone copy too.
-constexpr int kCellSmallWidth = ( 1 << kCellSmallMaxLevel ) + 1, kCellSmallIter = 2;
-template < typename T, bool F2C_ >
-__global__ __launch_bounds__( 1024 ) void kCellSorSmall( LV g, const int* __restrict__ pts, ColourStarts cs,
+// LMAX: the finest level of an instance, which sizes its LDS and its workgroups (about one point of a colour per thread).
+// With level 5's 52 KB at every level three workgroups fitted a CU, and 10368 macro-tets took 352 us a sweep at level 3.
+constexpr int kCellSmallIter = 2;
+constexpr int cellSmallThreads( int lmax ) { return lmax <= 3 ? 64 : lmax == 4 ? 128 : 1024; }
+template < typename T, bool F2C_, int LMAX >
+__global__ __launch_bounds__( cellSmallThreads( LMAX ) ) void kCellSorSmall( LV g, const int* __restrict__ pts, ColourStarts cs,
                                                         const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
                                                         T* __restrict__ u, const T* __restrict__ b, T omega, int reverse,
                                                         const F2C* __restrict__ f2c )
 {
-   constexpr int wM = kCellSmallWidth;
+   constexpr int wM = ( 1 << LMAX ) + 1;
    constexpr int Q = ( wM * ( wM + 1 ) * ( wM + 2 ) / 6 + 3 ) / 4;
    __shared__ T  V[4 * Q];
    // point i of the cell lies at at( i ): the points of a colour are 4 apart in a row, so the four residues of i are kept
@@ -2332,18 +2335,19 @@ __global__ __launch_bounds__( kEdgeThreads ) void kEdgeSorFused( LV g, const Edg
 // off-plane terms, which read cell points that the phase does not change, all loaded together.  Every face copies its
 // edges, also one whose own points the flag leaves alone.  With the boundary copied in memory first and the colours
 // reading it from there, 36 macro-tets took 9.5 us at level 5 in FP64, now 7.4.
-constexpr int kFaceFusedThreads = 512;
-template < typename T >
-__global__ __launch_bounds__( kFaceFusedThreads ) void kFaceSorFused( LV g, const FaceGeom* __restrict__ fg,
+// LMAX sizes LDS and workgroups, as for kCellSorSmall.
+constexpr int faceFusedThreads( int lmax ) { return lmax <= 3 ? 64 : lmax == 4 ? 256 : 512; }
+template < typename T, int LMAX >
+__global__ __launch_bounds__( faceFusedThreads( LMAX ) ) void kFaceSorFused( LV g, const FaceGeom* __restrict__ fg,
                                                                       const E2F* __restrict__ e2f,
                                                                       const T* __restrict__ FW, int flag,
                                                                       T* __restrict__ u, const T* __restrict__ b, T omega,
                                                                       int reverse )
 {
-   constexpr int   wM = ( 1 << kFaceFusedMaxLevel ) + 1;
-   __shared__ T    V[wM * ( wM + 1 ) / 2], sOff[kFaceFusedMaxNp], sB[kFaceFusedMaxNp];
+   constexpr int   wM = ( 1 << LMAX ) + 1, npM = ( wM - 3 ) * ( wM - 2 ) / 2;
+   __shared__ T    V[wM * ( wM + 1 ) / 2], sOff[npM], sB[npM];
    const FaceGeom& G  = fg[blockIdx.x];
-   const int       w = g.w, m = w - 3, np = m * ( m + 1 ) / 2, nV = w * ( w + 1 ) / 2; // np <= kFaceFusedMaxNp
+   const int       w = g.w, m = w - 3, np = m * ( m + 1 ) / 2, nV = w * ( w + 1 ) / 2;
    const int       tid = (int) threadIdx.x, nt = (int) blockDim.x;
    const int64_t   fo = g.offF + (int64_t) G.face * g.fS;
    const bool      on = ( G.type & flag ) != 0; // uniform over the workgroup
@@ -4575,6 +4579,19 @@ bool cellSorMulti( Mesh& M, LevelPlan& P, const T* CW, int flag, T* u, const T* 
    return true;
 }
 
+// calls f with the LMAX of the kernels that keep a face or a cell of a level up to 5 in LDS
+template < typename F >
+void smallLevel( int level, F&& f )
+{
+   static_assert( kFaceFusedMaxLevel == 5 && kCellSmallMaxLevel == 5, "the last instance covers the finest level" );
+   if ( level <= 3 )
+      f( std::integral_constant< int, 3 >{} );
+   else if ( level == 4 )
+      f( std::integral_constant< int, 4 >{} );
+   else
+      f( std::integral_constant< int, 5 >{} );
+}
+
 // withF2C: the one-workgroup-per-cell phase also does the face-to-cell refresh that precedes a forward cell
 // phase (the caller then skips it); ignored by the other forms of the phase.
 template < typename T, int NR >
@@ -4593,18 +4610,19 @@ void cellSorPhase( Mesh& M, LevelPlan& P, const T* CW, int flag, T* u, const T* 
       ColourStarts cs;
       for ( int k = 0; k < 5; k++ )
          cs.s[k] = P.colourStart[k];
-      // threads: about one point of a colour each, from 64 (level 2) up to 1024 (level 5: 1124 per colour)
-      const int perColour = ( P.colourStart[4] + 3 ) / 4;
-      const int threads   = std::min( 1024, std::max( 64, ( perColour + 63 ) / 64 * 64 ) );
-      for ( int k = 0; k < 4; k++ )
-         if ( cs.s[k + 1] - cs.s[k] > kCellSmallIter * threads )
-            throw std::logic_error( "cell SOR: more points of a colour than its threads take" );
-      if ( withF2C )
-         hipLaunchKernelGGL( ( kCellSorSmall< T, true > ), dim3( M.T.nC() ), dim3( threads ), 0, M.ctx->stream, viewOf( P ),
-                             P.dColourPts.p, cs, CW, P.dCellType.p, flag, u, b, om, rev, P.dF2C.p );
-      else
-         hipLaunchKernelGGL( ( kCellSorSmall< T, false > ), dim3( M.T.nC() ), dim3( threads ), 0, M.ctx->stream,
-                             viewOf( P ), P.dColourPts.p, cs, CW, P.dCellType.p, flag, u, b, om, rev, nullptr );
+      smallLevel( P.L, [&]( auto lmax ) {
+         constexpr int LMAX = decltype( lmax )::value, threads = cellSmallThreads( LMAX );
+         for ( int k = 0; k < 4; k++ )
+            if ( cs.s[k + 1] - cs.s[k] > kCellSmallIter * threads )
+               throw std::logic_error( "cell SOR: more points of a colour than its threads take" );
+         if ( withF2C )
+            hipLaunchKernelGGL( ( kCellSorSmall< T, true, LMAX > ), dim3( M.T.nC() ), dim3( threads ), 0, M.ctx->stream,
+                                viewOf( P ), P.dColourPts.p, cs, CW, P.dCellType.p, flag, u, b, om, rev, P.dF2C.p );
+         else
+            hipLaunchKernelGGL( ( kCellSorSmall< T, false, LMAX > ), dim3( M.T.nC() ), dim3( threads ), 0, M.ctx->stream,
+                                viewOf( P ), P.dColourPts.p, cs, CW, P.dCellType.p, flag, u, b, om, rev,
+                                (const F2C*) nullptr );
+      } );
    }
    else
       for ( int cc = 0; cc < 4; cc++ )
@@ -4873,8 +4891,11 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
       auto facePhase = [&]() {
          if ( nF == 0 ) return;
          if ( level <= kFaceFusedMaxLevel )
-            hipLaunchKernelGGL( ( kFaceSorFused< T > ), dim3( nF ), dim3( kFaceFusedThreads ), 0, s, g, P.dFaceGeom.p, P.dE2F.p,
-                                wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om, rev );
+            smallLevel( level, [&]( auto lmax ) {
+               constexpr int LMAX = decltype( lmax )::value;
+               hipLaunchKernelGGL( ( kFaceSorFused< T, LMAX > ), dim3( nF ), dim3( faceFusedThreads( LMAX ) ), 0, s, g,
+                                   P.dFaceGeom.p, P.dE2F.p, wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om, rev );
+            } );
          else
          {
             // large faces: one workgroup per face would leave most of the chip idle.  Forward, the faces'

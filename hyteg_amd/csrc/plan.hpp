@@ -163,14 +163,13 @@ constexpr int kSweepCellMaxLevel = 4;
 // staircase with steps at one and two workgroups per CU, that of the separate launches grows slowly.  FP64, us a sweep of
 // a pair (alone), separate launches -> one launch:
 //             216 macro-tets          288                   480                   750
-//   level 1   12.3 -> 6.2             13.0 -> 9.3           14.8 -> 9.8           16.8 -> 13.4
-//   level 2   16.7 -> 10.8            17.9 -> 17.8          20.6 -> 18.8          23.5 -> 26.8
-//             (23.2 -> 13.2)          (22.3 -> 20.2)        (27.1 -> 21.1)        (31.6 -> 29.3)
-//   level 3   18.6 -> 12.3            18.9 -> 22.4          23.0 -> 22.2          26.3 -> 32.0
-//   level 4   22.2 -> 17.4            23.6 -> 29.3          28.8 -> 32.8          37.2 -> 48.8
-// (level 4, 3072 macro-tets, alone: 131 -> 205).  FP32 lies alike.  The one-launch apply and the restriction's owner
-// tables write every point once and win at any size (level 4, 10368 macro-tets, FP64: apply 278 -> 199, restriction
-// 196 -> 65).
+//   level 1   12.3 -> 6.2             13.0 -> 9.3           14.8 -> 9.7           16.9 -> 13.4
+//   level 2   17.0 -> 10.8            17.8 -> 17.9          18.1 -> 18.8          19.0 -> 26.9
+//             (22.0 -> 13.1)          (23.1 -> 20.2)        (25.0 -> 21.2)        (27.7 -> 29.2)
+//   level 3   18.8 -> 12.2            19.8 -> 22.2          20.5 -> 22.2          21.3 -> 31.9
+//   level 4   21.9 -> 17.4            23.5 -> 29.2          25.7 -> 33.0          31.4 -> 48.9
+// FP32 lies alike.  The one-launch apply and the restriction's owner tables write every point once and win at any size
+// (level 4, 10368 macro-tets, FP64: apply 278 -> 199, restriction 196 -> 65).
 bool sweepsInOneLaunch( int level, int nCells );
 
 // Operator weights aligned with the geometry tables.
