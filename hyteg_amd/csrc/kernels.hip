@@ -2934,7 +2934,8 @@ __global__ __launch_bounds__( 256 ) void kCopyLevel( const T* __restrict__ src, 
 // The columns of an interleaved function do not couple, so a workgroup takes one primitive and RG of its NR columns
 // through a whole phase with barriers between the colours: vertices and edges (with the edges' end copies) in one launch,
 // up to level 5 faces (with the edge-to-face copy) in one, up to level 4 cells (with the face-to-cell copy) in one.  A
-// sweep was thirteen launches, most of them of 4 to 7 us that are latency; it is three (eight at level 5).  Values and
+// sweep was thirteen launches, most of them of 4 to 7 us that are latency; it is three (eight at level 5), where that pays
+// (edgesInOneLaunch, facesInOneLaunch).  Values and
 // expressions are those of the launches they replace; only the vertices' sums (eight slices) and the faces' (off-plane
 // terms first) are ordered anew.  Launches of a sweep, 48 macro-tets, 32 columns, FP32, us, before -> now: vertices and
 // edges 22 -> 10.5; faces 17, 18, 22, 42 at levels 2 to 5 -> 6, 9, 16, 37; cells 18, 21, 25 at levels 2 to 4 -> 7, 11, 14.
@@ -3010,13 +3011,19 @@ __global__ __launch_bounds__( kMultiThreads ) void kEdgeSorMulti( LV g, const Ed
 
 // one macro-face in LDS (levels <= kFaceFusedMaxLevel): V the whole face, its boundary straight from the edges, Q the
 // right-hand side less the off-plane terms, which read cell points that the phase does not change
-template < typename T, int NR, int RG >
-__global__ __launch_bounds__( 1024 ) void kFaceSorMulti( LV g, const FaceGeom* __restrict__ fg, const E2F* __restrict__ e2f,
+// (LMAX sizes the arrays and the workgroup, as for kCellSorSmall)
+constexpr int faceMultiThreads( int level, int rg )
+{
+   const int np = ( ( 1 << level ) - 2 ) * ( ( 1 << level ) - 1 ) / 2, t = np * rg / 64 * 64;
+   return t < 64 ? 64 : t > 1024 ? 1024 : t;
+}
+template < typename T, int NR, int RG, int LMAX >
+__global__ __launch_bounds__( faceMultiThreads( LMAX, RG ) ) void kFaceSorMulti( LV g, const FaceGeom* __restrict__ fg, const E2F* __restrict__ e2f,
                                                         const T* __restrict__ FW, int flag, T* __restrict__ u,
                                                         const T* __restrict__ b, T omega )
 {
-   constexpr int wMax = ( 1 << kFaceFusedMaxLevel ) + 1;
-   __shared__ T    V[wMax * ( wMax + 1 ) / 2 * RG], Q[kFaceFusedMaxNp * RG];
+   constexpr int   wM = ( 1 << LMAX ) + 1;
+   __shared__ T    V[wM * ( wM + 1 ) / 2 * RG], Q[( wM - 3 ) * ( wM - 2 ) / 2 * RG];
    const FaceGeom& G  = fg[blockIdx.x / ( NR / RG )];
    const int       rl = (int) threadIdx.x % RG, r = (int) ( blockIdx.x % ( NR / RG ) ) * RG + rl, w = g.w, m = w - 3;
    const int       t = (int) threadIdx.x / RG, step = (int) blockDim.x / RG, np = m * ( m + 1 ) / 2, nV = w * ( w + 1 ) / 2;
@@ -3066,14 +3073,14 @@ __global__ __launch_bounds__( 1024 ) void kFaceSorMulti( LV g, const FaceGeom* _
 // one macro-cell in LDS (pts: its interior points by colour, as for kCellSorSmall), its boundary planes straight from
 // the faces.  A thread holds the place and right-hand side of its point of each colour (at most one) from the start.  The
 // groups of a cell's columns run on one XCD: they share the lines of its points.
-template < typename T, int NR, int RG >
-__global__ __launch_bounds__( 1024 ) void kCellSorMulti( LV g, const int* __restrict__ pts, ColourStarts cs, int nCells,
+template < typename T, int NR, int RG, int LMAX >
+__global__ __launch_bounds__( LMAX <= 3 ? 128 : 1024 ) void kCellSorMulti( LV g, const int* __restrict__ pts, ColourStarts cs, int nCells,
                                                          const T* __restrict__ W8, const int* __restrict__ ctype, int flag,
                                                          T* __restrict__ u, const T* __restrict__ b, T omega,
                                                          const F2C* __restrict__ f2c )
 {
-   constexpr int wMax = ( 1 << kCellMultiMaxLevel ) + 1, groups = NR / RG;
-   __shared__ T  V[wMax * ( wMax + 1 ) * ( wMax + 2 ) / 6 * RG];
+   constexpr int wM = ( 1 << LMAX ) + 1, groups = NR / RG;
+   __shared__ T  V[wM * ( wM + 1 ) * ( wM + 2 ) / 6 * RG];
    const int     slot = (int) blockIdx.x >> 3, cell = slot / groups * 8 + ( (int) blockIdx.x & 7 );
    if ( cell >= nCells ) return;
    const int     rl = (int) threadIdx.x % RG, r = slot % groups * RG + rl, t = (int) threadIdx.x / RG;
@@ -4520,6 +4527,25 @@ void copyCells( Mesh& M, const LevelPlan& P, const T* src, T* dst )
                        (const uint4*) ( src + P.offC ), (uint4*) ( dst + P.offC ), n );
 }
 
+// Where a sweep on several right-hand sides takes its edges (with the vertices) and its faces in one launch each.  A
+// workgroup holds a whole primitive, so most of its lanes wait on small levels and few workgroups fit a CU on large ones;
+// the launches saved are 5 to 10 us.  Gain of the one launch over the separate ones, us a sweep (macro-tets: 48, 162, 750,
+// 3072; 32 columns):
+//   edges  FP32 level 1  +4, +9, +4, -15    level 2  +9, +10, +9, -8    level 3  +9, +9, +11, 0    level 4  +8, +9, +12, +8
+//   faces  FP64 level 3  +4, +5, +7, +16    level 4  +6, -3, -33, -147  level 5  -2, -23
+//          FP32 level 3  +5, +4, +12, +38   level 4  +1, -10, -74, -406 level 5  +1, +6
+// Edges: up to 2560 workgroups per level number (750 macro-tets are 2230 workgroups, 3072 are 8368).  Faces: up to level 3,
+// above as long as all their threads are resident at once.  (Cells always gain up to level 4: FP64 level 4 15 to 389.)
+bool edgesInOneLaunch( int level, int64_t workgroups, size_t lds )
+{
+   return level >= 1 && lds <= 60 * 1024 && workgroups <= 2560 * level;
+}
+bool facesInOneLaunch( int level, int64_t workgroups, int threads )
+{
+   constexpr int64_t resident = 256 * 2048;
+   return level >= 2 && level <= kFaceFusedMaxLevel && ( level <= 3 || workgroups * threads <= resident );
+}
+
 // Whether a forward smoothing sequence on this level can run its sweeps in ping-pong pairs: the fused cell phase
 // is selected for T (one right-hand side), the face phase reads the cells through ghost layers (levels above the
 // one-workgroup-per-face phase), and every macro-cell is updated (a cell the flag leaves alone would leave the
@@ -4556,6 +4582,19 @@ bool cellSorIsSmall( const LevelPlan& P )
    }
 }
 
+// calls f with the LMAX of the kernels that keep a face or a cell of a level up to 5 in LDS
+template < typename F >
+void smallLevel( int level, F&& f )
+{
+   static_assert( kFaceFusedMaxLevel == 5 && kCellSmallMaxLevel == 5, "the last instance covers the finest level" );
+   if ( level <= 3 )
+      f( std::integral_constant< int, 3 >{} );
+   else if ( level == 4 )
+      f( std::integral_constant< int, 4 >{} );
+   else
+      f( std::integral_constant< int, 5 >{} );
+}
+
 // The face-to-cell refresh and SOR cell phase of a forward sweep on several right-hand sides in one launch
 // (kCellSorMulti); false (nothing launched) above level 4: a level-5 cell leaves room for 16 bytes of columns per point
 // and one workgroup per CU, and took 79 us against 61 for the refresh and the four colour passes (48 cells, FP32).
@@ -4572,24 +4611,16 @@ bool cellSorMulti( Mesh& M, LevelPlan& P, const T* CW, int flag, T* u, const T* 
    }
    constexpr int RG      = 32 / (int) sizeof( T );
    const int     threads = ( most * RG + 63 ) / 64 * 64;
-   if ( threads > 1024 ) throw std::logic_error( "cell SOR: more points of a colour than a workgroup has threads" );
-   hipLaunchKernelGGL( ( kCellSorMulti< T, NR, RG > ), dim3( ( M.T.nC() + 7 ) / 8 * 8 * ( NR / RG ) ), dim3( threads ), 0,
-                       M.ctx->stream, viewOf( P ), P.dColourPts.p, cs, M.T.nC(), CW, P.dCellType.p, flag, u, b, om,
-                       P.dF2C.p );
+   static_assert( kCellMultiMaxLevel == 4, "the last instance covers the finest level" );
+   if ( threads > ( P.L <= 3 ? 128 : 1024 ) )
+      throw std::logic_error( "cell SOR: more points of a colour than a workgroup has threads" );
+   smallLevel( P.L, [&]( auto lmax ) {
+      constexpr int LMAX = std::min( decltype( lmax )::value, kCellMultiMaxLevel );
+      hipLaunchKernelGGL( ( kCellSorMulti< T, NR, RG, LMAX > ), dim3( ( M.T.nC() + 7 ) / 8 * 8 * ( NR / RG ) ), dim3( threads ),
+                          0, M.ctx->stream, viewOf( P ), P.dColourPts.p, cs, M.T.nC(), CW, P.dCellType.p, flag, u, b, om,
+                          P.dF2C.p );
+   } );
    return true;
-}
-
-// calls f with the LMAX of the kernels that keep a face or a cell of a level up to 5 in LDS
-template < typename F >
-void smallLevel( int level, F&& f )
-{
-   static_assert( kFaceFusedMaxLevel == 5 && kCellSmallMaxLevel == 5, "the last instance covers the finest level" );
-   if ( level <= 3 )
-      f( std::integral_constant< int, 3 >{} );
-   else if ( level == 4 )
-      f( std::integral_constant< int, 4 >{} );
-   else
-      f( std::integral_constant< int, 5 >{} );
 }
 
 // withF2C: the one-workgroup-per-cell phase also does the face-to-cell refresh that precedes a forward cell
@@ -4998,49 +5029,45 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
          cellSorLaunch< T, NR >( M, P, wsel< T >( Wt.cell64, Wt.cell32 ), flag, u, b, om, c );
    };
    // (closure copies are current: refreshed above when asked for, and every sweep ends with all of them current)
-   if constexpr ( NR > 1 )
+   // columns of a workgroup: 64 to 128 bytes of an edge point, 32 of a face point
+   constexpr int RE = NR > 1 ? 16 : 1, RF = 32 / (int) sizeof( T );
+   const size_t  edgeLds = 2 * (size_t) P.w * RE * sizeof( T );
+   if ( NR > 1 && edgesInOneLaunch( level, nE * ( NR / RE ), edgeLds ) )
    {
-      // columns of a workgroup: 64 to 128 bytes of an edge point, 32 of a face point
-      constexpr int RE = 16, RF = 32 / (int) sizeof( T );
-      const size_t  edgeLds = 2 * (size_t) P.w * RE * sizeof( T );
-      if ( level >= 1 && edgeLds <= 60 * 1024 ) // beyond (level 8), the launches are long anyway
-      {
+      if constexpr ( NR > 1 )
          hipLaunchKernelGGL( ( kEdgeSorMulti< T, NR, RE > ), dim3( nE * ( NR / RE ) ), dim3( kMultiThreads ), edgeLds, s, g,
                              P.dEdgeGeom.p, P.dEdgeTerms.p, wsel< T >( Wt.edge64, Wt.edge32 ), flag, u, b, om,
                              P.dVertexSnap.p, P.dEdgeEnds.p, wsel< T >( Wt.vertex64, Wt.vertex32 ) );
-         if ( level >= 2 && level <= kFaceFusedMaxLevel && nF > 0 )
-         {
-            const int threads = std::min( 1024, std::max( 64, ( P.w - 3 ) * ( P.w - 2 ) / 2 * RF / 64 * 64 ) );
-            hipLaunchKernelGGL( ( kFaceSorMulti< T, NR, RF > ), dim3( nF * ( NR / RF ) ), dim3( threads ), 0, s, g,
-                                P.dFaceGeom.p, P.dE2F.p, wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om );
-         }
-         else
-         {
-            refreshT< T, NR >( xf, level, 2 );
-            if ( level >= 2 ) faceColours();
-         }
-         if ( !cellSorMulti< T, NR >( M, P, wsel< T >( Wt.cell64, Wt.cell32 ), flag, u, b, om ) )
-         {
-            refreshT< T, NR >( xf, level, 4 );
-            if ( level >= 2 ) cellColours();
-         }
-         return;
-      }
    }
-   hipLaunchKernelGGL( ( kVertexSor< T, NR > ), dim3( blocksFor( (int64_t) nV * NR, 256 ) ), dim3( 256 ), 0, s, g,
-                       P.dVertexGeom.p, P.dVertexTerms.p, nV, wsel< T >( Wt.vertex64, Wt.vertex32 ), flag, u, b, om );
-   refreshT< T, NR >( xf, level, 1 );
-   if ( level >= 1 )
-      for ( int c = 0; c < 2; c++ )
-         hipLaunchKernelGGL( ( kEdgeSor< T, NR > ), dim3( blocksFor( (int64_t) ( P.w - 1 ) / 2 * NR, 64 ), nE ), dim3( 64 ), 0,
-                             s, g, P.dEdgeGeom.p, P.dEdgeTerms.p, wsel< T >( Wt.edge64, Wt.edge32 ), flag, u, b, om, c );
-   refreshT< T, NR >( xf, level, 2 );
-   if ( level >= 2 )
+   else
    {
-      faceColours();
-      refreshT< T, NR >( xf, level, 4 );
-      cellColours();
+      hipLaunchKernelGGL( ( kVertexSor< T, NR > ), dim3( blocksFor( (int64_t) nV * NR, 256 ) ), dim3( 256 ), 0, s, g,
+                          P.dVertexGeom.p, P.dVertexTerms.p, nV, wsel< T >( Wt.vertex64, Wt.vertex32 ), flag, u, b, om );
+      refreshT< T, NR >( xf, level, 1 );
+      if ( level >= 1 )
+         for ( int c = 0; c < 2; c++ )
+            hipLaunchKernelGGL( ( kEdgeSor< T, NR > ), dim3( blocksFor( (int64_t) ( P.w - 1 ) / 2 * NR, 64 ), nE ), dim3( 64 ), 0,
+                                s, g, P.dEdgeGeom.p, P.dEdgeTerms.p, wsel< T >( Wt.edge64, Wt.edge32 ), flag, u, b, om, c );
    }
+   if ( NR > 1 && facesInOneLaunch( level, nF * ( NR / RF ), faceMultiThreads( level, RF ) ) )
+   {
+      if constexpr ( NR > 1 )
+         smallLevel( level, [&]( auto lmax ) {
+            constexpr int LMAX = decltype( lmax )::value;
+            hipLaunchKernelGGL( ( kFaceSorMulti< T, NR, RF, LMAX > ), dim3( nF * ( NR / RF ) ),
+                                dim3( faceMultiThreads( level, RF ) ), 0, s, g, P.dFaceGeom.p, P.dE2F.p,
+                                wsel< T >( Wt.face64, Wt.face32 ), flag, u, b, om );
+         } );
+   }
+   else
+   {
+      refreshT< T, NR >( xf, level, 2 );
+      if ( level >= 2 ) faceColours();
+   }
+   if constexpr ( NR > 1 )
+      if ( cellSorMulti< T, NR >( M, P, wsel< T >( Wt.cell64, Wt.cell32 ), flag, u, b, om ) ) return;
+   if ( level >= 1 ) refreshT< T, NR >( xf, level, 4 );
+   if ( level >= 2 ) cellColours();
 }
 
 // One smoothing sequence of `count` forward sweeps.  Where pingPongOk holds, the sweeps run in pairs (u -> B, B -> u), after
