@@ -3923,15 +3923,16 @@ __global__ __launch_bounds__( 256 ) void kLowProlong( LowGrid L, LV gc, LV gf, c
 
 // --------------------------------------------------------------------------------------------------------
 // vector operations over closure ranges: workgroup (range, part), the parts of a range interleaved.  A range holds at
-// most 4096 points; with 32 right-hand sides one workgroup per range left the chip nearly empty on the levels that
-// such functions live on (level 5, 48 macro-tets: x += e 421 us, conversion to FP32 198 us; 61 and
-// 34 us with kRangeParts workgroups per range).
-
-constexpr int kRangeParts = 16;
+// most 4096 points; with 32 right-hand sides one workgroup per range leaves the chip nearly empty on meshes of few cells
+// (level 5, 48 macro-tets: x += e 421 us, conversion to FP32 198 us; with 16 parts 61 and 34 us).  A part has some 1024
+// values, and from 8192 ranges on each is one part: empty and short workgroups are launched one after another too (3072
+// macro-tets, 13.9 thousand ranges, y += x in 1 and 16 parts, us: FP64 level 1 11, 47, level 3 118, 137, FP32 level 4 415,
+// 470; 750 macro-tets, FP64 level 1 6.2, 11.7, level 4 204, 141).
 template < int NR >
-inline dim3 rangeGrid( int64_t ranges )
+inline dim3 rangeGrid( const LevelPlan& P, int64_t ranges )
 {
-   return dim3( (unsigned) ranges, NR == 1 ? 1 : kRangeParts );
+   const int64_t parts = ranges < 8192 ? P.total * NR / ( ranges * 1024 ) : 1;
+   return dim3( (unsigned) ranges, NR == 1 ? 1 : (unsigned) std::max< int64_t >( 1, std::min< int64_t >( parts, 16 ) ) );
 }
 __device__ __forceinline__ int64_t rangeBegin() { return (int64_t) blockIdx.y * blockDim.x + threadIdx.x; }
 __device__ __forceinline__ int64_t rangeStep() { return (int64_t) gridDim.y * blockDim.x; }
@@ -5304,7 +5305,7 @@ void lincombT( Function& dst, int level, int flag, int n, const double* c, Funct
    const S* s0 = n > 0 ? (const S*) src[0]->ptr( level ) : nullptr;
    const S* s1 = n > 1 ? (const S*) src[1]->ptr( level ) : nullptr;
    const S* s2 = n > 2 ? (const S*) src[2]->ptr( level ) : nullptr;
-   hipLaunchKernelGGL( ( kLincomb< T, S, NR > ), rangeGrid< NR >( nr ), dim3( 256 ), 0, M.ctx->stream, R,
+   hipLaunchKernelGGL( ( kLincomb< T, S, NR > ), rangeGrid< NR >( P, nr ), dim3( 256 ), 0, M.ctx->stream, R,
                        (T*) dst.ptr( level ), n, s0, s1, s2, n > 0 ? c[0] : 0.0, n > 1 ? c[1] : 0.0, n > 2 ? c[2] : 0.0,
                        acc ? 1 : 0, k );
 }
@@ -5317,7 +5318,7 @@ void axpyScalarT( Function& y, Function& x, int level, int flag, int slot, doubl
    int64_t      nr = 0;
    const Range* R  = M.closureRanges( P, flag, &nr );
    if ( nr == 0 ) return;
-   hipLaunchKernelGGL( ( kAxpyScalar< T, NR > ), rangeGrid< NR >( nr ), dim3( 256 ), 0, M.ctx->stream, R,
+   hipLaunchKernelGGL( ( kAxpyScalar< T, NR > ), rangeGrid< NR >( P, nr ), dim3( 256 ), 0, M.ctx->stream, R,
                        (T*) y.ptr( level ), (const T*) x.ptr( level ), M.ctx->scalars.p + (int64_t) slot * NR, sign );
 }
 
@@ -5329,7 +5330,7 @@ void xpbyScalarT( Function& p, Function& r, int level, int flag, int slot )
    int64_t      nr = 0;
    const Range* R  = M.closureRanges( P, flag, &nr );
    if ( nr == 0 ) return;
-   hipLaunchKernelGGL( ( kXpbyScalar< T, NR > ), rangeGrid< NR >( nr ), dim3( 256 ), 0, M.ctx->stream, R,
+   hipLaunchKernelGGL( ( kXpbyScalar< T, NR > ), rangeGrid< NR >( P, nr ), dim3( 256 ), 0, M.ctx->stream, R,
                        (T*) p.ptr( level ), (const T*) r.ptr( level ), M.ctx->scalars.p + (int64_t) slot * NR );
 }
 
@@ -5597,7 +5598,7 @@ void launchConvert( Function& dst, int dstLevel, Function& src, int srcLevel, in
       using TD            = std::remove_pointer_t< decltype( d ) >;
       using TS            = std::remove_const_t< std::remove_pointer_t< decltype( sp ) > >;
       constexpr int NRv   = decltype( nrTag )::value;
-      hipLaunchKernelGGL( ( kLincomb< TD, TS, NRv > ), rangeGrid< NRv >( nr ), dim3( 256 ), 0, s, R, d, 1, sp,
+      hipLaunchKernelGGL( ( kLincomb< TD, TS, NRv > ), rangeGrid< NRv >( P, nr ), dim3( 256 ), 0, s, R, d, 1, sp,
                           (const TS*) nullptr, (const TS*) nullptr, c1[0], 0.0, 0.0, 0, 0.0 );
    };
    auto run = [&]( auto nrTag ) {
@@ -5784,7 +5785,7 @@ struct ColumnSelectF
       int64_t      nr = 0;
       const Range* R  = M.closureRanges( P, kAll, &nr );
       if ( nr > 0 )
-         hipLaunchKernelGGL( ( kColumnSelect< T, NR > ), rangeGrid< NR >( nr ), dim3( 256 ), 0, M.ctx->stream, R,
+         hipLaunchKernelGGL( ( kColumnSelect< T, NR > ), rangeGrid< NR >( P, nr ), dim3( 256 ), 0, M.ctx->stream, R,
                              (T*) f.ptr( level ), keep );
    }
 };
@@ -5826,7 +5827,7 @@ void launchAddFromMasked( Function& x, Function& e, int level, int flag, unsigne
       using TD          = std::remove_pointer_t< decltype( d ) >;
       using TS          = std::remove_const_t< std::remove_pointer_t< decltype( sp ) > >;
       constexpr int NRv = decltype( nrTag )::value;
-      hipLaunchKernelGGL( ( kColumnAddFrom< TD, TS, NRv > ), rangeGrid< NRv >( nr ), dim3( 256 ), 0, s, R, d, sp, mask, 1.0,
+      hipLaunchKernelGGL( ( kColumnAddFrom< TD, TS, NRv > ), rangeGrid< NRv >( P, nr ), dim3( 256 ), 0, s, R, d, sp, mask, 1.0,
                           0.0 );
    };
    auto run = [&]( auto nrTag ) {
@@ -5860,7 +5861,7 @@ void launchAddFrom( Function& x, Function& e, int level, int flag )
       using TD          = std::remove_pointer_t< decltype( d ) >;
       using TS          = std::remove_const_t< std::remove_pointer_t< decltype( sp ) > >;
       constexpr int NRv = decltype( nrTag )::value;
-      hipLaunchKernelGGL( ( kLincomb< TD, TS, NRv > ), rangeGrid< NRv >( nr ), dim3( 256 ), 0, s, R, d, 1, sp,
+      hipLaunchKernelGGL( ( kLincomb< TD, TS, NRv > ), rangeGrid< NRv >( P, nr ), dim3( 256 ), 0, s, R, d, 1, sp,
                           (const TS*) nullptr, (const TS*) nullptr, 1.0, 0.0, 0.0, 1, 0.0 );
    };
    auto run = [&]( auto nrTag ) {
