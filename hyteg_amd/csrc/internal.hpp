@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -130,6 +131,10 @@ struct LevelPlan
    const int32_t *   own = nullptr, *edgeNbr = nullptr, *faceNbr = nullptr;
    const CellLocal*  cellLocal    = nullptr;
    double*           sweepScratch = nullptr;
+   // set once the above are; what goes through sweepScratch is enqueued under sweepLock, a whole sequence at a time, since
+   // threads may sweep different functions of one mesh
+   std::atomic< bool > sweepReady{ false };
+   std::mutex          sweepLock;
    // interior points of one macro-cell grouped by SOR colour (x + 2y + 3z) mod 4, packed x | y << 10 | z << 20,
    // colour c at [colourStart[c], colourStart[c+1]) (levels <= kCellSmallMaxLevel)
    DevBuf< int32_t >    dColourPts;
@@ -215,6 +220,7 @@ struct Mesh
    // tables and scratch arrays of the one-launch sweep on the levels of 1 .. kSweepCellMaxLevel in [minL, maxL] (outside
    // capture)
    void prepareSweepCells( int minL, int maxL );
+   std::mutex prepareLock; // of prepareSweepCells
    bool cellSorReady( const LevelPlan& P ) const;
    // fused residual and restriction from `level` (one right-hand side): -1 default, 0 off, 1 on (level >= 3);
    // bumps scheduleEpoch like setSchedule

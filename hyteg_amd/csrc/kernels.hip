@@ -4731,7 +4731,7 @@ void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, in
    T*          y  = (T*) dst.ptr( level );
    const T*    b  = rhs ? (const T*) rhs->ptr( level ) : nullptr;
    if constexpr ( NR == 1 )
-      if ( cells && P.cellLocal ) // small levels, once their tables are prepared
+      if ( cells && P.sweepReady.load( std::memory_order_acquire ) ) // small levels, once their tables are prepared
       {
          const SweepCellTables< T > S  = sweepCellTables< T >( P, Wt );
          const ColourStarts         cs = colourStarts( P );
@@ -4832,7 +4832,7 @@ void applyT( Operator& op, Function& src, Function& dst, const Function* rhs, in
 template < typename T >
 bool sweepCellOk( const LevelPlan& P )
 {
-   return P.sweepScratch && !( P.sorTile > 0 && ( P.sorPrecisions & ( std::is_same< T, double >::value ? 1 : 2 ) ) );
+   return P.sweepReady.load( std::memory_order_acquire ) && P.sweepScratch && !( P.sorTile > 0 && ( P.sorPrecisions & ( std::is_same< T, double >::value ? 1 : 2 ) ) );
 }
 
 // `count` forward sweeps, each from one of x and the level's scratch array to the other; after an odd count, the scratch
@@ -4847,6 +4847,7 @@ void sweepCells( Operator& op, Function& xf, const Function& bf, double omega, i
    T *         u = (T*) xf.ptr( level ), *other = reinterpret_cast< T* >( P.sweepScratch );
    const SweepCellTables< T > S  = sweepCellTables< T >( P, Wt );
    const ColourStarts         cs = colourStarts( P );
+   std::lock_guard< std::mutex > lock( P.sweepLock );
    for ( int k = 0; k < count; k++ )
    {
       const T* src = k % 2 ? other : u;
@@ -5120,7 +5121,8 @@ void restrictT( Function& f, Function& dst, int srcLevel, int flag, bool cells =
    T*          uc = (T*) dst.ptr( srcLevel - 1 );
    // of the cells' closures the restriction reads points within distance 1 of the faces' edges only (the cell-interior part
    // gathers interior fine points); on small levels it reads the owners instead
-   const int32_t *eNbr = NR == 1 ? Pf.edgeNbr : nullptr, *fNbr = NR == 1 ? Pf.faceNbr : nullptr;
+   const bool     owners = NR == 1 && Pf.sweepReady.load( std::memory_order_acquire );
+   const int32_t *eNbr = owners ? Pf.edgeNbr : nullptr, *fNbr = owners ? Pf.faceNbr : nullptr;
    if ( !eNbr ) refreshT< T, NR >( f, srcLevel, NR == 1 ? 1 | 2 | 8 : 7 );
    const int nV = M.T.nV(), nE = M.T.nE(), nF = M.T.nF();
    // coarse vertices, edge interiors, face interiors and (one right-hand side) macro-cell interiors in one launch,

@@ -912,13 +912,14 @@ void Mesh::prepareSweepCells( int minL, int maxL )
 {
    // the one-launch kernels run a workgroup per macro-cell: a vertex of no cell would be left out by all of them
    if ( ctx->hostOnly || T.loneVertices ) return;
-   std::vector< LevelPlan* > levels;
+   std::lock_guard< std::mutex > lock( prepareLock );
+   std::vector< LevelPlan* >     levels;
    for ( int L = std::max( 1, minL ); L <= std::min( maxL, kSweepCellMaxLevel ); L++ )
    {
       LevelPlan&    P  = plan( L );
       const int64_t w  = P.w, most = int64_t( 1 ) << 30; // the kernels index elements and tables in 32 bits
       const bool    ok = P.total < most && T.nF() * ( w - 3 ) * ( w - 2 ) / 2 * 8 < most && (int64_t) P.hEdgeTerms.size() * ( w - 2 ) < most;
-      if ( ok && !P.cellLocal ) levels.push_back( &P );
+      if ( ok && !P.sweepReady.load( std::memory_order_acquire ) ) levels.push_back( &P );
    }
    if ( levels.empty() ) return;
    // one allocation for all of them, filled on the device (in 32-bit words; every table starts on 256 bytes)
@@ -965,6 +966,7 @@ void Mesh::prepareSweepCells( int minL, int maxL )
       P->edgeNbr      = part[2];
       P->faceNbr      = part[3];
       P->sweepScratch = n[4] ? reinterpret_cast< double* >( part[4] ) : nullptr;
+      P->sweepReady.store( true, std::memory_order_release );
    }
 }
 
