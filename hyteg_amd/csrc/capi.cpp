@@ -1656,7 +1656,8 @@ int hymi_mesh_autotune( hymi_mesh mesh, int level, int precisions, int reps, dou
       };
 
       // 1. launch schedule of the macro-cell kernels, measured on the apply, the residual and the four SOR colour
-      //    passes of the first selected precision (the schedule is shared by both precisions)
+      //    passes of the first selected precision (the schedule is shared by both precisions; on levels up to
+      //    kSweepCellMaxLevel only what runs without the one-launch kernels' tables follows it)
       const int firstPrec = ( precisions & 1 ) ? kF64 : kF32;
       auto      f         = scratchFunctions( firstPrec );
       std::vector< MarchSchedule > cand;
@@ -1699,7 +1700,10 @@ int hymi_mesh_autotune( hymi_mesh mesh, int level, int precisions, int reps, dou
       f.clear();
 
       // 2. the SOR cell phase per selected precision: four colour passes against the fused launch, measured as
-      //    the cell phases of two chained sweeps (one smoothing sequence of a V(2, 2) cycle)
+      //    the cell phases of two chained sweeps (one smoothing sequence of a V(2, 2) cycle); where a sweep without the
+      //    fused phase is one launch for all primitives, as two whole sweeps either way
+      const bool wholeSweeps = sweepsInOneLaunch( level, M.T.nC() );
+      M.prepareSweepCells( level, level );
       int tileBits = M.plan( level ).sorTile ? M.plan( level ).sorPrecisions : 0;
       if ( level >= 3 )
          for ( int prec : { kF64, kF32 } )
@@ -1708,7 +1712,12 @@ int hymi_mesh_autotune( hymi_mesh mesh, int level, int precisions, int reps, dou
             if ( !( precisions & bit ) ) continue;
             auto   g       = scratchFunctions( prec );
             auto   timeSeq = [&]() {
-               return timeLaunches( s, reps, [&]() { launchCellSorSequence( A, *g[0], *g[1], 1.0, level, flag, 2 ); } );
+               return timeLaunches( s, reps, [&]() {
+                  if ( wholeSweeps )
+                     launchSorSweeps( A, *g[0], *g[1], 1.0, level, flag, 2 );
+                  else
+                     launchCellSorSequence( A, *g[0], *g[1], 1.0, level, flag, 2 );
+               } );
             };
             M.setCellSor( level, 0, 0 );
             const double tPass = timeSeq();

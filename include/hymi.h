@@ -274,7 +274,8 @@ int hymi_mesh_get_residual_restrict( hymi_mesh mesh, int level, int* out );
  *      on the macro-cell apply, the residual and the four SOR colour passes of the first precision selected
  *      in `precisions` (bit 0 FP64, bit 1 FP32; the schedule is shared by both), and keeps the fastest;
  *   2. for each selected precision (FP64 first), on levels >= 3: the SOR cell phase of two chained sweeps as
- *      four colour passes and as the fused launch, and keeps the faster.
+ *      four colour passes and as the fused launch, and keeps the faster; on levels 3 and 4, where a sweep without
+ *      the fused launch is one launch for all primitives (meshes of up to 256 macro-cells), as whole sweeps.
  * The choice is stored in the mesh as hymi_mesh_set_schedule and hymi_mesh_set_cell_sor would store it (the
  * results do not change: every schedule gives the same values bit for bit); captured V-cycle graphs are
  * captured again.  report (report_len doubles, may be NULL with report_len 0) receives the ms of every
