@@ -3152,6 +3152,10 @@ __global__ __launch_bounds__( LMAX <= 3 ? 128 : 1024 ) void kCellSorMulti( LV g,
 // One thread per point and right-hand side (neighbouring threads, so that they store contiguously).  The sines bound it:
 // with a thread per point that looped over 32 right-hand sides of 8 modes, a level-5 function of 48 macro-tets took
 // 2.17 ms, 0.53 now.
+__device__ __forceinline__ double modesCoordinate( const double* __restrict__ fr, int d, double h, int x, int y, int z )
+{
+   return fr[d] + h * ( x * fr[3 + d] + y * fr[6 + d] + z * fr[9 + d] );
+}
 template < typename T, int NR >
 __device__ __forceinline__ void putModes( T* __restrict__ u, int64_t idx, int r, const double* __restrict__ fr, double h,
                                           int x, int y, int z, const double* __restrict__ modes, int nModes )
@@ -3159,7 +3163,7 @@ __device__ __forceinline__ void putModes( T* __restrict__ u, int64_t idx, int r,
    double p[3];
 #pragma unroll
    for ( int d = 0; d < 3; d++ )
-      p[d] = fr[d] + h * ( x * fr[3 + d] + y * fr[6 + d] + z * fr[9 + d] );
+      p[d] = modesCoordinate( fr, d, h, x, y, z );
    const double pi = 3.141592653589793;
    const double* m   = modes + (int64_t) r * nModes * 4;
    double        acc = 0.0;
@@ -3219,13 +3223,38 @@ __global__ void kModesCell( LV g, const CellSeg* __restrict__ segs, int64_t nseg
 }
 
 // The macro-cell interiors for one right-hand side and at most kModesMax modes.  A point's coordinates are those of its
-// row's start plus x steps along the first edge, so by the addition theorem sin( k pi p ) = s0 cx + c0 sx with (s0, c0)
-// of the row and (sx, cx) of the x step: two fused operations in place of a sine, which bound the direct form (24 sines of
-// some 50 instructions per point and 8 modes: 7.1 ms a function at level 8, 48 macro-tets, 1.8 now).  Workgroup (part, chunk
-// of 64 x, cell): the step factors of its x in LDS, then each wave takes kModesRows rows of a slab at a time, computes
-// their factors lane by lane (LDS) and sums the modes of 64 points per row.  The parts take the slabs in turn.  Against
-// 64-bit values the error is that of the direct form, whose arguments are rounded as often.
+// row's first point plus steps along the first edge, so by the addition theorem its sine is s0 cx + c0 sx with (s0, c0) of
+// the row and (sx, cx) of the step.  The argument that the direct form takes the sine of is A = c p with c = k pi and the
+// coordinate p rounded, and A itself rounded (by up to 1e-13 for the waves that a level-8 mesh resolves).  The factors are
+// those of the unrounded products c p0 and c st; what A differs from their sum, the rest of the coordinate and the rounding
+// of the product, enters with the cosine, so that the result is the direct form's but for a few roundings of the sine.
+// Workgroup (part, chunk of 64 x, cell): the step factors of its x in LDS, then each wave takes kModesRows rows of a slab
+// at a time, computes their factors lane by lane (LDS) and sums the modes of 64 points per row.  The parts take the slabs
+// in turn.  Bound by FP64 arithmetic, 28 operations per point and mode where each of the direct form's three sines has
+// some 50: level 8, 48 macro-tets, 8 modes 7.1 ms, 3.3 so (1.6 without the rounding of A, 8e-14 off the direct form).
 constexpr int kModesMax = 8, kModesRows = 4, kModesThreads = 512;
+// p - q - s where q + s is p but for a few roundings
+__device__ __forceinline__ double sumRest( double p, double q, double s )
+{
+#pragma clang fp contract( off )
+   const double t = p - q, v = t - p; // p - q = t + what the difference lost
+   return ( t - s ) + ( ( p - ( t - v ) ) - ( q + v ) );
+}
+// c p rounded, less c p
+__device__ __forceinline__ double productRest( double c, double p )
+{
+#pragma clang fp contract( off )
+   const double a = c * p;
+   return __builtin_fma( -c, p, a );
+}
+// sine and cosine of the unrounded product c p
+__device__ __forceinline__ double2 productSinCos( double c, double p )
+{
+   const double e = productRest( c, p );
+   double       s, cs;
+   sincos( c * p, &s, &cs );
+   return make_double2( s - e * cs, cs + e * s );
+}
 template < typename T >
 __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const int* __restrict__ ctype, int frameOff, int flag,
                                                                    const double* __restrict__ fr,
@@ -3234,22 +3263,24 @@ __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const i
 {
    constexpr int CM = 3 * kModesMax, NW = kModesThreads / 64;
    __shared__ double2 sx[CM][64], sr[NW][kModesRows][CM];
-   __shared__ double  amp[kModesMax];
    const int cell = (int) blockIdx.z, tid = (int) threadIdx.x, wave = tid >> 6, lane = tid & 63, nc = 3 * nModes;
    if ( !( ctype[cell] & flag ) ) return;
    const int     w = g.w, t0 = tet32( w ), x0 = 1 + 64 * (int) blockIdx.y, x = x0 + lane;
    const double* f = fr + 12 * ( (int64_t) frameOff + cell );
    const double  h = 1.0 / ( w - 1 ), pi = 3.141592653589793;
+   auto          step = [&]( int d, int k ) { return h * ( k * f[3 + d] ); }; // k points along the first edge
+   auto          freq = [&]( int c ) { return modes[4 * ( c / 3 ) + 1 + c % 3] * pi; };
    for ( int k = tid; k < nc * 64; k += kModesThreads )
    {
-      const int c = k >> 6, d = c % 3;
-      double    s, cs;
-      sincos( modes[4 * ( c / 3 ) + 1 + d] * pi * ( h * ( x0 + ( k & 63 ) ) * f[3 + d] ), &s, &cs );
-      sx[c][k & 63] = make_double2( s, cs );
+      const int c   = k >> 6;
+      sx[c][k & 63] = productSinCos( freq( c ), step( c % 3, k & 63 ) );
    }
-   if ( tid < nModes ) amp[tid] = modes[4 * tid];
    __syncthreads();
    T* cu = u + g.offC + (int64_t) cell * g.cS;
+   double st[3];
+#pragma unroll
+   for ( int d = 0; d < 3; d++ )
+      st[d] = step( d, lane );
    for ( int z = 1 + (int) blockIdx.x; z <= w - 3 - x0; z += (int) gridDim.x )
    {
       const int last = w - 2 - z - x0; // rows 1 .. last hold an interior point at x0
@@ -3257,30 +3288,51 @@ __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const i
       {
          for ( int k = lane; k < kModesRows * nc; k += 64 )
          {
-            const int r = k / nc, c = k % nc, d = c % 3;
-            double    s, cs;
-            sincos( modes[4 * ( c / 3 ) + 1 + d] * pi * ( f[d] + h * ( ( y0 + r ) * f[6 + d] + z * f[9 + d] ) ), &s, &cs );
-            sr[wave][r][c] = make_double2( s, cs );
+            const int r = k / nc, c = k % nc;
+            sr[wave][r][c] = productSinCos( freq( c ), modesCoordinate( f, c % 3, h, x0, y0 + r, z ) );
          }
-         __builtin_amdgcn_wave_barrier(); // the wave's own writes, read below by its other lanes
-         double acc[kModesRows];
+         // the wave's own writes, read below by its other lanes
+         __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+         __builtin_amdgcn_wave_barrier();
+         double acc[kModesRows], p[kModesRows][3], rest[kModesRows][3];
 #pragma unroll
          for ( int r = 0; r < kModesRows; r++ )
+         {
             acc[r] = 0.0;
+#pragma unroll
+            for ( int d = 0; d < 3; d++ )
+            {
+               p[r][d]    = modesCoordinate( f, d, h, x, y0 + r, z );
+               rest[r][d] = sumRest( p[r][d], modesCoordinate( f, d, h, x0, y0 + r, z ), st[d] );
+            }
+         }
          for ( int m = 0; m < nModes; m++ )
          {
-            const double2 X = sx[3 * m][lane], Y = sx[3 * m + 1][lane], Z = sx[3 * m + 2][lane];
-            const double  a = amp[m];
+            double prod[kModesRows];
 #pragma unroll
             for ( int r = 0; r < kModesRows; r++ )
+               prod[r] = modes[4 * m];
+#pragma unroll
+            for ( int d = 0; d < 3; d++ )
             {
-               const double2 *q = sr[wave][r] + 3 * m;
-               acc[r] += a * ( q[0].x * X.y + q[0].y * X.x ) * ( q[1].x * Y.y + q[1].y * Y.x ) * ( q[2].x * Z.y + q[2].y * Z.x );
+               const double2 X = sx[3 * m + d][lane];
+               const double  c = modes[4 * m + 1 + d] * pi;
+#pragma unroll
+               for ( int r = 0; r < kModesRows; r++ )
+               {
+                  const double2 q = sr[wave][r][3 * m + d];
+                  const double  more = c * rest[r][d] + productRest( c, p[r][d] );
+                  prod[r] *= more * ( q.y * X.y - q.x * X.x ) + ( q.x * X.y + q.y * X.x );
+               }
             }
+#pragma unroll
+            for ( int r = 0; r < kModesRows; r++ )
+               acc[r] += prod[r];
          }
 #pragma unroll
          for ( int r = 0; r < kModesRows; r++ )
             if ( x + y0 + r + z <= w - 2 ) cu[crow32( w, t0, y0 + r, z ) + x] = (T) acc[r];
+         __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
          __builtin_amdgcn_wave_barrier();
       }
    }
