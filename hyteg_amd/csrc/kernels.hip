@@ -3222,7 +3222,7 @@ __global__ void kModesCell( LV g, const CellSeg* __restrict__ segs, int64_t nseg
                       fr + 12 * ( (int64_t) frameOff + sg.cell ), 1.0 / ( g.w - 1 ), x, sg.y, sg.z, modes, nModes );
 }
 
-// The macro-cell interiors for one right-hand side and at most kModesMax modes.  A point's coordinates are those of its
+// The macro-cell interiors for one right-hand side.  A point's coordinates are those of its
 // row's first point plus steps along the first edge, so by the addition theorem its sine is s0 cx + c0 sx with (s0, c0) of
 // the row and (sx, cx) of the step.  The argument that the direct form takes the sine of is A = c p with c = k pi and the
 // coordinate p rounded, and A itself rounded (by up to 1e-13 for the waves that a level-8 mesh resolves).  The factors are
@@ -3230,9 +3230,10 @@ __global__ void kModesCell( LV g, const CellSeg* __restrict__ segs, int64_t nseg
 // of the product, enters with the cosine, so that the result is the direct form's but for a few roundings of the sine.
 // Workgroup (part, chunk of 64 x, cell): the step factors of its x in LDS, then each wave takes kModesRows rows of a slab
 // at a time, computes their factors lane by lane (LDS) and sums the modes of 64 points per row.  The parts take the slabs
-// in turn.  Bound by FP64 arithmetic, 28 operations per point and mode where each of the direct form's three sines has
+// in turn.  Modes go in groups that fit LDS: of several, a group's step factors are formed anew for every 32 rows, 3 sines
+// a thread beside 8 modes of its 4 points.  Bound by FP64 arithmetic, 28 operations per point and mode where each of the direct form's three sines has
 // some 50: level 8, 48 macro-tets, 8 modes 7.1 ms, 3.3 so (1.6 without the rounding of A, 8e-14 off the direct form).
-constexpr int kModesMax = 8, kModesRows = 4, kModesThreads = 512;
+constexpr int kModesGroup = 8, kModesRows = 4, kModesThreads = 512;
 // p - q - s where q + s is p but for a few roundings
 __device__ __forceinline__ double sumRest( double p, double q, double s )
 {
@@ -3255,27 +3256,33 @@ __device__ __forceinline__ double2 productSinCos( double c, double p )
    sincos( c * p, &s, &cs );
    return make_double2( s - e * cs, cs + e * s );
 }
-template < typename T >
+template < typename T, bool GROUPS >
 __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const int* __restrict__ ctype, int frameOff, int flag,
                                                                    const double* __restrict__ fr,
                                                                    const double* __restrict__ modes, int nModes,
                                                                    T* __restrict__ u )
 {
-   constexpr int CM = 3 * kModesMax, NW = kModesThreads / 64;
+   constexpr int CM = 3 * kModesGroup, NW = kModesThreads / 64;
    __shared__ double2 sx[CM][64], sr[NW][kModesRows][CM];
-   const int cell = (int) blockIdx.z, tid = (int) threadIdx.x, wave = tid >> 6, lane = tid & 63, nc = 3 * nModes;
-   if ( !( ctype[cell] & flag ) ) return;
+   const int cell = (int) blockIdx.z, tid = (int) threadIdx.x, wave = tid >> 6, lane = tid & 63;
+   if ( !( ctype[cell] & flag ) ) return; // uniform over the workgroup
    const int     w = g.w, t0 = tet32( w ), x0 = 1 + 64 * (int) blockIdx.y, x = x0 + lane;
    const double* f = fr + 12 * ( (int64_t) frameOff + cell );
    const double  h = 1.0 / ( w - 1 ), pi = 3.141592653589793;
    auto          step = [&]( int d, int k ) { return h * ( k * f[3 + d] ); }; // k points along the first edge
    auto          freq = [&]( int c ) { return modes[4 * ( c / 3 ) + 1 + c % 3] * pi; };
-   for ( int k = tid; k < nc * 64; k += kModesThreads )
+   auto          steps = [&]( int m0 ) { // of modes m0 and up
+      for ( int k = tid; k < 3 * min( kModesGroup, nModes - m0 ) * 64; k += kModesThreads )
+      {
+         const int c   = k >> 6;
+         sx[c][k & 63] = productSinCos( freq( 3 * m0 + c ), step( c % 3, k & 63 ) );
+      }
+   };
+   if ( !GROUPS )
    {
-      const int c   = k >> 6;
-      sx[c][k & 63] = productSinCos( freq( c ), step( c % 3, k & 63 ) );
+      steps( 0 );
+      __syncthreads();
    }
-   __syncthreads();
    T* cu = u + g.offC + (int64_t) cell * g.cS;
    double st[3];
 #pragma unroll
@@ -3284,16 +3291,11 @@ __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const i
    for ( int z = 1 + (int) blockIdx.x; z <= w - 3 - x0; z += (int) gridDim.x )
    {
       const int last = w - 2 - z - x0; // rows 1 .. last hold an interior point at x0
-      for ( int y0 = 1 + wave * kModesRows; y0 <= last; y0 += NW * kModesRows )
+      for ( int yb = 1; yb <= last; yb += NW * kModesRows )
       {
-         for ( int k = lane; k < kModesRows * nc; k += 64 )
-         {
-            const int r = k / nc, c = k % nc;
-            sr[wave][r][c] = productSinCos( freq( c ), modesCoordinate( f, c % 3, h, x0, y0 + r, z ) );
-         }
-         // the wave's own writes, read below by its other lanes
-         __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
-         __builtin_amdgcn_wave_barrier();
+         const int  y0   = yb + wave * kModesRows;
+         const bool mine = y0 <= last;                // uniform over the wave
+         if ( !GROUPS && !mine ) break; // (of several groups, every wave takes part in their steps)
          double acc[kModesRows], p[kModesRows][3], rest[kModesRows][3];
 #pragma unroll
          for ( int r = 0; r < kModesRows; r++ )
@@ -3306,34 +3308,54 @@ __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const i
                rest[r][d] = sumRest( p[r][d], modesCoordinate( f, d, h, x0, y0 + r, z ), st[d] );
             }
          }
-         for ( int m = 0; m < nModes; m++ )
+         for ( int m0 = 0; GROUPS ? m0 < nModes : m0 == 0; m0 += kModesGroup )
          {
-            double prod[kModesRows];
-#pragma unroll
-            for ( int r = 0; r < kModesRows; r++ )
-               prod[r] = modes[4 * m];
-#pragma unroll
-            for ( int d = 0; d < 3; d++ )
+            if ( GROUPS )
             {
-               const double2 X = sx[3 * m + d][lane];
-               const double  c = modes[4 * m + 1 + d] * pi;
+               __syncthreads(); // every wave is done with the group before
+               steps( m0 );
+               __syncthreads();
+            }
+            if ( GROUPS && !mine ) continue;
+            const int n = GROUPS ? min( kModesGroup, nModes - m0 ) : nModes;
+            for ( int k = lane; k < kModesRows * 3 * n; k += 64 )
+            {
+               const int r = k / ( 3 * n ), c = k % ( 3 * n );
+               sr[wave][r][c] = productSinCos( freq( 3 * m0 + c ), modesCoordinate( f, c % 3, h, x0, y0 + r, z ) );
+            }
+            // the wave's own writes, read below by its other lanes
+            __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+            __builtin_amdgcn_wave_barrier();
+            for ( int m = 0; m < n; m++ )
+            {
+               const double* mode = modes + 4 * ( m0 + m );
+               double        prod[kModesRows];
 #pragma unroll
                for ( int r = 0; r < kModesRows; r++ )
-               {
-                  const double2 q = sr[wave][r][3 * m + d];
-                  const double  more = c * rest[r][d] + productRest( c, p[r][d] );
-                  prod[r] *= more * ( q.y * X.y - q.x * X.x ) + ( q.x * X.y + q.y * X.x );
-               }
-            }
+                  prod[r] = mode[0];
 #pragma unroll
-            for ( int r = 0; r < kModesRows; r++ )
-               acc[r] += prod[r];
+               for ( int d = 0; d < 3; d++ )
+               {
+                  const double2 X = sx[3 * m + d][lane];
+                  const double  c = mode[1 + d] * pi;
+#pragma unroll
+                  for ( int r = 0; r < kModesRows; r++ )
+                  {
+                     const double2 q = sr[wave][r][3 * m + d];
+                     const double  more = c * rest[r][d] + productRest( c, p[r][d] );
+                     prod[r] *= more * ( q.y * X.y - q.x * X.x ) + ( q.x * X.y + q.y * X.x );
+                  }
+               }
+#pragma unroll
+               for ( int r = 0; r < kModesRows; r++ )
+                  acc[r] += prod[r];
+            }
+            __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+            __builtin_amdgcn_wave_barrier();
          }
 #pragma unroll
          for ( int r = 0; r < kModesRows; r++ )
-            if ( x + y0 + r + z <= w - 2 ) cu[crow32( w, t0, y0 + r, z ) + x] = (T) acc[r];
-         __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
-         __builtin_amdgcn_wave_barrier();
+            if ( mine && x + y0 + r + z <= w - 2 ) cu[crow32( w, t0, y0 + r, z ) + x] = (T) acc[r];
       }
    }
 }
@@ -5958,12 +5980,16 @@ void launchInterpolateModes( Function& f, int level, int flag, int nModes, const
       if ( m > 0 && nF > 0 )
          hipLaunchKernelGGL( ( kModesFace< T, NR > ), dim3( blocksFor( m * ( m + 1 ) / 2 * NR, 128 ), nF ), dim3( 128 ), 0, s,
                              g, P.dFaceGeom.p, nV + nE, flag, fr, dModes, nModes, u );
-      if ( NR == 1 && nseg > 0 && nModes <= kModesMax )
+      // by factors where a cell has rows enough for them, more where the steps of several groups are formed for every 32
+      // rows (us by factors and directly: 10368 macro-tets, 8 modes, level 2 376, 270, level 3 550, 650; 750 macro-tets, 9
+      // modes, level 4 356, 251, level 5 830, 960)
+      if ( NR == 1 && nseg > 0 && level >= ( nModes <= kModesGroup ? 3 : 5 ) )
       {
          // slabs in parts, so that about 2048 workgroups share the cells' rows
          const int chunks = ( P.w - 4 + 63 ) / 64, parts = std::max( 1, std::min( P.w - 4, 2048 / ( nC * chunks ) ) );
-         hipLaunchKernelGGL( ( kModesRowsCell< T > ), dim3( parts, chunks, nC ), dim3( kModesThreads ), 0, s, g,
-                             P.dCellType.p, nV + nE + nF, flag, fr, dModes, nModes, u );
+         auto      rows   = nModes <= kModesGroup ? kModesRowsCell< T, false > : kModesRowsCell< T, true >;
+         hipLaunchKernelGGL( rows, dim3( parts, chunks, nC ), dim3( kModesThreads ), 0, s, g, P.dCellType.p, nV + nE + nF, flag,
+                             fr, dModes, nModes, u );
       }
       else if ( nseg > 0 )
          hipLaunchKernelGGL( ( kModesCell< T, NR > ), dim3( (unsigned) ( ( nseg + 3 ) / 4 ), NR ), dim3( 256 ), 0, s, g, sg,

@@ -12,9 +12,9 @@ from helpers import mesh_pair, say
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind", [("cube", 1), ("cube", 2), ("gmsh", "regular_octahedron_8el.msh")])
-@pytest.mark.parametrize("level", [3, 5, 7])
-@pytest.mark.parametrize("n_modes", [1, 8])
+@pytest.mark.parametrize("kind", [("cube", 1), ("gmsh", "regular_octahedron_8el.msh")])
+@pytest.mark.parametrize("level", [2, 3, 4, 5, 7])
+@pytest.mark.parametrize("n_modes", [1, 8, 9, 20])
 @pytest.mark.parametrize("precision", [0, 1])
 def test_short_waves_match_host(kind, level, n_modes, precision, gpu_ctx):
     import hyteg_amd as H
