@@ -1417,7 +1417,11 @@ int hymi_gmg_create( hymi_operator op, hymi_function xt, int minL, int maxL, int
       g->cg.r   = makeFunction( M, minL, minL, g->prec, g->nrhs );
       g->cg.ap  = makeFunction( M, minL, minL, g->prec, g->nrhs );
       // build every table a V-cycle uses now, so that a V-cycle never allocates (graph capture)
-      if ( g->nrhs == 1 ) M.prepareSweepCells( minL, maxL );
+      if ( g->nrhs == 1 )
+      {
+         M.prepareSweepCells( minL, maxL );
+         M.prepareProlongUnits( minL, maxL );
+      }
       const int segLen = 64 / g->nrhs;
       for ( int L = minL; L <= maxL; L++ )
       {
@@ -1425,10 +1429,8 @@ int hymi_gmg_create( hymi_operator op, hymi_function xt, int minL, int maxL, int
          int64_t    n = 0;
          M.segments( P, segLen, &n );
          if ( g->nrhs > 1 ) M.segments( P, kRowSeg, &n ); // cell apply, SOR and prolongation, several right-hand sides
-         M.marchUnits( P, &n );
+         if ( !P.sweepReady.load( std::memory_order_acquire ) ) M.marchUnits( P, &n ); // (its residual needs none then)
          M.transferUnits( P, &n );
-         int perCell = 0;
-         if ( g->nrhs == 1 ) M.prolongUnits( P, &perCell );
          if ( g->nrhs == 1 ) M.faceGhost( P );
          M.closureRanges( P, kInner | kNeumann, &n );
          M.closureRanges( P, kInner | kNeumann | kFreeslip, &n );

@@ -155,7 +155,9 @@ struct LevelPlan
    int64_t                                transferCount = -1;
    // work units of the prolongation to this level, of one macro-cell (the same for every cell): 64-element windows of
    // slab za marched up to zEnd, z = za | zEnd << 16, za odd, x0 = first element
-   std::unique_ptr< DevBuf< MarchUnit > > prolong;
+   // (in a table that the levels prepared together share, from prolongFirst on)
+   std::shared_ptr< DevBuf< MarchUnit > > prolong;
+   size_t                                 prolongFirst   = 0;
    int                                    prolongPerCell = -1;
    // work units of the fused residual-and-restriction kernel (this level as the coarse one): cell, run of coarse
    // slabs Za | Zb << 16, x0, y0 of the tile (1 + multiples of kResBandX, kResBandY), longest runs first; then the fine
@@ -203,6 +205,7 @@ struct Mesh
    const MarchUnit* marchUnits( LevelPlan& P, int64_t* count );
    const MarchUnit* transferUnits( LevelPlan& P, int64_t* count );
    const MarchUnit* prolongUnits( LevelPlan& P, int* perCell );
+   void             prepareProlongUnits( int minL, int maxL );
    const MarchUnit* residualRestrictUnits( LevelPlan& Pc, int64_t* count, int* extra );
    // face ghost buffer of level P (allocated on first use)
    void* faceGhost( LevelPlan& P );

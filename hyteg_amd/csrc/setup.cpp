@@ -797,12 +797,19 @@ const MarchUnit* Mesh::transferUnits( LevelPlan& P, int64_t* count )
    return P.transfer->p;
 }
 
-const MarchUnit* Mesh::prolongUnits( LevelPlan& P, int* perCell )
+// one allocation and copy for all levels of [minL, maxL] that lack their units
+void Mesh::prepareProlongUnits( int minL, int maxL )
 {
-   if ( P.prolongPerCell < 0 )
+   std::vector< MarchUnit >  v;
+   std::vector< LevelPlan* > levels;
+   std::vector< size_t >     first;
+   for ( int L = minL; L <= maxL; L++ )
    {
-      std::vector< MarchUnit > v;
-      const int                w = P.w, Zc = 8; // kProlongGroup slabs, all in flight together
+      LevelPlan& P = plan( L );
+      if ( P.prolongPerCell >= 0 ) continue;
+      const int w = P.w, Zc = 8; // kProlongGroup slabs, all in flight together
+      levels.push_back( &P );
+      first.push_back( v.size() );
       for ( int z = 1; z <= w - 4; z += Zc )
       {
          const int W     = w - z;
@@ -820,13 +827,25 @@ const MarchUnit* Mesh::prolongUnits( LevelPlan& P, int* perCell )
             if ( zEnd >= z ) v.push_back( { 0, z | ( zEnd << 16 ), e0, 0 } );
          }
       }
-      P.prolong = std::make_unique< DevBuf< MarchUnit > >();
-      P.prolong->upload( v, ctx->stream );
-      HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
-      P.prolongPerCell = (int) v.size();
    }
+   if ( levels.empty() ) return;
+   first.push_back( v.size() );
+   auto buf = std::make_shared< DevBuf< MarchUnit > >();
+   buf->upload( v, ctx->stream );
+   HYMI_HIP( hipStreamSynchronize( ctx->stream ) );
+   for ( size_t k = 0; k < levels.size(); k++ )
+   {
+      levels[k]->prolong        = buf;
+      levels[k]->prolongFirst   = first[k];
+      levels[k]->prolongPerCell = (int) ( first[k + 1] - first[k] );
+   }
+}
+
+const MarchUnit* Mesh::prolongUnits( LevelPlan& P, int* perCell )
+{
+   prepareProlongUnits( P.L, P.L );
    *perCell = P.prolongPerCell;
-   return P.prolong->p;
+   return P.prolong->p + P.prolongFirst;
 }
 
 // the SOR face phase's scratch: two ghost layers per face and a snapshot of the faces (face layout each)
