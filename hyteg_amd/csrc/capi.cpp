@@ -49,7 +49,8 @@ namespace {
 thread_local std::string g_lastError;
 
 // Fixed device scratch of hymi_dot_noalloc: the block partials of one dot product (at most kDotBlocks cell
-// workgroups plus 64 for the lower-dimensional primitives, times 32 right-hand sides: 528 KiB).  Each GPU the
+// workgroups plus 64 for the lower-dimensional primitives for one right-hand side, 1024 plus 256 for 32, times 32
+// right-hand sides: 528 KiB).  Each GPU the
 // library runs on holds its own copy until the process ends.  Host code never passes the array's name to a
 // kernel: it uses the address that hipGetSymbolAddress returned for the device (scratchOf).
 constexpr int64_t kScratchDoubles = kPartialsCap;
@@ -1153,7 +1154,7 @@ int hymi_dot_noalloc( hymi_function a, hymi_function b, int level, int flag, dou
       requireLevel( b->f, level );
       Context& ctx = *a->f.mesh->ctx;
       HYMI_HIP( hipSetDevice( ctx.device ) );
-      // partials beyond kScratchDoubles are refused inside (the grid is fixed: at most kDotBlocks + 64 blocks)
+      // partials beyond kScratchDoubles are refused inside (at most kDotBlocks + 64 blocks of one right-hand side or 1024 + 256 of 32)
       launchDotInto( a->f, b->f, level, flag, scratchOf( ctx.device ), kScratchDoubles, out_device );
    } );
 }

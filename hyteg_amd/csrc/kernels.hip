@@ -140,7 +140,7 @@ __device__ __forceinline__ int cellRel( int w, int t0, int x, int y, int z ) { r
 __device__ __forceinline__ int faceRel( int w, int i, int j ) { return fidx( w, i, j ); }
 // Row of flat index f in a triangle of width W stored row by row (row y has W - y points and starts at
 // R(y) = y (2W + 1 - y) / 2): the integer part of the smaller root of R(y) = f, taken in float, corrected by
-// one row either way (the float root is off by less than one row for W <= 1025).  0 <= f < W (W + 1) / 2.
+// one row either way (the float root is off by less than one row up to kTriRowMaxW).  0 <= f < W (W + 1) / 2.
 __device__ __forceinline__ int triRow32( int W, int f )
 {
    const float q = (float) ( 2 * W + 1 );
@@ -151,9 +151,8 @@ __device__ __forceinline__ int triRow32( int W, int f )
 }
 
 // (a, b) of flat index k in the triangle of width m (row-major, row b has m - b points).  The closed form in float
-// holds up to the widths of level 11 (triRow32).  With a double root and 64-bit products instead, the level-8 FP32
-// prolongation took 302 us (296 us now) and a level-4 V(2,2) cycle of 6 macro-tets 345 us (342 us); the level-8 apply
-// did not change: its face part is bound by the scattered cell reads.
+// holds up to the widths of level 11 (checked against exact rows for widths up to 2050); a double root and 64-bit products
+// instead cost a level-8 FP32 prolongation 2 %.
 constexpr int kTriRowMaxW = 2050;
 __device__ __forceinline__ void triPos( int m, int k, int& a, int& b )
 {
@@ -2412,8 +2411,8 @@ __global__ __launch_bounds__( faceFusedThreads( LMAX ) ) void kFaceSorFused( LV 
 // Three launches (vertices and edges, faces, cells), each a few microseconds of latency at these sizes, become one, and
 // the refresh before the first sweep goes.  The expressions are those of the launches it replaces, bit for bit.  Bound by
 // the latency of two dependent loads and some twelve barriers: 10 us at levels 1 to 3 and 15 us at level 4 (48
-// macro-tets, FP32) against 18 and 20 us for the three launches and their gaps; level-4 V(2,2) of 6 macro-tets 333 -> 240
-// us, level-6 FP32 solve 24.6 -> 21.7 ms, level-7 FP64 V(3,3) 3.45 -> 3.32 ms.  At level 5 a cell took 41 us against 30.
+// macro-tets, FP32) against 18 and 20 us for the three launches and their gaps (at level 5 a cell would take 41 us against
+// 30).  Where that holds for more cells: sweepsInOneLaunch.
 template < typename T >
 struct SweepCellTables
 {
@@ -3832,10 +3831,9 @@ __global__ __launch_bounds__( 256 ) void kProlongCell( LV gc, LV gf, const CellS
 
 // Column form for one right-hand side: a wave takes 64 consecutive elements of slab za of one macro-cell (unit:
 // z = za | zEnd << 16 with za odd, x0 = first element, the units of one cell, the same for every cell)
-// and marches these positions (x, y) up through slabs za .. zEnd.  What bounded the flat form (64-element windows of
-// one slab) was its index arithmetic, about 60 vector instructions per window; here a position's row and parities are
-// found once per unit, and a step advances the fine index by W (W + 1) / 2 - y (W: width of the slab) and, every
-// second step, the coarse row start by the same rule.  With h = y / 2, hx = x / 2 and Q(Z) the coarse index of row h,
+// and marches these positions (x, y) up through slabs za .. zEnd.  A position's row and parities are found once per unit
+// (in windows of one slab each, that arithmetic bound the kernel), and a step advances the fine index by
+// W (W + 1) / 2 - y (W: width of the slab) and, every second step, the coarse row start by the same rule.  With h = y / 2, hx = x / 2 and Q(Z) the coarse index of row h,
 // column hx of coarse slab Z, (p - d) / 2 and (p + d) / 2 (prolongDir) are, for odd z = 2Z + 1,
 //   Q(Z) + [y odd] (W_Z - h) + [x odd, y even]  and  Q(Z + 1) + [x odd, y odd],
 // and for even z = 2Z
@@ -3843,10 +3841,9 @@ __global__ __launch_bounds__( 256 ) void kProlongCell( LV gc, LV gf, const CellS
 // Slabs are taken kProlongGroup at a time, all loads of a group before its stores.  Closure positions are written too
 // (with the interpolation along the closure; every reader of a closure refreshes it first): left out, each row would
 // have a hole, and its lines would go to memory in parts.  A replacement of an array larger than the memory-side cache
-// (kStreamBytes) is written with non-temporal stores.  Bound by memory traffic now.  With the coarse refresh, 48
-// macro-tets, level 8, us: replacement FP32 296 -> 192 in turn with other work, 172 alone (265 with ordinary stores), FP64 600 -> 282 (448);
-// level 7 FP64 49 -> 41 (49 with non-temporal stores); addition FP32 333 -> 299, FP64 551 -> 552 (4.6 TB/s).  Units of 8
-// slabs: 4 or 16 are 2 to 30 % slower.
+// (kStreamBytes) is written with non-temporal stores.  Bound by memory traffic.  With the coarse refresh, 48 macro-tets,
+// us: replacement at level 8 FP32 180 (265 with ordinary stores), FP64 282 (448), at level 7 FP64 41 (49 with non-temporal
+// stores); addition at level 8 FP32 299, FP64 552 (4.6 TB/s).  Units of 8 slabs: 4 or 16 are 2 to 30 % slower.
 constexpr int     kProlongGroup = 8;
 constexpr int64_t kStreamBytes  = int64_t( 256 ) << 20; // the card's memory-side cache
 template < typename T, bool REPL >
@@ -5150,9 +5147,9 @@ void sorT( Operator& op, Function& xf, const Function& bf, double omega, int lev
 // one by itself (pp 3) if count is odd; otherwise sweep k is chained to sweep k - 1.  A sweep by itself in place needs
 // the band copy (43 % of the points at level 7, gathered row by row) and both face-to-cell copies; a plain copy of the
 // cells is shorter, unless there are fewer tiles than CUs: the sweep then takes as long as its longest tile, whose steps
-// are shorter in place (they choose between no two arrays).  One sweep, us, in place -> by itself: 48 macro-tets FP32
-// level 7 219 -> 199, level 8 1682 -> 1421, FP64 level 7 365 -> 343; 6 macro-tets FP64 level 8 (396 tiles) 416 -> 372,
-// FP32 level 7 (126 tiles) 131 -> 141.
+// are shorter in place (they choose between no two arrays).  One sweep, us, in place and by itself: 48 macro-tets FP32
+// level 7 219, 199, level 8 1682, 1421, FP64 level 7 365, 343; 6 macro-tets FP64 level 8 (396 tiles) 416, 372, FP32 level
+// 7 (126 tiles) 131, 141.
 constexpr int64_t kSorAloneUnits = 256;
 template < typename T, int NR >
 void sorSweepsT( Operator& op, Function& xf, const Function& bf, double omega, int level, int flag, int count,

@@ -5,7 +5,9 @@
  * (HYMI_OK == 0); on failure hymi_last_error_string() describes the error.  No entry point aborts the
  * process.  Work is enqueued on the context's HIP stream; entry points that return host-visible results
  * (downloads, dot products) synchronise that stream.  Calls on one handle are not thread-safe; different
- * contexts may be used concurrently.
+ * contexts may be used concurrently.  The first apply, residual or sweep of one right-hand side on a level from 1 to 4
+ * of a mesh, and the creation of a solver, also allocate that level's owner tables and fill them on the device (10 to
+ * 60 us for up to 3072 macro-cells, most of it the allocation).
  *
  * Each entry point names the reference interface it replaces (paths relative to the HyTeG source root).
  */
