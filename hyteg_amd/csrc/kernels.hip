@@ -3271,10 +3271,11 @@ __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const i
    auto          step = [&]( int d, int k ) { return h * ( k * f[3 + d] ); }; // k points along the first edge
    auto          freq = [&]( int c ) { return modes[4 * ( c / 3 ) + 1 + c % 3] * pi; };
    auto          steps = [&]( int m0 ) { // of modes m0 and up
-      for ( int k = tid; k < 3 * min( kModesGroup, nModes - m0 ) * 64; k += kModesThreads )
+      const int nx = min( 64, w - 3 - x0 ); // points of the chunk that the longest row has
+      for ( int k = tid; k < 3 * min( kModesGroup, nModes - m0 ) * nx; k += kModesThreads )
       {
-         const int c   = k >> 6;
-         sx[c][k & 63] = productSinCos( freq( 3 * m0 + c ), step( c % 3, k & 63 ) );
+         const int c = k / nx, i = k % nx;
+         sx[c][i]    = productSinCos( freq( 3 * m0 + c ), step( c % 3, i ) );
       }
    };
    if ( !GROUPS )
@@ -5977,10 +5978,11 @@ void launchInterpolateModes( Function& f, int level, int flag, int nModes, const
       if ( m > 0 && nF > 0 )
          hipLaunchKernelGGL( ( kModesFace< T, NR > ), dim3( blocksFor( m * ( m + 1 ) / 2 * NR, 128 ), nF ), dim3( 128 ), 0, s,
                              g, P.dFaceGeom.p, nV + nE, flag, fr, dModes, nModes, u );
-      // by factors where a cell has rows enough for them, more where the steps of several groups are formed for every 32
-      // rows (us by factors and directly: 10368 macro-tets, 8 modes, level 2 376, 270, level 3 550, 650; 750 macro-tets, 9
-      // modes, level 4 356, 251, level 5 830, 960)
-      if ( NR == 1 && nseg > 0 && level >= ( nModes <= kModesGroup ? 3 : 5 ) )
+      // by factors where a cell has points and modes enough for them: us directly and by factors, 10368 macro-tets, 8 modes,
+      // level 2 270, 376, level 3 653, 527; 750 macro-tets, 2 modes, level 3 62, 66, level 4 108, 99; 9 modes (the steps of
+      // two groups, formed for every 32 rows) level 4 251, 356, level 5 979, 848
+      const int byFactors = nModes < 4 ? 4 : nModes <= kModesGroup ? 3 : 5;
+      if ( NR == 1 && nseg > 0 && level >= byFactors )
       {
          // slabs in parts, so that about 2048 workgroups share the cells' rows
          const int chunks = ( P.w - 4 + 63 ) / 64, parts = std::max( 1, std::min( P.w - 4, 2048 / ( nC * chunks ) ) );
