@@ -30,7 +30,7 @@ def test_forward_sweep_of_many_cells(precision, gpu_ctx):
             gpu_ctx.synchronize()
             best[sweep.__name__] = min(best.get(sweep.__name__, 1e9), (time.perf_counter() - t) / 20)
     say(f"[sweep route] precision={precision} {({k: round(1e6 * v, 1) for k, v in best.items()})} us")
-    assert best["smooth_sor"] < best["smooth_sor_backwards"]
+    assert best["smooth_sor"] < 1.1 * best["smooth_sor_backwards"]
 
 
 @pytest.mark.parametrize("cells", [250, 258, 510, 516])
