@@ -3230,8 +3230,9 @@ __global__ void kModesCell( LV g, const CellSeg* __restrict__ segs, int64_t nseg
 // Workgroup (part, chunk of 64 x, cell): the step factors of its x in LDS, then each wave takes kModesRows rows of a slab
 // at a time, computes their factors lane by lane (LDS) and sums the modes of 64 points per row.  The parts take the slabs
 // in turn.  Modes go in groups that fit LDS: of several, a group's step factors are formed anew for every 32 rows, 3 sines
-// a thread beside 8 modes of its 4 points.  Bound by FP64 arithmetic, 28 operations per point and mode where each of the direct form's three sines has
-// some 50: level 8, 48 macro-tets, 8 modes 7.1 ms, 3.3 so (1.6 without the rounding of A, 8e-14 off the direct form).
+// a thread beside 8 modes of its 4 points.  Bound by FP64 arithmetic, 25 operations per point and mode where each of the
+// direct form's three sines has some 50, and by the waves in flight (two workgroups per CU with 128 registers; with 136 one
+// fits, 3.2 ms): level 8, 48 macro-tets, 8 modes 7.1 ms, 3.0 so (1.6 without the rounding of A, 8e-14 off the direct form).
 constexpr int kModesGroup = 8, kModesRows = 4, kModesThreads = 512;
 // p - q - s where q + s is p but for a few roundings
 __device__ __forceinline__ double sumRest( double p, double q, double s )
@@ -3256,7 +3257,7 @@ __device__ __forceinline__ double2 productSinCos( double c, double p )
    return make_double2( s - e * cs, cs + e * s );
 }
 template < typename T, bool GROUPS >
-__global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const int* __restrict__ ctype, int frameOff, int flag,
+__global__ __launch_bounds__( kModesThreads, 4 ) void kModesRowsCell( LV g, const int* __restrict__ ctype, int frameOff, int flag,
                                                                    const double* __restrict__ fr,
                                                                    const double* __restrict__ modes, int nModes,
                                                                    T* __restrict__ u )
@@ -3343,7 +3344,7 @@ __global__ __launch_bounds__( kModesThreads ) void kModesRowsCell( LV g, const i
                   {
                      const double2 q = sr[wave][r][3 * m + d];
                      const double  more = c * rest[r][d] + productRest( c, p[r][d] );
-                     prod[r] *= more * ( q.y * X.y - q.x * X.x ) + ( q.x * X.y + q.y * X.x );
+                     prod[r] *= q.x * ( X.y - more * X.x ) + q.y * ( X.x + more * X.y );
                   }
                }
 #pragma unroll
@@ -5979,8 +5980,8 @@ void launchInterpolateModes( Function& f, int level, int flag, int nModes, const
          hipLaunchKernelGGL( ( kModesFace< T, NR > ), dim3( blocksFor( m * ( m + 1 ) / 2 * NR, 128 ), nF ), dim3( 128 ), 0, s,
                              g, P.dFaceGeom.p, nV + nE, flag, fr, dModes, nModes, u );
       // by factors where a cell has points and modes enough for them: us directly and by factors, 10368 macro-tets, 8 modes,
-      // level 2 270, 376, level 3 653, 527; 750 macro-tets, 2 modes, level 3 62, 66, level 4 108, 99; 9 modes (the steps of
-      // two groups, formed for every 32 rows) level 4 251, 356, level 5 979, 848
+      // level 2 270, 376, level 3 653, 527; 750 macro-tets, 2 modes, level 3 62, 66, level 4 108, 97; 9 modes (the steps of
+      // two groups, formed for every 32 rows) level 4 251, 356, level 5 979, 711
       const int byFactors = nModes < 4 ? 4 : nModes <= kModesGroup ? 3 : 5;
       if ( NR == 1 && nseg > 0 && level >= byFactors )
       {
